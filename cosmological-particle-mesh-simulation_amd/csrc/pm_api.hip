@@ -67,6 +67,87 @@ int ensure_init() {
   } while (0)
 
 // ------------------------------------------------------------------------------------------
+// device memory
+// ------------------------------------------------------------------------------------------
+// pm_malloc / pm_free keep freed blocks for the next allocation of the same size.  Every density or
+// potential on device arrays allocates its result: hipMalloc + hipFree of a 384^3 grid cost 0.3 ms
+// a call, and the driver clears freed memory at about 35 GB/s, so a loop that allocates faster
+// than that ends up waiting for it (6.4 ms per 384^3 density, 0.5 ms of which are kernels).
+// A block is put back only when the device is idle, as hipFree would have waited too, so no stream
+// can still use it when it is handed out again.  The pool holds at most kPoolBytes (the oldest blocks
+// go first), and everything is given back before an allocation fails and before free memory is
+// reported.
+constexpr size_t kPoolBytes = (size_t)4 << 30;
+constexpr size_t kPoolGrain = (size_t)64 << 10;  // blocks are whole multiples of this
+
+constexpr int kPoolBlocks = 64;
+
+struct PoolBlock {
+  void* ptr;
+  size_t bytes;
+};
+std::mutex g_pool_mu;
+PoolBlock g_pool[kPoolBlocks];  // free blocks, oldest first
+int g_pool_n = 0;
+size_t g_pool_bytes = 0;  // their bytes
+
+// (callers hold g_pool_mu)
+void* pool_take(int i) {
+  void* p = g_pool[i].ptr;
+  g_pool_bytes -= g_pool[i].bytes;
+  --g_pool_n;
+  for (; i < g_pool_n; ++i) g_pool[i] = g_pool[i + 1];
+  return p;
+}
+void pool_empty() {
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  while (g_pool_n) (void)hipFree(pool_take(0));
+}
+
+// hipMalloc that gives the pool's free blocks back before it fails (every allocation of the library)
+hipError_t dev_malloc(void** ptr, size_t bytes) {
+  hipError_t e = hipMalloc(ptr, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    pool_empty();
+    e = hipMalloc(ptr, bytes);
+  }
+  return e;
+}
+template <class T> hipError_t dev_malloc(T** ptr, size_t bytes) { return dev_malloc((void**)ptr, bytes); }
+
+hipError_t pool_alloc(void** ptr, size_t bytes) {
+  bytes = std::max((bytes + kPoolGrain - 1) / kPoolGrain, (size_t)1) * kPoolGrain;
+  {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    for (int i = 0; i < g_pool_n; ++i)
+      if (g_pool[i].bytes == bytes) {
+        *ptr = pool_take(i);
+        return hipSuccess;
+      }
+  }
+  return dev_malloc(ptr, bytes);
+}
+
+hipError_t pool_free(void* ptr) {
+  hipDeviceptr_t base = nullptr;
+  size_t bytes = 0;
+  // pointers that do not start an allocation go to hipFree, which names the error
+  if (hipMemGetAddressRange(&base, &bytes, ptr) != hipSuccess || base != ptr || bytes % kPoolGrain ||
+      bytes > kPoolBytes || hipDeviceSynchronize() != hipSuccess) {
+    (void)hipGetLastError();
+    return hipFree(ptr);
+  }
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  for (int i = 0; i < g_pool_n; ++i)
+    if (g_pool[i].ptr == ptr) return hipErrorInvalidValue;  // freed twice
+  while (g_pool_n == kPoolBlocks || g_pool_bytes + bytes > kPoolBytes) (void)hipFree(pool_take(0));
+  g_pool[g_pool_n++] = {ptr, bytes};
+  g_pool_bytes += bytes;
+  return hipSuccess;
+}
+
+// ------------------------------------------------------------------------------------------
 // per-size FFT tables and complex128 workspaces
 // ------------------------------------------------------------------------------------------
 std::map<std::pair<int, int>, FftTables> g_tables;
@@ -95,9 +176,9 @@ int get_tables(int n, int prec, FftTables** out) {
   t.n = n;
   t.prec = prec;
   const size_t rb = (size_t)prec;
-  PM_HIP(hipMalloc(&t.tw, 2 * (size_t)n * rb));
-  PM_HIP(hipMalloc(&t.sin2, (size_t)n * rb));
-  PM_HIP(hipMalloc(&t.wdec, (size_t)n * rb));
+  PM_HIP(dev_malloc(&t.tw, 2 * (size_t)n * rb));
+  PM_HIP(dev_malloc(&t.sin2, (size_t)n * rb));
+  PM_HIP(dev_malloc(&t.wdec, (size_t)n * rb));
   if (prec == 8) {
     PM_HIP(hipMemcpy(t.tw, tw.data(), tw.size() * 8, hipMemcpyHostToDevice));
     PM_HIP(hipMemcpy(t.sin2, s2.data(), s2.size() * 8, hipMemcpyHostToDevice));
@@ -125,13 +206,13 @@ int get_workspace(int n, bool need_phi, Workspace** out) {
   Workspace& w = g_ws[n];
   const size_t nn = (size_t)n;
   if (!w.H) {
-    if (hipMalloc(&w.H, nn * nn * (nn / 2) * sizeof(double2)) != hipSuccess)
+    if (dev_malloc(&w.H, nn * nn * (nn / 2) * sizeof(double2)) != hipSuccess)
       return fail(PM_E_NOMEM, "cannot allocate the complex128 half spectrum for N=%d", n);
-    if (hipMalloc(&w.Q, nn * nn * sizeof(double2)) != hipSuccess)
+    if (dev_malloc(&w.Q, nn * nn * sizeof(double2)) != hipSuccess)
       return fail(PM_E_NOMEM, "cannot allocate the Nyquist plane for N=%d", n);
   }
   if (need_phi && !w.phi) {
-    if (hipMalloc(&w.phi, nn * nn * nn * sizeof(float)) != hipSuccess)
+    if (dev_malloc(&w.phi, nn * nn * nn * sizeof(float)) != hipSuccess)
       return fail(PM_E_NOMEM, "cannot allocate the potential scratch for N=%d", n);
   }
   *out = &w;
@@ -229,12 +310,12 @@ PM_API int pm_supported_grid(int n_cells) { return fft_size_supported(n_cells) ?
 PM_API int pm_malloc(void** ptr, size_t bytes) {
   PM_INIT();
   if (!ptr) return fail(PM_E_INVALID, "null output pointer");
-  if (hipMalloc(ptr, bytes ? bytes : 1) != hipSuccess) return fail(PM_E_NOMEM, "hipMalloc(%zu) failed", bytes);
+  if (pool_alloc(ptr, bytes) != hipSuccess) return fail(PM_E_NOMEM, "hipMalloc(%zu) failed", bytes);
   return PM_OK;
 }
 PM_API int pm_free(void* ptr) {
   PM_INIT();
-  if (ptr) PM_HIP(hipFree(ptr));
+  if (ptr) PM_HIP(pool_free(ptr));
   return PM_OK;
 }
 PM_API int pm_memcpy_htod(void* dst, const void* src, size_t bytes) {
@@ -260,6 +341,7 @@ PM_API int pm_memset(void* dst, int value, size_t bytes) {
 PM_API int pm_mem_info(size_t* free_bytes, size_t* total_bytes) {
   PM_INIT();
   if (!free_bytes || !total_bytes) return fail(PM_E_INVALID, "null argument");
+  pool_empty();
   PM_HIP(hipMemGetInfo(free_bytes, total_bytes));
   return PM_OK;
 }
@@ -762,8 +844,8 @@ template <typename R> int sim_build_graph(pm_sim* s) {
   const int c0 = s->cur, g0 = s->gb;
   if (s->graph[c0][g0]) return PM_OK;
   if (!s->d_table) {
-    PM_HIP(hipMalloc(&s->d_table, sizeof(double) * 3 * kTableSteps));
-    PM_HIP(hipMalloc(&s->d_step, sizeof(int)));
+    PM_HIP(dev_malloc(&s->d_table, sizeof(double) * 3 * kTableSteps));
+    PM_HIP(dev_malloc(&s->d_step, sizeof(int)));
   }
   hipGraph_t graph = nullptr;
   PM_HIP(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
@@ -1047,12 +1129,12 @@ PM_API int pm_sim_create(int n_cells, int n_parts_side, int precision, unsigned 
   if (int rc = get_tables(n_cells, s->prec, &s->tab)) return cleanup(rc);
   bool ok = true;
   for (int k = 0; k < 2; ++k)
-    ok = ok && hipMalloc(&s->sb[k], 3 * (size_t)s->L.np * pr) == hipSuccess &&
-         hipMalloc(&s->vb[k], 3 * (size_t)s->L.np * pr) == hipSuccess &&
-         hipMalloc(&s->idb[k], (size_t)s->L.np * 6) == hipSuccess;  // ids, then the tile scatter's bin codes
-  if (!ok || hipMalloc(&s->grid[0], nn * nn * nn * pr) != hipSuccess ||
-      hipMalloc(&s->grid[1], nn * nn * nn * pr) != hipSuccess || hipMalloc(&s->Q, nn * nn * 2 * pr) != hipSuccess ||
-      (has_edge(n_cells, s->prec) && hipMalloc(&s->edge, edge_bytes(n_cells)) != hipSuccess))
+    ok = ok && dev_malloc(&s->sb[k], 3 * (size_t)s->L.np * pr) == hipSuccess &&
+         dev_malloc(&s->vb[k], 3 * (size_t)s->L.np * pr) == hipSuccess &&
+         dev_malloc(&s->idb[k], (size_t)s->L.np * 6) == hipSuccess;  // ids, then the tile scatter's bin codes
+  if (!ok || dev_malloc(&s->grid[0], nn * nn * nn * pr) != hipSuccess ||
+      dev_malloc(&s->grid[1], nn * nn * nn * pr) != hipSuccess || dev_malloc(&s->Q, nn * nn * 2 * pr) != hipSuccess ||
+      (has_edge(n_cells, s->prec) && dev_malloc(&s->edge, edge_bytes(n_cells)) != hipSuccess))
     return cleanup(fail(PM_E_NOMEM, "device allocation of %zu bytes failed", sim_bytes(n_cells, n_parts_side, s->prec)));
   s->G = make_tiles(n_cells, s->prec);
   const TileGeom gmax = max_tiles(n_cells, s->prec);
@@ -1060,10 +1142,10 @@ PM_API int pm_sim_create(int n_cells, int n_parts_side, int precision, unsigned 
   if (8 * (size_t)s->L.np >= (size_t)UINT32_MAX) return cleanup(fail(PM_E_INVALID, "too many particles (N_PARTS > 812)"));
   s->B.capacity = (uint32_t)(8 * (size_t)s->L.np);
   const size_t cw = counts_words(n_cells, gmax);
-  if (hipMalloc(&s->B.counts, cw * 4) != hipSuccess || hipMalloc(&s->B.offsets, (m + 1) * 4) != hipSuccess ||
-      hipMalloc(&s->B.cursors, m * 4) != hipSuccess || hipMalloc(&s->B.entries, 8 * (size_t)s->L.np * 4) != hipSuccess ||
-      hipMalloc(&s->B.block_sums, ((size_t)scan_blocks(gmax) + 1) * 4) != hipSuccess ||
-      hipMalloc(&s->B.health, sizeof(uint32_t) * PM_HEALTH_COUNT) != hipSuccess ||
+  if (dev_malloc(&s->B.counts, cw * 4) != hipSuccess || dev_malloc(&s->B.offsets, (m + 1) * 4) != hipSuccess ||
+      dev_malloc(&s->B.cursors, m * 4) != hipSuccess || dev_malloc(&s->B.entries, 8 * (size_t)s->L.np * 4) != hipSuccess ||
+      dev_malloc(&s->B.block_sums, ((size_t)scan_blocks(gmax) + 1) * 4) != hipSuccess ||
+      dev_malloc(&s->B.health, sizeof(uint32_t) * PM_HEALTH_COUNT) != hipSuccess ||
       hipHostMalloc(&s->h_health, sizeof(uint32_t) * PM_HEALTH_COUNT, hipHostMallocDefault) != hipSuccess)
     return cleanup(fail(PM_E_NOMEM, "device allocation of the tile bins failed"));
   std::memset(s->h_health, 0, sizeof(uint32_t) * PM_HEALTH_COUNT);
@@ -1153,7 +1235,7 @@ PM_API int pm_sim_set_density(pm_sim* s, const void* rho, int dtype_bytes, int o
     const void* src = rho;
     void* tmp = nullptr;
     if (!on_device) {
-      if (hipMalloc(&tmp, cnt * dtype_bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
+      if (dev_malloc(&tmp, cnt * dtype_bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
       if (hipMemcpyAsync(tmp, rho, cnt * dtype_bytes, hipMemcpyHostToDevice, s->stream) != hipSuccess) {
         (void)hipFree(tmp);
         return fail(PM_E_HIP, "host to device copy failed");
@@ -1180,7 +1262,7 @@ PM_API int pm_sim_set_state(pm_sim* s, const void* pos, const void* vel, int dty
   const void* dv = vel;
   void* tmp = nullptr;
   if (!on_device) {
-    if (hipMalloc(&tmp, 2 * bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
+    if (dev_malloc(&tmp, 2 * bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
     dp = tmp;
     dv = (char*)tmp + bytes;
     hipError_t e1 = hipMemcpyAsync((void*)dp, pos, bytes, hipMemcpyHostToDevice, s->stream);
@@ -1229,7 +1311,7 @@ PM_API int pm_sim_get_state(pm_sim* s, void* pos, void* vel, int dtype_bytes, in
   void* dv = vel;
   void* tmp = nullptr;
   if (!on_device) {
-    if (hipMalloc(&tmp, 2 * bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
+    if (dev_malloc(&tmp, 2 * bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
     dp = tmp;
     dv = (char*)tmp + bytes;
   }
@@ -1273,7 +1355,7 @@ static int copy_grid_out(pm_sim* s, const void* src, void* dst, int dtype_bytes,
     return PM_OK;
   }
   if (!on_device) {
-    if (hipMalloc(&tmp, cnt * dtype_bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
+    if (dev_malloc(&tmp, cnt * dtype_bytes) != hipSuccess) return fail(PM_E_NOMEM, "staging allocation failed");
     d = tmp;
   }
   hipError_t e = s->prec == 4 ? convert_grid<float, double>((const float*)src, (double*)d, cnt, s->stream)
@@ -1385,7 +1467,7 @@ PM_API int pm_sim_zeldovich(pm_sim* s, const double* amp, int64_t n_amp, double 
   FftTables* t;
   if (int rc = get_tables(n, s->prec, &t)) return rc;
   double* d_amp = nullptr;
-  if (hipMalloc(&d_amp, sizeof(double) * need) != hipSuccess) return fail(PM_E_NOMEM, "amplitude table allocation failed");
+  if (dev_malloc(&d_amp, sizeof(double) * need) != hipSuccess) return fail(PM_E_NOMEM, "amplitude table allocation failed");
   hipError_t e = hipMemcpyAsync(d_amp, amp, sizeof(double) * need, hipMemcpyHostToDevice, s->stream);
   if (e == hipSuccess) {
     if (s->prec == 4)
@@ -1420,7 +1502,7 @@ PM_API int pm_sim_power_spectrum(pm_sim* s, double box, int n_bins, double* k, d
   const long cells = (long)n * n * n;
   double* d = nullptr;  // [0]: sum of rho, then 3 (n_bins + 1) shell sums
   const size_t nd = 1 + 3 * (size_t)(n_bins + 1);
-  if (hipMalloc(&d, sizeof(double) * nd) != hipSuccess) return fail(PM_E_NOMEM, "spectrum scratch allocation failed");
+  if (dev_malloc(&d, sizeof(double) * nd) != hipSuccess) return fail(PM_E_NOMEM, "spectrum scratch allocation failed");
   std::vector<double> h(nd);
   hipError_t e = hipMemsetAsync(d, 0, sizeof(double) * nd, s->stream);
   if (e == hipSuccess) {
@@ -1684,9 +1766,9 @@ PM_API int pm_ensemble_create(pm_ensemble** out) {
   if (init_err != hipSuccess) return fail(PM_E_HIP, "batched FFT set-up failed: %s", hipGetErrorString(init_err));
   pm_ensemble* e = new pm_ensemble();
   e->host = new BatchDesc();
-  if (hipMalloc(&e->d_desc, sizeof(BatchDesc)) != hipSuccess ||
-      hipMalloc(&e->d_table, sizeof(double) * 3 * kBatchMax * kEnsTableSteps) != hipSuccess ||
-      hipMalloc(&e->d_step, sizeof(int)) != hipSuccess || hipStreamCreate(&e->stream) != hipSuccess) {
+  if (dev_malloc(&e->d_desc, sizeof(BatchDesc)) != hipSuccess ||
+      dev_malloc(&e->d_table, sizeof(double) * 3 * kBatchMax * kEnsTableSteps) != hipSuccess ||
+      dev_malloc(&e->d_step, sizeof(int)) != hipSuccess || hipStreamCreate(&e->stream) != hipSuccess) {
     pm_ensemble_destroy(e);
     return fail(PM_E_NOMEM, "ensemble allocation failed");
   }
