@@ -120,7 +120,7 @@ hipError_t pool_alloc(void** ptr, size_t bytes) {
   bytes = std::max((bytes + kPoolGrain - 1) / kPoolGrain, (size_t)1) * kPoolGrain;
   {
     std::lock_guard<std::mutex> lk(g_pool_mu);
-    for (int i = 0; i < g_pool_n; ++i)
+    for (int i = g_pool_n - 1; i >= 0; --i)  // the one freed last
       if (g_pool[i].bytes == bytes) {
         *ptr = pool_take(i);
         return hipSuccess;
