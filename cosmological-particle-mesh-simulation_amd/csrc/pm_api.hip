@@ -219,6 +219,92 @@ int get_workspace(int n, bool need_phi, Workspace** out) {
   return PM_OK;
 }
 
+// The reference-layout entry points share the workspaces of this section: each holds this mutex
+// from its first launch to its synchronisation, so calls from several threads take turns.
+std::mutex g_ref_mu;
+
+// Tile bins of the reference-layout density and integrate (callers hold g_ref_mu): one slab grown to
+// the largest call so far; a slab above kRefKeepBytes is given back when its call ends.
+struct RefBins {
+  void* slab = nullptr;
+  size_t bytes = 0;
+} g_ref_bins;
+constexpr size_t kRefKeepBytes = (size_t)1 << 30;
+// Below these many particles the kernels without bins run: five short launches cost more than the
+// atomics or line fetches that the tiles save.  Whole calls at 2 cells per particle and axis, evenly
+// spread / clustered particles, in us, without and with bins:
+//   density    33 k: 28 / 33 and 40 / 50,   111 k: 63 / 71 and 43 / 57,   262 k: 118 / 132 and 49 / 61,
+//              2.1 M: 815 / 839 and 125 / 138
+//   integrate  133 k: 27 / 31 and 42 / 53,  262 k: 46 / 44 and 47 / 58,   885 k: 125 / 147 and 67 / 82,
+//              2.1 M: 295 / 308 and 102 / 132
+constexpr int64_t kRefDepositMin = 1 << 16;
+constexpr int64_t kRefPushMin = 1 << 19;
+// ... and above this many cells per particle (a 16^3 tile then holds fewer than 16 particles, and the
+// tile deposit's pass over the empty cells costs more than the atomics).
+constexpr int64_t kRefTileCells = 256;
+
+// The bins for a call with n_p particles on an n^3 grid; false: the call runs without (a grid that
+// no tile divides, fewer than `least` or too many particles, or no memory for the entries).
+bool ref_bins_begin(int64_t n_p, int64_t least, int n, TileGeom& G, Bins& B) {
+  if (n_p < least || n % 8 || kRefTileCells * n_p < (int64_t)n * n * n) return false;
+  const int t = n % 16 ? 8 : 16;
+  G = make_tiles(n, 4, t, t, t);
+  if (!ref_tiles_ok(n_p, G)) return false;
+  const size_t m = 2 * (size_t)G.ntiles, nb = (size_t)scan_blocks(G);
+  const size_t words = m + 1 + (m + 1) + m + nb + 8 * (size_t)n_p;
+  RefBins& r = g_ref_bins;
+  if (words * 4 > r.bytes) {
+    if (r.slab) (void)hipFree(r.slab);
+    r = RefBins{};
+    if (dev_malloc(&r.slab, words * 4) != hipSuccess) {
+      (void)hipGetLastError();
+      r.slab = nullptr;
+      return false;
+    }
+    r.bytes = words * 4;
+  }
+  uint32_t* w = (uint32_t*)r.slab;
+  B = Bins{};
+  B.counts = w;
+  B.done = w + m;  // cleared together with the counts
+  B.offsets = B.done + 1;
+  B.cursors = B.offsets + m + 1;
+  B.block_sums = B.cursors + m;
+  B.entries = B.block_sums + nb;
+  B.capacity = (uint32_t)(8 * (size_t)n_p);
+  return true;
+}
+// the work is done (the stream is idle): a large slab goes back
+void ref_bins_end() {
+  RefBins& r = g_ref_bins;
+  if (r.bytes <= kRefKeepBytes) return;
+  (void)hipFree(r.slab);
+  r = RefBins{};
+}
+
+int density_into(const float* pos, int64_t n_p, int n, double mass, float* rho, hipStream_t st) {
+  TileGeom G;
+  Bins B;
+  if (!ref_bins_begin(n_p, kRefDepositMin, n, G, B)) {
+    PM_HIP(ref_density(pos, n_p, n, mass, rho, st));
+    return PM_OK;
+  }
+  PM_HIP(ref_density_tiles(pos, n_p, n, mass, rho, G, B, st));
+  return PM_OK;
+}
+
+int integrate_into(float* pos, float* vel, int64_t n_p, int n, double a, double fa1, double da, const float* phi,
+                   hipStream_t st) {
+  TileGeom G;
+  Bins B;
+  if (!ref_bins_begin(n_p, kRefPushMin, n, G, B)) {
+    PM_HIP(ref_integrate(pos, vel, n_p, n, a, fa1, da, phi, st));
+    return PM_OK;
+  }
+  PM_HIP(ref_integrate_tiles(pos, vel, n_p, n, a, fa1, da, phi, G, B, st));
+  return PM_OK;
+}
+
 // ------------------------------------------------------------------------------------------
 // fixed device scratch of pm_potential_static: the complex128 half spectrum, the Nyquist plane
 // and the FFT tables of one N^3 grid, N <= kStaticMaxN (about 17 MiB, held by each device the
@@ -358,8 +444,10 @@ PM_API int pm_synchronize(void) {
 PM_API int pm_density(const float* pos, int64_t n_p, int n, double mass, float* rho) {
   PM_INIT();
   if (n <= 0 || n_p < 0 || !rho || (n_p > 0 && !pos)) return fail(PM_E_INVALID, "pm_density: bad arguments");
-  PM_HIP(ref_density(pos, n_p, n, mass, rho, g_stream));
+  std::lock_guard<std::mutex> turn(g_ref_mu);
+  if (int rc = density_into(pos, n_p, n, mass, rho, g_stream)) return rc;
   PM_HIP(hipStreamSynchronize(g_stream));
+  ref_bins_end();
   return PM_OK;
 }
 
@@ -375,6 +463,7 @@ PM_API int pm_density_k(const float* rho, int n, void* rho_k) {
   PM_INIT();
   if (int rc = check_grid(n)) return rc;
   if (!rho || !rho_k) return fail(PM_E_INVALID, "pm_density_k: null pointer");
+  std::lock_guard<std::mutex> turn(g_ref_mu);
   FftTables* t;
   Workspace* w;
   if (int rc = get_tables(n, 8, &t)) return rc;
@@ -400,6 +489,7 @@ PM_API int pm_potential_real(const void* phi_k, int n, float* phi) {
   PM_INIT();
   if (int rc = check_grid(n)) return rc;
   if (!phi_k || !phi) return fail(PM_E_INVALID, "pm_potential_real: null pointer");
+  std::lock_guard<std::mutex> turn(g_ref_mu);
   FftTables* t;
   Workspace* w;
   if (int rc = get_tables(n, 8, &t)) return rc;
@@ -434,6 +524,7 @@ PM_API int pm_potential(const float* rho, const float* fgrid, int n, double a, d
   PM_INIT();
   if (int rc = check_grid(n)) return rc;
   if (!rho || !fgrid || !phi || a == 0.0) return fail(PM_E_INVALID, "pm_potential: bad arguments");
+  std::lock_guard<std::mutex> turn(g_ref_mu);
   if (int rc = potential_into(rho, fgrid, n, a, omega_m0, phi)) return rc;
   PM_HIP(hipStreamSynchronize(g_stream));
   return PM_OK;
@@ -507,8 +598,10 @@ PM_API int pm_integrate(float* pos, float* vel, int64_t n_p, int n, double a_val
                         const float* phi) {
   PM_INIT();
   if (n <= 0 || n_p < 0 || (n_p && (!pos || !vel || !phi))) return fail(PM_E_INVALID, "pm_integrate: bad arguments");
-  PM_HIP(ref_integrate(pos, vel, n_p, n, a_val, f_a1, da, phi, g_stream));
+  std::lock_guard<std::mutex> turn(g_ref_mu);
+  if (int rc = integrate_into(pos, vel, n_p, n, a_val, f_a1, da, phi, g_stream)) return rc;
   PM_HIP(hipStreamSynchronize(g_stream));
+  ref_bins_end();
   return PM_OK;
 }
 
@@ -519,12 +612,14 @@ PM_API int pm_advance_time(const float* rho, float* pos, float* vel, const float
   if (int rc = check_grid(n)) return rc;
   if (n_p < 0 || !rho || !fgrid || (n_p && (!pos || !vel)) || a == 0.0)
     return fail(PM_E_INVALID, "pm_advance_time: bad arguments");
+  std::lock_guard<std::mutex> turn(g_ref_mu);
   Workspace* w;
   if (int rc = get_workspace(n, true, &w)) return rc;
   if (int rc = potential_into(rho, fgrid, n, a, omega_m0, w->phi)) return rc;
   const double fa1 = f_of_a(a + da, h0, omega_lambda0, omega_k0);  // integrate.py:12 (Q1)
-  PM_HIP(ref_integrate(pos, vel, n_p, n, a, fa1, da, w->phi, g_stream));
+  if (int rc = integrate_into(pos, vel, n_p, n, a, fa1, da, w->phi, g_stream)) return rc;
   PM_HIP(hipStreamSynchronize(g_stream));
+  ref_bins_end();
   return PM_OK;
 }
 

@@ -175,6 +175,14 @@ hipError_t gkd_tiles(const PState<R>& in, const PState<R>& out, const R* phi, do
 
 // ---- reference-layout kernels (absolute float32 positions, reference order) ------------------
 hipError_t ref_density(const float* pos, long np, int n, double mass, float* rho, hipStream_t st);
+// The same through tile bins (own + halo entries of the tiles G, at most 8 N_p): the sums of a cell
+// meet in FP64 in LDS.  B: entries of 8 N_p words, the scan's ticket right after the 2*ntiles counts;
+// ref_tiles_ok tells whether G and N_p allow it.
+bool ref_tiles_ok(long np, const TileGeom& G);
+hipError_t ref_density_tiles(const float* pos, long np, int n, double mass, float* rho, const TileGeom& G,
+                             const Bins& B, hipStream_t st);
+hipError_t ref_integrate_tiles(float* pos, float* vel, long np, int n, double a, double fa1, double da,
+                               const float* phi, const TileGeom& G, const Bins& B, hipStream_t st);
 hipError_t ref_cell_centers(const float* pos, long np, int n, int64_t* cells, hipStream_t st);
 hipError_t ref_weights(const int64_t* cells, const float* pos, long np, float* t, hipStream_t st);
 hipError_t ref_sweep(const int64_t* cells, float* xd, float* vd, const float* t, const float* phi, long np,

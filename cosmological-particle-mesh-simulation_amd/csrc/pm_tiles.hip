@@ -76,6 +76,18 @@ __device__ __forceinline__ void cell_and_frac(const R* __restrict__ s, long e, u
   cell_and_frac<R>(s[e], s[L.np + e], s[2 * L.np + e], id, L, c, d, q);
 }
 
+// cell and CIC fractions of an absolute float32 position (the reference layout's arrays): a value
+// equal to n maps to 0, out-of-range and NaN positions to a clamped cell
+__device__ __forceinline__ void abs_cell_and_frac(float x, float y, float z, int n, int c[3], float d[3]) {
+  const float xv[3] = {x, y, z};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float w = wrap_pos<float>(xv[a], float(n));
+    c[a] = cell_of<float>(w, n);
+    d[a] = w - float(c[a]);
+  }
+}
+
 // home tile of a cell and whether the cloud reaches the next tile along each axis
 template <int TX, int TY, int TZ>
 __device__ __forceinline__ void tile_of(const int c[3], const TileGeom& G, int t[3], int up[3]) {
@@ -572,9 +584,10 @@ template <int TX, int TY, int TZ> constexpr int deposit_lds_cells() { return (TX
 // DET: the LDS sums are 64-bit fixed point with `fix` units per unit mass (a power of two chosen
 // by the host so that the whole mass fits in 62 bits); integer adds are associative, so the
 // cell values do not depend on the order the atomics land in.
-template <typename R, int TX, int TY, int TZ, bool DET = false>
+// ABS: s holds absolute positions and there are no ids (only L.n and L.np are read).
+template <typename R, int TX, int TY, int TZ, bool DET = false, bool ABS = false>
 __device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint32_t* __restrict__ id,
-                                             R* __restrict__ rho, R mass, const Lattice& L, const TileGeom& G,
+                                             R* __restrict__ rho, double mass, const Lattice& L, const TileGeom& G,
                                              const uint32_t* __restrict__ offsets,
                                              const uint32_t* __restrict__ entries, uint32_t capacity, int tile,
                                              double* acc, uint32_t* __restrict__ health, double fix = 0.0) {
@@ -604,7 +617,7 @@ __device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint
     }
 #pragma unroll
     for (int u = 0; u < E; ++u) {
-      pid[u] = sl[u] != kNone ? id[sl[u]] : 0u;
+      pid[u] = !ABS && sl[u] != kNone ? id[sl[u]] : 0u;
 #pragma unroll
       for (int a = 0; a < 3; ++a) sv[u][a] = sl[u] != kNone ? s[a * np + sl[u]] : R(0);
     }
@@ -623,9 +636,14 @@ __device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint
     for (int u = 0; u < E; ++u) {
       if (sl[u] == kNone) continue;
       int c[3];
-      R d[3], q[3];
-      cell_and_frac<R>(sv[u][0], sv[u][1], sv[u][2], pid[u], L, c, d, q);
-      if (base + u * kT + threadIdx.x < n_own) {  // each particle is an own entry once
+      R d[3];
+      if constexpr (ABS) {
+        abs_cell_and_frac(sv[u][0], sv[u][1], sv[u][2], n, c, d);
+      } else {
+        R q[3];
+        cell_and_frac<R>(sv[u][0], sv[u][1], sv[u][2], pid[u], L, c, d, q);
+      }
+      if (!ABS && base + u * kT + threadIdx.x < n_own) {  // each particle is an own entry once
         bad += (c[0] / TX != tix || c[1] / TY != tiy || c[2] / TZ != tiz) ? 1u : 0u;
         nonfinite += is_finite3(sv[u][0], sv[u][1], sv[u][2]) ? 0u : 1u;
       }
@@ -646,7 +664,7 @@ __device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint
       for (int oz = 0; oz < 2; ++oz) {
         const int rz = oz ? r1[2] : r0[2];
         if (rz < 0) continue;
-        const double wz = (double)mass * (oz ? dd[2] : w0[2]);
+        const double wz = mass * (oz ? dd[2] : w0[2]);
 #pragma unroll
         for (int oy = 0; oy < 2; ++oy) {
           const int ry = oy ? r1[1] : r0[1];
@@ -1317,6 +1335,305 @@ __global__ __launch_bounds__(kT) void k_batch_scan_apply(const BatchDesc* __rest
   if (b == 0 && threadIdx.x == 0) *gmem(D->step) += 1;
 }
 
+
+// ------------------------------------------------------------------------------------------
+// reference-layout particles (absolute float32 positions (3, N_p) in any order), binned into tiles
+// for one call: density() deposits through own + halo entries, integrate() gathers through own ones
+//
+// The reference orders particles with the slowest grid axis fastest, so 64 consecutive ones lie in
+// 64 planes: one device atomic per corner and particle ran at 21 G/s (134 M atomics: 6.3 ms at
+// 256^3 particles on 512^3), and a gather from the grid fetched a cache line per sample (7.8 ms).
+// ------------------------------------------------------------------------------------------
+
+// Particle of thread `tid` of block `blk` in the binning passes.  side > 0 (N_p = side^3): a
+// wavefront takes 8 (fastest index) x 8 (middle index) particles, 16 x 16 cells at the usual
+// spacing of 2, so it meets one or two tiles, and its block 32 x 8, whole cache lines; side = 0
+// (N_p is no cube): consecutive particles.  False: none.
+__device__ __forceinline__ bool ref_particle(long blk, int tid, long np, int side, long& p) {
+  if (side == 0) {
+    p = blk * kT + tid;
+    return p < np;
+  }
+  const int kb = (side + 31) / 32, jb = (side + 7) / 8;
+  const long t = blk / kb;
+  const int k = (int)(blk - t * kb) * 32 + (tid >> 6) * 8 + (tid & 7);
+  const int i = (int)(t / jb), j = (int)(t - (long)i * jb) * 8 + ((tid >> 3) & 7);
+  p = ((long)i * side + j) * side + k;
+  return i < side && j < side && k < side;
+}
+inline long ref_blocks(long np, int side) {
+  return side == 0 ? (np + kT - 1) / kT : (long)((side + 31) / 32) * ((side + 7) / 8) * side;
+}
+
+// block -> tile with z fastest: the tiles of one (x, y) column hold the particles of the same
+// cache lines of the reference's arrays, so they share them in one L2
+__device__ __forceinline__ int ref_tile(const TileGeom& G) {
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const int tz = b % G.ntz, r = b / G.ntz, tx = r % G.ntx, ty = r / G.ntx;
+  return (tz * G.nty + ty) * G.ntx + tx;
+}
+
+// Places for the active lanes' keys: a run of active lanes with equal keys gets consecutive places
+// from one cursor atomic issued by its first lane.  All runs of a wavefront share one atomic
+// instruction, so its time does not grow with the number of distinct keys (WaveReserve waits for an
+// atomic per key beyond its first ones), and lanes in an order that follows the grid form few runs:
+// 7.6 M clustered particles of a truncated 200^3 lattice on 384^3, count + scatter 310 -> 250 us.
+// issue() leaves the atomic in flight until finish() reads it; every lane of the wavefront must reach
+// both.
+struct RunReserve {
+  uint32_t res;   // atomic result, held by the run's first lane
+  int head;       // first lane of this lane's run
+  uint32_t rank;  // place within the run
+
+  template <bool RESULT>
+  __device__ __forceinline__ void issue(uint32_t* __restrict__ cursors, uint32_t key, bool active) {
+    const int lane = __lane_id();
+    const unsigned long long act = __ballot(active), lt = (1ull << lane) - 1ull, below = act & lt;
+    const uint32_t prev = __shfl(key, below ? 63 - __clzll((long long)below) : lane);
+    const bool first = active && (below == 0ull || prev != key);
+    const unsigned long long heads = __ballot(first), upto = heads & (lt | (1ull << lane)), after = heads & ~upto;
+    head = upto ? 63 - __clzll((long long)upto) : lane;
+    const unsigned long long span = after ? (after & (~after + 1ull)) - 1ull : ~0ull;  // lanes before the next run
+    res = 0u;
+    if (first) {
+      const uint32_t len = (uint32_t)__popcll(act & span & ~lt);
+      if (RESULT) res = atomicAdd(&cursors[key], len);
+      else atomicAdd(&cursors[key], len);
+    }
+    rank = (uint32_t)__popcll(below & ~((1ull << head) - 1ull));
+  }
+  __device__ __forceinline__ uint32_t finish() const { return (uint32_t)__shfl((int)res, head) + rank; }
+};
+
+// Binning of one call's particles, in one of two forms.
+// SCATTER = false counts the entries of every key, true places them at offsets[key] + a range of the
+// key's cursor.  HALO: also the halo keys of the tiles the cloud reaches (the deposit); the gather
+// needs own keys only.
+
+// Up to kRefLdsKeys keys: the block counts its kRefP particles per thread in LDS and takes one device
+// atomic per key it met; places within the block's range are LDS atomics.  On small grids the
+// counters are few and device atomics of every wavefront queue up at the same addresses: the binning
+// and push of 133 k clustered particles on 96^3 took 138 us with the atomics of k_ref_bin, 53 us so;
+// 885 k on 192^3 155 and 82 us.  8192 keys (own and halo at 256^3) are 32 KB of LDS; the next grid,
+// 384^3, would take 110 KB and leave one block per CU.
+constexpr int kRefP = 4;
+constexpr int kRefLdsKeys = 8192;
+
+template <int TX, int TY, int TZ, bool HALO, bool SCATTER>
+__global__ __launch_bounds__(kT) void k_ref_bin_lds(const float* __restrict__ pos, long np, int side, int n, TileGeom G,
+                                                    uint32_t* __restrict__ counts,
+                                                    const uint32_t* __restrict__ offsets,
+                                                    uint32_t* __restrict__ entries, uint32_t capacity) {
+  extern __shared__ uint32_t table[];
+  const int keys = (HALO ? 2 : 1) * G.ntiles;
+  long p[kRefP];
+  int t[kRefP][3], up[kRefP][3];
+  bool valid[kRefP];
+#pragma unroll
+  for (int u = 0; u < kRefP; ++u) {
+    valid[u] = ref_particle((long)blockIdx.x * kRefP + u, threadIdx.x, np, side, p[u]);
+    int c[3] = {0, 0, 0};
+    float d[3];
+    if (valid[u]) abs_cell_and_frac(pos[p[u]], pos[np + p[u]], pos[2 * np + p[u]], n, c, d);
+    tile_of<TX, TY, TZ>(c, G, t[u], up[u]);
+  }
+  for (int k = threadIdx.x; k < keys; k += kT) table[k] = 0u;
+  __syncthreads();
+  auto each = [&](auto&& f) {
+#pragma unroll
+    for (int u = 0; u < kRefP; ++u) {
+      if (!valid[u]) continue;
+      f(target_key(t[u], 0, G), u);
+      if (HALO && (up[u][0] | up[u][1] | up[u][2])) {
+#pragma unroll 1
+        for (int o = 1; o < 8; ++o)
+          if (target_active(up[u], o)) f(target_key(t[u], o, G), u);
+      }
+    }
+  };
+  each([&](uint32_t key, int) { atomicAdd(&table[key], 1u); });
+  __syncthreads();
+  for (int k = threadIdx.x; k < keys; k += kT) {
+    const uint32_t cnt = table[k];
+    if (!cnt) continue;
+    if (SCATTER) table[k] = offsets[k] + atomicAdd(&counts[k], cnt);
+    else atomicAdd(&counts[k], cnt);
+  }
+  if (!SCATTER) return;
+  __syncthreads();
+  each([&](uint32_t key, int u) {
+    const uint32_t at = atomicAdd(&table[key], 1u);
+    if (at < capacity) entries[at] = (uint32_t)p[u];
+  });
+}
+
+// More keys: device atomics from every wavefront, one per run of equal keys
+template <int TX, int TY, int TZ, bool HALO, bool SCATTER>
+__global__ __launch_bounds__(kT) void k_ref_bin(const float* __restrict__ pos, long np, int side, int n, TileGeom G,
+                                                uint32_t* __restrict__ counts, const uint32_t* __restrict__ offsets,
+                                                uint32_t* __restrict__ entries, uint32_t capacity) {
+  long p;
+  const bool valid = ref_particle(blockIdx.x, threadIdx.x, np, side, p);
+  int c[3] = {0, 0, 0}, t[3], up[3];
+  float d[3];
+  if (valid) abs_cell_and_frac(pos[p], pos[np + p], pos[2 * np + p], n, c, d);
+  tile_of<TX, TY, TZ>(c, G, t, up);
+  // halo keys only in wavefronts that have any (wave-uniform)
+  const bool any_halo = HALO && __ballot(valid && (up[0] | up[1] | up[2])) != 0ull;
+  RunReserve r[HALO ? 8 : 1];
+  uint32_t beg[HALO ? 8 : 1];
+  r[0].template issue<SCATTER>(counts, target_key(t, 0, G), valid);
+  if (SCATTER && valid) beg[0] = offsets[target_key(t, 0, G)];
+  if constexpr (HALO) {
+    if (any_halo) {
+#pragma unroll
+      for (int o = 1; o < 8; ++o) {
+        const bool act = valid && target_active(up, o);
+        const uint32_t key = act ? target_key(t, o, G) : 0u;
+        r[o].template issue<SCATTER>(counts, key, act);
+        if (SCATTER && act) beg[o] = offsets[key];
+      }
+    }
+  }
+  if constexpr (SCATTER) {
+    const uint32_t at = r[0].finish() + beg[0];
+    if (valid && at < capacity) entries[at] = (uint32_t)p;
+    if constexpr (HALO) {
+      if (any_halo) {
+#pragma unroll
+        for (int o = 1; o < 8; ++o) {
+          const uint32_t ah = r[o].finish() + beg[o];
+          if (valid && target_active(up, o) && ah < capacity) entries[ah] = (uint32_t)p;
+        }
+      }
+    }
+  }
+}
+
+template <int TX, int TY, int TZ>
+__global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ pos, float* __restrict__ rho, double mass,
+                                                    Lattice L, TileGeom G, const uint32_t* __restrict__ offsets,
+                                                    const uint32_t* __restrict__ entries, uint32_t capacity) {
+  __shared__ double acc[deposit_lds_cells<TX, TY, TZ>()];
+  deposit_body<float, TX, TY, TZ, false, true>(pos, nullptr, rho, mass, L, G, offsets, entries, capacity, ref_tile(G),
+                                               acc, nullptr);
+}
+
+// integrate.py:15-97 for the particles of one tile, in place: the potential of the tile and its
+// -1/+2 stencil margin staged in LDS, the arithmetic of k_ref_integrate term by term
+template <int TX, int TY, int TZ>
+__global__ __launch_bounds__(kT) void k_ref_push(float* __restrict__ pos, float* __restrict__ vel, long np, int n,
+                                                 double a, double fa1, double da, const float* __restrict__ phi,
+                                                 TileGeom G, const uint32_t* __restrict__ offsets,
+                                                 const uint32_t* __restrict__ entries, uint32_t capacity) {
+  constexpr int BX = TX + 3, BY = TY + 3, BZ = TZ + 3, PLANE = BX * BY;
+  constexpr int NW = kT / 64, PL = (PLANE + 63) / 64, ZIT = (BZ + NW - 1) / NW, E = 2;
+  __shared__ float box[BX * BY * BZ];
+  const int tile = ref_tile(G);
+  uint32_t beg, end;
+  tile_range(offsets, capacity, tile, beg, end);
+  if (beg == end) return;
+  const int tix = tile % G.ntx, tiy = (tile / G.ntx) % G.nty, tiz = tile / (G.ntx * G.nty);
+  const int o0[3] = {tix * TX, tiy * TY, tiz * TZ};
+  const size_t nn = (size_t)n;
+  uint32_t sl[E];
+  float xv[E][3], vv[E][3];
+  auto load_entries = [&](uint32_t base) {
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const uint32_t e = base + u * kT + threadIdx.x;
+      sl[u] = e < end ? min(entries[e], (uint32_t)(np - 1)) : kNone;
+    }
+  };
+  auto load_state = [&]() {
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        xv[u][q] = sl[u] != kNone ? pos[q * np + sl[u]] : 0.f;
+        vv[u][q] = sl[u] != kNone ? vel[q * np + sl[u]] : 0.f;
+      }
+  };
+  load_entries(beg);
+  {
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t off[PL];
+#pragma unroll
+    for (int k = 0; k < PL; ++k) {
+      const int e = k * 64 + lane;
+      const int by = e / BX, x = e - by * BX;
+      off[k] = e < PLANE ? (uint32_t)(fold(o0[1] - 1 + by, n) * n + fold(o0[0] - 1 + x, n)) : 0u;
+    }
+    float tmp[ZIT][PL];
+#pragma unroll
+    for (int it = 0; it < ZIT; ++it) {
+      const int bz = wv + NW * it;
+      if (bz < BZ) {
+        const float* plane = phi + (size_t)fold(o0[2] - 1 + bz, n) * nn * nn;
+#pragma unroll
+        for (int k = 0; k < PL; ++k)
+          if (k * 64 + lane < PLANE) tmp[it][k] = plane[off[k]];
+      }
+    }
+    load_state();
+#pragma unroll
+    for (int it = 0; it < ZIT; ++it) {
+      const int bz = wv + NW * it;
+      if (bz < BZ) {
+#pragma unroll
+        for (int k = 0; k < PL; ++k)
+          if (k * 64 + lane < PLANE) box[bz * PLANE + k * 64 + lane] = tmp[it][k];
+      }
+    }
+  }
+  __syncthreads();
+  const double kick = da * fa1, a1 = (a + da) * (a + da), dn = (double)n;
+  for (uint32_t base = beg; base < end; base += kT * E) {
+    if (base != beg) {
+      load_entries(base);
+      load_state();
+    }
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      if (sl[u] == kNone) continue;
+      int b[3];
+      float x[3];
+      double d[3];
+      const int T[3] = {TX, TY, TZ};
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        x[q] = wrap_pos<float>(xv[u][q], float(n));
+        const int c = cell_of<float>(x[q], n);  // integrate.py:20
+        d[q] = (double)x[q] - (double)c;        // integrate.py:36-38
+        b[q] = min(max(c - o0[q], 0), T[q] - 1);  // own entries lie in the tile; the clamp keeps reads inside the box
+      }
+      const double tx = 1 - d[0], ty = 1 - d[1], tz = 1 - d[2];
+      const float t8[8] = {float(tx * ty * tz),     float(d[0] * ty * tz),   float(tx * d[1] * tz),
+                           float(tx * ty * d[2]),   float(d[0] * d[1] * tz), float(d[0] * ty * d[2]),
+                           float(tx * d[1] * d[2]), float(d[0] * d[1] * d[2])};  // integrate.py:44-51
+      const float* bp = box + ((b[2] + 1) * BY + b[1] + 1) * BX + b[0] + 1;
+      constexpr int step[3] = {1, BX, PLANE};
+#pragma unroll
+      for (int dir = 0; dir < 3; ++dir) {  // integrate.py:84-92
+        auto diff = [&](int off) { return -bp[off + step[dir]] + bp[off - step[dir]]; };
+        const float g = diff(0) * t8[0] + diff(1) * t8[1] + diff(BX) * t8[2] + diff(PLANE) * t8[3] +
+                        diff(BX + 1) * t8[4] + diff(PLANE + 1) * t8[5] + diff(PLANE + BX) * t8[6] +
+                        diff(PLANE + BX + 1) * t8[7];
+        const double gp = (double)g / 2.;
+        const float v = float((double)vv[u][dir] + kick * gp);  // integrate.py:94
+        double r = (double)x[dir] + da * (double)v / a1 * fa1;  // integrate.py:95, modulo n
+        if (!(r >= 0.0 && r < dn)) {
+          r = fmod(r, dn);
+          if (r < 0.0) r += dn;
+        }
+        vel[dir * np + sl[u]] = v;
+        pos[dir * np + sl[u]] = float(r);
+      }
+    }
+  }
+}
+
 }  // namespace
 
 
@@ -1392,6 +1709,14 @@ static bool tile_scatter_on(const TileGeom& G, const Bins& B) { return B.tile_sc
     else return hipErrorInvalidValue;                                                               \
   } while (0)
 
+// tile shapes of the reference-layout kernels (16^3 wherever it divides the grid, else 8^3)
+#define PM_REF_TILE_DISPATCH(G, CALL)                                    \
+  do {                                                                   \
+    if ((G).tx == 16 && (G).ty == 16 && (G).tz == 16) CALL(16, 16, 16);  \
+    else if ((G).tx == 8 && (G).ty == 8 && (G).tz == 8) CALL(8, 8, 8);   \
+    else return hipErrorInvalidValue;                                    \
+  } while (0)
+
 template <typename R>
 hipError_t bins_count(const PState<R>& p, const Lattice& L, const TileGeom& G, const Bins& B, hipStream_t st) {
 #define PM_L(X, Y, Z) k_bin_count<R, X, Y, Z><<<blocks_for(L.np), kT, 0, st>>>(p.s, p.id, L, G, B.counts)
@@ -1429,6 +1754,70 @@ hipError_t bins_scatter(const PState<R>& p, const Lattice& L, const TileGeom& G,
   k_bin_scatter<R, X, Y, Z><<<blocks_for(L.np), kT, 0, st>>>(p.s, p.id, L, G, B.offsets, B.cursors, B.entries, \
                                                              B.capacity, B.health)
   PM_TILE_DISPATCH(G, PM_L);
+#undef PM_L
+  return hipGetLastError();
+}
+
+bool ref_tiles_ok(long np, const TileGeom& G) { return G.ntiles > 0 && 8 * (uint64_t)np < (uint64_t)UINT32_MAX; }
+
+// bins the particles of one call (own entries, and the halo ones the deposit needs)
+static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const TileGeom& G, const Bins& B,
+                          hipStream_t st) {
+  int side = (int)std::lround(std::cbrt((double)np));
+  if ((long)side * side * side != np) side = 0;
+  const long nb = ref_blocks(np, side);
+  const long nbl = (nb + kRefP - 1) / kRefP;
+  const int keys = (halo ? 2 : 1) * G.ntiles;
+  const bool lds = keys <= kRefLdsKeys;
+  // the counts and the scan's ticket after them (never captured: the callers synchronise)
+  if (hipError_t e = hipMemsetAsync(B.counts, 0, (2 * (size_t)G.ntiles + 1) * sizeof(uint32_t), st)) return e;
+#define PM_ONE(X, Y, Z, HALO, SCATTER, CTR)                                                                          \
+  do {                                                                                                               \
+    if (lds)                                                                                                         \
+      k_ref_bin_lds<X, Y, Z, HALO, SCATTER>                                                                          \
+          <<<nbl, kT, keys * sizeof(uint32_t), st>>>(pos, np, side, n, G, CTR, B.offsets, B.entries, B.capacity);    \
+    else                                                                                                             \
+      k_ref_bin<X, Y, Z, HALO, SCATTER><<<nb, kT, 0, st>>>(pos, np, side, n, G, CTR, B.offsets, B.entries, B.capacity); \
+  } while (0)
+#define PM_L(X, Y, Z)                                        \
+  do {                                                       \
+    if (halo) PM_ONE(X, Y, Z, true, false, B.counts);        \
+    else PM_ONE(X, Y, Z, false, false, B.counts);            \
+  } while (0)
+  PM_REF_TILE_DISPATCH(G, PM_L);
+#undef PM_L
+  if (hipError_t e = bins_scan(G, B, st)) return e;
+#define PM_L(X, Y, Z)                                        \
+  do {                                                       \
+    if (halo) PM_ONE(X, Y, Z, true, true, B.cursors);        \
+    else PM_ONE(X, Y, Z, false, true, B.cursors);            \
+  } while (0)
+  PM_REF_TILE_DISPATCH(G, PM_L);
+#undef PM_L
+#undef PM_ONE
+  return hipGetLastError();
+}
+
+hipError_t ref_density_tiles(const float* pos, long np, int n, double mass, float* rho, const TileGeom& G,
+                             const Bins& B, hipStream_t st) {
+  if (hipError_t e = ref_bin(pos, np, n, true, G, B, st)) return e;
+  Lattice L{};
+  L.n = n;
+  L.np = np;
+#define PM_L(X, Y, Z) \
+  k_ref_deposit<X, Y, Z><<<G.ntiles, kT, 0, st>>>(pos, rho, mass, L, G, B.offsets, B.entries, B.capacity)
+  PM_REF_TILE_DISPATCH(G, PM_L);
+#undef PM_L
+  return hipGetLastError();
+}
+
+hipError_t ref_integrate_tiles(float* pos, float* vel, long np, int n, double a, double fa1, double da,
+                               const float* phi, const TileGeom& G, const Bins& B, hipStream_t st) {
+  if (hipError_t e = ref_bin(pos, np, n, false, G, B, st)) return e;
+#define PM_L(X, Y, Z)                                                                                     \
+  k_ref_push<X, Y, Z><<<G.ntiles, kT, 0, st>>>(pos, vel, np, n, a, fa1, da, phi, G, B.offsets, B.entries, \
+                                               B.capacity)
+  PM_REF_TILE_DISPATCH(G, PM_L);
 #undef PM_L
   return hipGetLastError();
 }
