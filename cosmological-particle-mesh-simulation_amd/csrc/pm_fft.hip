@@ -297,13 +297,13 @@ __device__ __forceinline__ void twiddle_row(T (&v)[M], const T* tw, int f) {
 template <typename R> struct PencilAddr {
   cpx<R>* base;
   long stride_n, stride_w;
-  long stride_blk;  // from row r to row r + kThreads / W of a column
+  long stride_blk;  // from row r to row r + ROWS of a column
   int contig;
   int kx0, dkx, ky0, dky;
   long tail;  // elements of the array from base to its end
 };
 
-template <typename R, int N, int W = pencil_w<R, N>()>
+template <typename R, int N, int W = pencil_w<R, N>(), int ROWS = kThreads / W>
 __device__ __forceinline__ PencilAddr<R> pencil_addr(cpx<R>* H, cpx<R>* Q, const PencilSeg& s0, const PencilSeg& s1,
                                                      long blk) {
   const bool first = blk < s0.nblk;
@@ -314,7 +314,7 @@ __device__ __forceinline__ PencilAddr<R> pencil_addr(cpx<R>* H, cpx<R>* Q, const
   p.contig = s.contig;
   p.stride_n = s.stride_n;
   p.stride_w = s.stride_w;
-  p.stride_blk = s.stride_blk ? s.stride_blk : (long)(kThreads / W) * (s.contig ? s.stride_n : 1);
+  p.stride_blk = s.stride_blk ? s.stride_blk : (long)ROWS * (s.contig ? s.stride_n : 1);
   if (s.contig) {
     const long o = blk / s.ncol_blk, c = blk - o * s.ncol_blk;
     const long oo = s.outer_stride_hi ? (o / kPencilTile) * s.outer_stride_hi + (o % kPencilTile) * s.outer_stride
@@ -340,17 +340,22 @@ __device__ __forceinline__ PencilAddr<R> pencil_addr(cpx<R>* H, cpx<R>* Q, const
 // to the end of its array (out-of-range accesses read 0 and write nothing), so each element's
 // address is a per-thread VGPR offset plus a block-uniform SGPR offset.
 using u32x2 = unsigned int __attribute__((ext_vector_type(2)));
+using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* base, long bytes) {
   // 0x00020000: the buffer-resource format word of the gfx9 family (raw 32-bit dwords)
   // num_records is an unsigned 32-bit byte count; the register pass keeps every offset below 4 GiB
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0,
                                            (int)(uint32_t)(bytes < 0xffffffffL ? bytes : 0xffffffffL), 0x00020000);
 }
-__device__ __forceinline__ cpx<float> buffer_load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  return __builtin_bit_cast(cpx<float>, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+template <typename T> __device__ __forceinline__ T buffer_load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, int voff, int soff, cpx<float> v) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, voff, soff, 0);
+}
+__device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, int voff, int soff, cpx<double> v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, soff, 0);
 }
 
 // elements of one pencil per thread
@@ -412,92 +417,39 @@ __device__ __forceinline__ void pencil_load(const PencilAddr<R>& p, cpx<R>* lds,
   }
 }
 
-// Four-step transform of the staged pencil with the columns' DFTs in registers: N = A * TT,
-// TT = threads per column.  Thread t of a column takes x[a TT + t] (a < A), does the A-point
-// DFT and the twiddle W_N^{t ka}; after one exchange through LDS it takes, for each of its
-// J = A / TT values ka = t + j TT, the TT values Y[t'][ka] and does the TT-point DFT, giving
-// X[ka + A kb].  The inverse of the fused z pass runs the same steps backwards from there.
+// Four-step transform with the columns' DFTs in registers: N = A * TT, TT = threads per column.
+// Thread t of a column takes x[a TT + t] (a < A), does the A-point DFT and the twiddle W_N^{t ka};
+// after one exchange through LDS it takes, for each of its J = A / TT values ka = t + j TT, the TT
+// values Y[t'][ka] and does the TT-point DFT, giving X[ka + A kb].  The inverse of the fused z pass
+// runs the same steps backwards from there.
+// Shape: W columns per block (whole 128-byte row segments), NT = W * TT threads.  FP64 takes 16
+// threads per column like FP32 but half the columns, so a block of 128 threads holds A = 32 complex
+// values per thread (N = 512) in 256 registers and its exchange slice is 37 KB: four blocks per CU.
+// FP64 runs only the z pass this way.  As an LDS pass its pencil, tables and twiddles left one block
+// per CU, so loads, the two transforms and stores took turns: 1116 (plain) / 1160 (deconvolved) /
+// 1580 us (caller's grid) at 512^3 against 666 / 701 / 848, 72 / 71 against 58 / 62 at 256^3.  The y
+// passes have LDS for two blocks and stay there: 373 and 364 us, 393 and 391 in registers.
+template <typename R, int N> struct RegShape {
+  static constexpr int W = pencil_w<R, N>();
+  static constexpr int TT = sizeof(R) == 4 ? kThreads / W : 16;
+  static constexpr int NT = W * TT;
+};
 template <typename R, int N> constexpr bool reg_transform() {
-  constexpr int W = pencil_w<R, N>();
-  constexpr int TT = kThreads / W;
+  using S = RegShape<R, N>;
   // (the raw-buffer offsets of the register pass are unsigned 32-bit: a column spans at most
-  // (N - 1) N (N/2) 8 bytes < 4 GiB for N <= 1024)
-  return sizeof(R) == 4 && kThreads % W == 0 && N % TT == 0 && (N / TT) % TT == 0 && (TT == 16 || TT == 32) &&
-         N / TT <= 32 && N <= 1024;
+  // (N - 1) N (N/2) complex values, < 4 GiB for N <= 1024 at FP32 and N <= 512 at FP64)
+  return S::NT % 64 == 0 && N % S::TT == 0 && (N / S::TT) % S::TT == 0 && (S::TT == 16 || S::TT == 32) &&
+         N / S::TT <= 32 && (sizeof(R) == 4 ? N <= 1024 : S::W == 8 && N <= 512);
 }
 
-template <typename R, int N, int MODE>
-__device__ __forceinline__ void pencil_transform_reg(const PencilAddr<R>& p, const GreenArgs& g, R coef, cpx<R>* lds,
-                                                     const cpx<R>* tw, const R* s2, const R* wd, int tid) {
-  using T = cpx<R>;
-  constexpr int W = pencil_w<R, N>();
-  constexpr int SN = W + 1;
-  constexpr int TT = kThreads / W;
-  constexpr int A = N / TT;
-  constexpr int J = A / TT;
-  constexpr int S1 = MODE == 1 ? +1 : -1;
-  const int w = tid % W, t = tid / W;
-  T v[A];
-#pragma unroll
-  for (int a = 0; a < A; ++a) v[a] = lds[(a * TT + t) * SN + w];
-  reg_dft<S1, A>(v);
-#pragma unroll
-  for (int ka = 1; ka < A; ++ka) {
-    const T c = tw[(t * ka) % N];
-    v[ka] = S1 < 0 ? cmul(v[ka], c) : cmulc(v[ka], c);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int ka = 0; ka < A; ++ka) lds[(ka * TT + t) * SN + w] = v[ka];
-  __syncthreads();
-  T u[J][TT];
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int ka = t + j * TT;
-#pragma unroll
-    for (int q = 0; q < TT; ++q) u[j][q] = lds[(ka * TT + q) * SN + w];
-    reg_dft<S1, TT>(u[j]);
-  }
-  if constexpr (MODE != 0) {
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-#pragma unroll
-      for (int kb = 0; kb < TT; ++kb) lds[(t + j * TT + A * kb) * SN + w] = u[j][kb];
-    __syncthreads();
-  } else {
-    // k-space operator on X[k], k = ka + A kb the z mode, then the inverse back to x
-    const int kx = p.kx0 + w * p.dkx, ky = p.ky0 + w * p.dky;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int ka = t + j * TT;
-#pragma unroll
-      for (int kb = 0; kb < TT; ++kb) u[j][kb] = cscale(u[j][kb], green_factor<R>(kx, ky, ka + A * kb, N, g, coef, s2, wd));
-      reg_dft<+1, TT>(u[j]);
-      twiddle_row<+1, N, TT, 8>(u[j], tw, ka);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-#pragma unroll
-      for (int q = 0; q < TT; ++q) lds[((t + j * TT) * TT + q) * SN + w] = u[j][q];
-    __syncthreads();
-#pragma unroll
-    for (int ka = 0; ka < A; ++ka) v[ka] = lds[(ka * TT + t) * SN + w];
-    reg_dft<+1, A>(v);
-    __syncthreads();
-#pragma unroll
-    for (int a = 0; a < A; ++a) lds[(a * TT + t) * SN + w] = v[a];
-    __syncthreads();
-  }
-}
-
-// the transform(s) of a staged pencil, in LDS (ends with the LDS holding the result)
 // Passes that run the register transform: every y and z pass up to N = 512; above that only
 // the fused z pass (its LDS slice takes 82-90 KB, one workgroup per CU: the y passes are faster
 // as LDS Stockham passes there, the z pass with its 4 MiB column stride is not)
-template <typename R, int N, int MODE> constexpr bool reg_pass() { return reg_transform<R, N>() && (N <= 512 || MODE == 0); }
+template <typename R, int N, int MODE> constexpr bool reg_pass() {
+  return reg_transform<R, N>() && ((sizeof(R) == 4 && N <= 512) || MODE == 0);
+}
 
+// the transform(s) of a staged pencil, in LDS (ends with the LDS holding the result)
 template <typename R, int N, int MODE, int W = pencil_w<R, N>()>
 __device__ __forceinline__ void pencil_transform(const PencilAddr<R>& p, const GreenArgs& g, R coef, cpx<R>* lds,
                                                  const cpx<R>* tw, const R* s2, const R* wd, int tid) {
@@ -505,9 +457,7 @@ __device__ __forceinline__ void pencil_transform(const PencilAddr<R>& p, const G
   constexpr int L = N;
   constexpr int SN = W + 1;
   constexpr int NT = kThreads;
-  if constexpr (W == pencil_w<R, N>() && reg_pass<R, N, MODE>()) {
-    pencil_transform_reg<R, N, MODE>(p, g, coef, lds, tw, s2, wd, tid);
-  } else if constexpr (MODE == -1) {
+  if constexpr (MODE == -1) {
     fft_passes<T, L, 1, -1, W, SN, NT, 1>(lds, tw, tid);
   } else if constexpr (MODE == 1) {
     fft_passes<T, L, 1, +1, W, SN, NT, 1>(lds, tw, tid);
@@ -548,7 +498,7 @@ __device__ __forceinline__ void pencil_store(const PencilAddr<R>& p, const cpx<R
 template <typename R, int N, int MODE>
 __device__ __forceinline__ void pencil_tables(const cpx<R>* __restrict__ twg, const R* __restrict__ s2g,
                                               const R* __restrict__ wdg, cpx<R>* tw, R* s2, R* wd, int tid) {
-  for (int i = tid; i < N; i += kThreads) {
+  for (int i = tid; i < N; i += kThreads) {  // (kThreads threads: the LDS tables go with FP32 shapes)
     tw[i] = twg[i];
     if constexpr (MODE == 0) {
       s2[i] = s2g[i];
@@ -598,8 +548,7 @@ __global__ __launch_bounds__(kThreads) void k_pencil(cpx<R>* H, cpx<R>* Q, Penci
 // pencil in LDS and more blocks stay resident.  Row r of a slice sits at r*SN + r/TT + w: the
 // extra word per TT rows spreads both the writers' and the readers' lanes over the banks.
 template <typename R, int N> constexpr int xslice_elems() {
-  constexpr int W = pencil_w<R, N>();
-  constexpr int TT = kThreads / W;
+  constexpr int W = RegShape<R, N>::W, TT = RegShape<R, N>::TT;
   return TT * TT * (W + 1) + TT;
 }
 
@@ -612,9 +561,8 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
                                                 const R* __restrict__ s2g, const R* __restrict__ wdg, long blk,
                                                 cpx<R>* xb, const cpx<R>* tw, const R* s2, const R* wd) {
   using T = cpx<R>;
-  constexpr int W = pencil_w<R, N>();
+  constexpr int W = RegShape<R, N>::W, TT = RegShape<R, N>::TT;
   constexpr int SN = W + 1;
-  constexpr int TT = kThreads / W;
   constexpr int A = N / TT;
   constexpr int J = A / TT;
   constexpr int S1 = MODE == 1 ? +1 : -1;
@@ -622,7 +570,7 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
   const int w = tid % W, t = tid / W;
   if constexpr (TAB_LDS)
     pencil_tables<R, N, MODE>(twg, s2g, wdg, const_cast<cpx<R>*>(tw), const_cast<R*>(s2), const_cast<R*>(wd), tid);
-  const PencilAddr<R> p = pencil_addr<R, N>(H, Q, s0, s1, blk);
+  const PencilAddr<R> p = pencil_addr<R, N, W, TT>(H, Q, s0, s1, blk);
   // element (n, w) of the pencil at byte n * sn8 + (w * sw) * 8 from its base
   const uint32_t sn8 = (uint32_t)((p.contig ? p.stride_n : 1) * (long)sizeof(T));
   const __amdgpu_buffer_rsrc_t buf = buffer_of(p.base, p.tail * (long)sizeof(T));
@@ -633,7 +581,7 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
   auto xrow = [&](int r) { return r * SN + r / TT + w; };
   T v[A];
 #pragma unroll
-  for (int a = 0; a < A; ++a) v[a] = buffer_load(buf, voff, roff(a * TT));
+  for (int a = 0; a < A; ++a) v[a] = buffer_load<T>(buf, voff, roff(a * TT));
   __syncthreads();  // tables in LDS
   reg_dft<S1, A>(v);
   twiddle_row<S1, N, A, 8>(v, tw, t);
@@ -657,12 +605,42 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
     // k-space operator on X[k], k = ka + A kb the z mode, then the same steps backwards
     const int kx = p.kx0 + w * p.dkx, ky = p.ky0 + w * p.dky;
     const R coef = R(coef_of(g));
-    if (g.from_grid || g.deconvolve) {
+    // green_factor(), each of its forms in a loop of its own (factors that live across a branch
+    // would cost the plain form's registers) with the loads of GB factors issued together
+    constexpr int GB = sizeof(R) == 8 ? 8 : TT;
+    if (g.from_grid) {
+      const uint32_t row = (uint32_t)N * N, g1 = (uint32_t)ky * N + kx;
+      const uint32_t g2 = (uint32_t)((N - ky) % N) * N + (N - kx) % N;  // the mode's conjugate
 #pragma unroll
       for (int j = 0; j < J; ++j)
 #pragma unroll
-        for (int kb = 0; kb < TT; ++kb)
-          u[j][kb] = cscale(u[j][kb], green_factor<R>(kx, ky, j * TT + t + A * kb, N, g, coef, s2, wd));
+        for (int k0 = 0; k0 < TT; k0 += GB) {
+          float fa[GB], fb[GB];
+#pragma unroll
+          for (int k = 0; k < GB; ++k) {
+            const int kz = j * TT + t + A * (k0 + k);
+            fa[k] = g.fgrid[kz * row + g1];
+            fb[k] = g.fgrid[((N - kz) % N) * row + g2];
+          }
+#pragma unroll
+          for (int k = 0; k < GB; ++k) u[j][k0 + k] = cscale(u[j][k0 + k], coef * R(0.5) * (R(fa[k]) + R(fb[k])));
+        }
+    } else if (g.deconvolve) {
+      const R sxy = s2[kx] + s2[ky], wxy = wd[kx] * wd[ky];
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int k0 = 0; k0 < TT; k0 += GB) {
+          R den[GB], w[GB];
+#pragma unroll
+          for (int k = 0; k < GB; ++k) {
+            den[k] = sxy + s2[j * TT + t + A * (k0 + k)];
+            w[k] = wxy * wd[j * TT + t + A * (k0 + k)];
+          }
+#pragma unroll
+          for (int k = 0; k < GB; ++k)
+            u[j][k0 + k] = cscale(u[j][k0 + k], den[k] > R(0) ? coef / den[k] * w[k] : R(0));
+        }
     } else {  // the plain Green's function: green_factor() without its optional terms
       const R sxy = s2[kx] + s2[ky];
 #pragma unroll
@@ -696,13 +674,13 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
 }
 
 template <typename R, int N, int MODE>
-__global__ __launch_bounds__(kThreads) void k_pencil_reg(cpx<R>* H, cpx<R>* Q, PencilSeg s0, PencilSeg s1, GreenArgs g,
-                                                         const cpx<R>* __restrict__ twg, const R* __restrict__ s2g,
-                                                         const R* __restrict__ wdg) {
+__global__ __launch_bounds__((RegShape<R, N>::NT), sizeof(R) == 8 ? 2 : 1) void k_pencil_reg(
+    cpx<R>* H, cpx<R>* Q, PencilSeg s0, PencilSeg s1, GreenArgs g, const cpx<R>* __restrict__ twg,
+    const R* __restrict__ s2g, const R* __restrict__ wdg) {
   __shared__ cpx<R> xb[xslice_elems<R, N>()];
-  // above N = 512 the tables stay in global memory: with them the block's LDS (90 KB at
-  // N = 1024) allows one block per CU, without them two
-  constexpr bool kTabLds = N <= 512;
+  // above N = 512, and in FP64, the tables stay in global memory: with them the block's LDS (90 KB
+  // at N = 1024) allows one block per CU, without them two
+  constexpr bool kTabLds = sizeof(R) == 4 && N <= 512;
   __shared__ cpx<R> tw[kTabLds ? N : 1];
   __shared__ R s2[kTabLds && MODE == 0 ? N : 1];
   __shared__ R wd[kTabLds && MODE == 0 ? N : 1];
@@ -791,12 +769,12 @@ template <typename R, int N> PencilSeg z_tiled(PencilSeg a) {  // outer y, rows 
   return a;
 }
 
-// The alternative shape of a Stockham pencil pass: half its default columns per block (less LDS,
-// more blocks per CU), for N >= 64 in the plain layout; 0 where there is none (register passes,
-// the page-tiled passes, widths below 2).
+// The alternative shape of a pencil pass: a Stockham pass with half the default columns per block
+// (less LDS, more blocks per CU), for N >= 64 in the plain layout; 0 where there is none (FP32
+// register passes, the page-tiled passes, widths below 2).
 template <typename R, int N, int MODE> constexpr int pencil_alt_w() {
   constexpr int W2 = pencil_w<R, N>() / 2;
-  if constexpr (reg_pass<R, N, MODE>() || tiled_spectrum<R, N>() || N < 64 || W2 < 2) return 0;
+  if constexpr ((sizeof(R) == 4 && reg_pass<R, N, MODE>()) || tiled_spectrum<R, N>() || N < 64 || W2 < 2) return 0;
   else return ((N / 2) % W2 == 0 && N % W2 == 0 && kThreads % W2 == 0) ? W2 : 0;
 }
 
@@ -830,7 +808,7 @@ hipError_t launch_pencil(cpx<R>* H, cpx<R>* Q, bool zaxis, const GreenArgs& g, c
       if (zaxis) {  // in place on the tiled array
         const PencilSeg at = z_tiled<R, N>(a);
         if constexpr (reg_pass<R, N, MODE>())
-          k_pencil_reg<R, N, MODE><<<nb, kThreads, 0, st>>>(work, Q, at, b, g, tw, s2, wd);
+          k_pencil_reg<R, N, MODE><<<nb, RegShape<R, N>::NT, 0, st>>>(work, Q, at, b, g, tw, s2, wd);
         else
           k_pencil<R, N, MODE><<<nb, kThreads, 0, st>>>(work, Q, at, b, g, tw, s2, wd, nullptr, at);
       } else if (MODE < 0) {  // plain H -> tiled work
@@ -842,7 +820,7 @@ hipError_t launch_pencil(cpx<R>* H, cpx<R>* Q, bool zaxis, const GreenArgs& g, c
     }
   }
   if constexpr (reg_pass<R, N, MODE>()) {
-    k_pencil_reg<R, N, MODE><<<nb, kThreads, 0, st>>>(H, Q, a, b, g, tw, s2, wd);
+    k_pencil_reg<R, N, MODE><<<nb, RegShape<R, N>::NT, 0, st>>>(H, Q, a, b, g, tw, s2, wd);
   } else {
     k_pencil<R, N, MODE><<<nb, kThreads, 0, st>>>(H, Q, a, b, g, tw, s2, wd, nullptr, a);
   }
