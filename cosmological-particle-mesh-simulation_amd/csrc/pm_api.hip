@@ -665,6 +665,7 @@ struct pm_sim {
   Bins B{};
   hipStream_t stream = nullptr;
   bool has_state = false, rho_valid = false, phi_valid = false, bins_valid = false;
+  bool slot_order = false;      // the particles are stored in slot order (no step since they were set)
   bool spec_valid = false;      // the density slot holds the x spectrum of the current density
   // the forward y, z and inverse y passes in their alternative pencil shape (fft_pencil_cols;
   // picked by the autotuner or set by the caller)
@@ -917,6 +918,7 @@ template <typename R> int sim_step_impl(pm_sim* s, double a, double da, bool tab
                         s->L, s->G, s->B, tab, s->stream, edge));
   }
   s->cur ^= 1;
+  s->slot_order = false;
   {
     // the gather counted the entries of the new positions: finish their binning
     StageTimer t(s, ST_BIN);
@@ -997,6 +999,7 @@ template <typename R> int sim_run_graph(pm_sim* s, double& a, double da, int n_s
     PM_HIP(hipMemcpyAsync(s->d_step, &zero, sizeof(int), hipMemcpyHostToDevice, s->stream));
     int k = 0;
     for (; k + kGraphSteps <= chunk; k += kGraphSteps) {
+      s->slot_order = false;
       PM_HIP(hipGraphLaunch(s->graph[s->cur][s->gb], s->stream));
       s->phi_valid = true;
     }
@@ -1061,7 +1064,10 @@ template <typename R> int sim_autotune_impl(pm_sim* s, int reps, double* best_ms
       if (!e) {
         e = gkd_tiles<R>(cur_state<R>(s), state_buf<R>(s, s->cur ^ 1), (const R*)spec_slot(s), 0.0, 0.0, s->L, s->G, s->B,
                          StepTable{}, s->stream);
-        if (!e) s->cur ^= 1;
+        if (!e) {
+          s->cur ^= 1;
+          s->slot_order = false;
+        }
       }
       if (!e) e = bins_scan(s->G, s->B, s->stream, true);
       if (!e) e = bins_scatter<R>(cur_state<R>(s), s->L, s->G, s->B, s->stream, true);
@@ -1386,7 +1392,7 @@ PM_API int pm_sim_set_state(pm_sim* s, const void* pos, const void* vel, int dty
   hipError_t es = hipStreamSynchronize(s->stream);
   if (tmp) (void)hipFree(tmp);
   if (e != hipSuccess || es != hipSuccess) return fail(PM_E_HIP, "set_state failed: %s", hipGetErrorString(e ? e : es));
-  s->has_state = true;
+  s->has_state = s->slot_order = true;
   s->bins_valid = false;
   s->rho_valid = s->spec_valid = false;
   s->phi_valid = false;
@@ -1411,13 +1417,16 @@ PM_API int pm_sim_get_state(pm_sim* s, void* pos, void* vel, int dtype_bytes, in
     dv = (char*)tmp + bytes;
   }
   hipError_t e;
+  const bool slots = s->slot_order;
+  const int nz = s->G.ntz;
+  const hipStream_t st = s->stream;
   if (s->prec == 4) {
-    e = dtype_bytes == 4 ? sim_get_state<float, float>(cur_state<float>(s), (float*)dp, (float*)dv, s->L, s->stream)
-                         : sim_get_state<float, double>(cur_state<float>(s), (double*)dp, (double*)dv, s->L, s->stream);
+    e = dtype_bytes == 4 ? sim_get_state<float, float>(cur_state<float>(s), (float*)dp, (float*)dv, s->L, slots, nz, st)
+                         : sim_get_state<float, double>(cur_state<float>(s), (double*)dp, (double*)dv, s->L, slots, nz, st);
   } else {
-    e = dtype_bytes == 4 ? sim_get_state<double, float>(cur_state<double>(s), (float*)dp, (float*)dv, s->L, s->stream)
-                         : sim_get_state<double, double>(cur_state<double>(s), (double*)dp, (double*)dv, s->L,
-                                                         s->stream);
+    e = dtype_bytes == 4
+            ? sim_get_state<double, float>(cur_state<double>(s), (float*)dp, (float*)dv, s->L, slots, nz, st)
+            : sim_get_state<double, double>(cur_state<double>(s), (double*)dp, (double*)dv, s->L, slots, nz, st);
   }
   if (e == hipSuccess && !on_device) {
     e = hipMemcpyAsync(pos, dp, bytes, hipMemcpyDeviceToHost, s->stream);
@@ -1579,7 +1588,7 @@ PM_API int pm_sim_zeldovich(pm_sim* s, const double* amp, int64_t n_amp, double 
   (void)hipFree(d_amp);
   if (e != hipSuccess || es != hipSuccess)
     return fail(PM_E_HIP, "device initial conditions failed: %s", hipGetErrorString(e ? e : es));
-  s->has_state = true;
+  s->has_state = s->slot_order = true;
   s->rho_valid = s->bins_valid = s->phi_valid = s->spec_valid = false;
   return PM_OK;
 }
@@ -1989,6 +1998,7 @@ PM_API int pm_ensemble_run(pm_ensemble* e, double* a, const double* da, int n_st
     a[i] = acur[i];
     pm_sim* s = e->members[i];
     s->cur ^= done & 1;  // every step's gather switched the member's state buffer
+    if (done) s->slot_order = false;
     s->rho_valid = s->bins_valid = s->phi_valid = true;
     s->spec_valid = false;
   }
