@@ -1140,6 +1140,7 @@ PM_API int pm_sim_set_tiles(pm_sim* s, int tx, int ty, int tz) {
     return fail(PM_E_UNSUPPORTED, "tile shape %dx%dx%d is not instantiated", tx, ty, tz);
   if (s->ens && !(tx == 16 && ty == 16 && tz == 16) && (tx || ty || tz))
     return fail(PM_E_STATE, "ensemble members keep 16^3 tiles");
+  if (s->ens) tx = ty = tz = 16;  // the default of a member is the ensemble's shape
   return sim_use_tiles(s, make_tiles(s->L.n, s->prec, tx, ty, tz));
 }
 

@@ -106,7 +106,7 @@ struct Bins {
 // among those that divide the grid.
 #define PM_TILE_SHAPES(X) X(16, 16, 16) X(32, 16, 8) X(32, 8, 8) X(16, 16, 8) X(64, 8, 8) X(8, 8, 8)
 bool tile_shape_supported(int tx, int ty, int tz);
-// tiles of shape (tx, ty, tz) on an n^3 grid (all 0: the default 16^3); ntiles = 0 if unusable
+// tiles of shape (tx, ty, tz) on an n^3 grid (all 0: the default for n); ntiles = 0 if unusable
 TileGeom make_tiles(int n, int prec_bytes, int tx = 0, int ty = 0, int tz = 0);
 std::vector<TileGeom> tile_candidates(int n, int prec_bytes);
 int scan_blocks(const TileGeom& g);

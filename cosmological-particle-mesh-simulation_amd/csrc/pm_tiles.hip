@@ -161,32 +161,25 @@ __device__ __forceinline__ uint32_t* ts_base(uint32_t* counts, const TileGeom& G
 // bits 0-5) and its upper-face flags (bits 6-8), or kCodeFar when it moved beyond the
 // neighbourhood.
 constexpr uint32_t kCodeFar = 0x8000u;
-constexpr int kScatterT = 64;  // threads per block of the tile scatter (one wavefront per tile)
-constexpr int kScatterE = 4;   // particles per thread and batch in the tile scatter
+// Threads per tile of the tile scatter: one wavefront where the tiles fill the chip (more tiles in
+// flight), four on smaller grids, whose few tiles, some of them dense, would each be one long serial
+// chain (bin stage of a clustered 192^3 step in 16x16x8 tiles: 35.8 -> 27.7 us;
+// evenly spread particles 23.3 -> 22.7).
+constexpr int kScatterT = 64, kScatterWide = 256;
+constexpr int kScatterTiles = 16384;  // tiles from which on one wavefront each is enough
 
-// Adds 1 to ctr[key] for every active lane with one atomic per distinct key in the wavefront
-// and returns each lane's rank among all additions to its key (old value + lane prefix).
+// Adds 1 to ctr[key] for every active lane with one atomic per distinct key in the wavefront.
 // Must be reached by every lane of the wavefront.
-template <bool RESULT>
-__device__ __forceinline__ uint32_t wave_add(uint32_t* ctr, uint32_t key, bool active) {
+__device__ __forceinline__ void wave_add(uint32_t* ctr, uint32_t key, bool active) {
   const int lane = __lane_id();
   unsigned long long pending = __ballot(active);
-  uint32_t res = 0;
   while (pending) {
     const int leader = __ffsll((unsigned long long)pending) - 1;
     const uint32_t lkey = __shfl(key, leader);
     const unsigned long long same = __ballot(active && key == lkey) & pending;
-    if (RESULT) {
-      uint32_t base = 0;
-      if (lane == leader) base = atomicAdd(&ctr[lkey], (uint32_t)__popcll(same));
-      base = __shfl(base, leader);
-      if ((same >> lane) & 1ull) res = base + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-    } else {
-      if (lane == leader) atomicAdd(&ctr[lkey], (uint32_t)__popcll(same));
-    }
+    if (lane == leader) atomicAdd(&ctr[lkey], (uint32_t)__popcll(same));
     pending &= ~same;
   }
-  return res;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -206,7 +199,7 @@ __global__ __launch_bounds__(kT) void k_bin_count(const R* __restrict__ s, const
 #pragma unroll 1
   for (int o = 0; o < 8; ++o) {
     const bool act = valid && target_active(up, o);
-    wave_add<false>(counts, act ? target_key(t, o, G) : 0u, act);
+    wave_add(counts, act ? target_key(t, o, G) : 0u, act);
   }
 }
 
@@ -341,16 +334,17 @@ __global__ __launch_bounds__(kT) void k_bin_scatter(const R* __restrict__ s, con
 // and id).  Particles that moved beyond the neighbourhood were counted in the far counts; the
 // scan put them after the reserved ranges of each key, and they take a device cursor atomic on
 // keys recomputed from their stored state.
-template <typename R, int TX, int TY, int TZ>
+template <typename R, int TX, int TY, int TZ, int NT>
 __device__ __forceinline__ void tile_scatter_body(const R* __restrict__ s, const uint32_t* __restrict__ id,
                                                   const Lattice& L, const TileGeom& G,
                                                   const uint32_t* __restrict__ offsets, uint32_t* __restrict__ cursors,
                                                   uint32_t* __restrict__ entries, uint32_t capacity,
                                                   uint32_t* __restrict__ health, uint32_t* __restrict__ counts,
                                                   int tile, uint32_t* cur, uint32_t* lim) {
-  constexpr int NT = kScatterT, E = kScatterE, BPT = kBins / NT;
-  static_assert(kBins % NT == 0, "whole bins per thread");
+  constexpr int E = NT == 64 ? 4 : 2;  // particles per thread and batch
+  constexpr int BPT = (kBins + NT - 1) / NT;
   const long np = L.np;
+  const int lane = __lane_id();
   const uint32_t* wbase = ts_base(counts, G);
   const uint32_t* old = counts + ts_old_at(G.ntiles);
   const uint32_t end = min(min(old[tile + 1], capacity), (uint32_t)np), beg = min(old[tile], end);
@@ -359,7 +353,10 @@ __device__ __forceinline__ void tile_scatter_body(const R* __restrict__ s, const
   const int tc[3] = {tix, tiy, tiz};
   uint32_t w[BPT];
 #pragma unroll
-  for (int k = 0; k < BPT; ++k) w[k] = wbase[(size_t)tile * kBins + k * NT + threadIdx.x];
+  for (int k = 0; k < BPT; ++k) {
+    const int b = k * NT + threadIdx.x;
+    w[k] = b < kBins ? wbase[(size_t)tile * kBins + b] : kNone;
+  }
   const uint16_t* codes = reinterpret_cast<const uint16_t*>(id) + 2 * np;
   uint32_t code[E];
   auto load = [&](uint32_t base) {
@@ -379,8 +376,10 @@ __device__ __forceinline__ void tile_scatter_body(const R* __restrict__ s, const
       c = offsets[key] + w[k];
       l = offsets[key + 1];
     }
-    cur[b] = c;
-    lim[b] = l;
+    if (b < kBins) {
+      cur[b] = c;
+      lim[b] = l;
+    }
   }
   __syncthreads();
   uint32_t lost = 0;
@@ -393,14 +392,22 @@ __device__ __forceinline__ void tile_scatter_body(const R* __restrict__ s, const
       const bool near = valid && !(code[u] & kCodeFar);
       const int h0 = 2 * (int)(code[u] & 63u);
       const int up[3] = {(int)(code[u] >> 6) & 1, (int)(code[u] >> 7) & 1, (int)(code[u] >> 8) & 1};
-      // one LDS atomic per distinct bin of the wavefront (lanes of a tile mostly share their
-      // home bin: per-lane atomics on one address serialize)
+      // one LDS atomic instruction per corner offset: the lanes that share the first active lane's
+      // bin (mostly all: the tile's own) take one place each from that lane's add, the others add
+      // for themselves
 #pragma unroll
       for (int o = 0; o < 8; ++o) {
         const bool act = near && target_active(up, o);
-        if (!__ballot(act)) continue;  // wave-uniform
+        const unsigned long long mask = __ballot(act);
+        if (!mask) continue;  // wave-uniform
         const int b = corner_bin(h0, o);
-        const uint32_t pos = wave_add<true>(cur, (uint32_t)b, act);
+        const int first = __ffsll(mask) - 1;
+        const unsigned long long same = __ballot(act && b == __shfl(b, first));
+        const bool shared = (same >> lane) & 1ull;
+        uint32_t pos = 0u;
+        if (act && (!shared || lane == first)) pos = atomicAdd(&cur[b], shared ? (uint32_t)__popcll(same) : 1u);
+        const uint32_t base = (uint32_t)__shfl((int)pos, first);
+        if (shared) pos = base + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
         if (act) {
           if (pos < lim[b] && pos < capacity) entries[pos] = e;
           else ++lost;
@@ -426,8 +433,8 @@ __device__ __forceinline__ void tile_scatter_body(const R* __restrict__ s, const
   if (lost && health) atomicAdd(&health[PM_HEALTH_OVERFLOW], lost);
 }
 
-template <typename R, int TX, int TY, int TZ>
-__global__ __launch_bounds__(kScatterT) void k_tile_scatter(const R* __restrict__ s, const uint32_t* __restrict__ id,
+template <typename R, int TX, int TY, int TZ, int NT>
+__global__ __launch_bounds__(NT) void k_tile_scatter(const R* __restrict__ s, const uint32_t* __restrict__ id,
                                                             Lattice L, TileGeom G, const uint32_t* __restrict__ offsets,
                                                             uint32_t* __restrict__ cursors,
                                                             uint32_t* __restrict__ entries, uint32_t capacity,
@@ -436,8 +443,8 @@ __global__ __launch_bounds__(kScatterT) void k_tile_scatter(const R* __restrict_
   __shared__ uint32_t cur[kBins], lim[kBins];
   // each XCD walks its run of tiles backwards, so it starts on what the gather (walking the same
   // runs forward) wrote last and the last-level cache still holds
-  tile_scatter_body<R, TX, TY, TZ>(s, id, L, G, offsets, cursors, entries, capacity, health, counts,
-                                   xcd_block(blockIdx.x, gridDim.x, 1), cur, lim);
+  tile_scatter_body<R, TX, TY, TZ, NT>(s, id, L, G, offsets, cursors, entries, capacity, health, counts,
+                                       xcd_block(blockIdx.x, gridDim.x, 1), cur, lim);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1170,7 +1177,7 @@ __device__ __forceinline__ void gkd_tile(const GkdState<R>& ps, const R* __restr
 #pragma unroll 1
         for (int o = 0; o < 8; ++o) {
           const bool act = valid && target_active(up, o);
-          wave_add<false>(counts, act ? target_key(tn, o, G) : 0u, act);
+          wave_add(counts, act ? target_key(tn, o, G) : 0u, act);
         }
       }
     }
@@ -1299,13 +1306,14 @@ __global__ __launch_bounds__(kT) void k_batch_scatter(const BatchDesc* __restric
                                          gmem(m.health));
 }
 
-__global__ __launch_bounds__(kScatterT) void k_batch_tile_scatter(const BatchDesc* __restrict__ D) {
+template <int NT>
+__global__ __launch_bounds__(NT) void k_batch_tile_scatter(const BatchDesc* __restrict__ D) {
   __shared__ uint32_t cur_bins[kBins], lim_bins[kBins];
   const long b = xcd_block(blockIdx.x, gridDim.x, 1);
   const int k = batch_member(D, BS_TILE_SCATTER, b);
   const BatchMember& m = D->m[k];
   const int cur = batch_state(D, m);
-  tile_scatter_body<float, kBT, kBT, kBT>(gmem(m.s[cur]), gmem(m.id[cur]), m.L, m.G, gmem(m.offsets),
+  tile_scatter_body<float, kBT, kBT, kBT, NT>(gmem(m.s[cur]), gmem(m.id[cur]), m.L, m.G, gmem(m.offsets),
                                           gmem(m.cursors), gmem(m.entries), m.capacity, gmem(m.health),
                                           gmem(m.counts), (int)(b - D->off[BS_TILE_SCATTER][k]), cur_bins, lim_bins);
 }
@@ -1647,19 +1655,26 @@ bool tile_shape_supported(int tx, int ty, int tz) {
 
 TileGeom make_tiles(int n, int prec_bytes, int tx, int ty, int tz) {
   TileGeom g{};
-  if (tx == 0 && ty == 0 && tz == 0 && prec_bytes == 4 && (n == 256 || n == 384 || n == 512)) {
-    // FP32 default where the fused deposit + R2C kernel runs: 32 x 8 x 8
-    tx = 32;
-    ty = tz = 8;
-  } else if (tx == 0 && ty == 0 && tz == 0) {  // default: 16^3 (8^3 on the smallest grids)
-    auto pick = [n](int pref) {
-      int t = pref;
-      while (t > 1 && n % t) t /= 2;
-      return t;
-    };
-    tx = pick(16);
-    ty = pick(16);
-    tz = pick(16);
+  (void)prec_bytes;  // the same line in both precisions
+  if (tx == 0 && ty == 0 && tz == 0) {
+    // Default shape by grid size: small grids need many tiles to occupy the chip, large ones tiles
+    // whose potential box and accumulator leave the most blocks per CU and whose rows are whole cache
+    // lines.  Step of a resident run, evenly spread / clustered particles, us, in 16^3, 16x16x8,
+    // 32x8x8 and 8^3 tiles:
+    //    64^3  49 / 61    45 / 54    50 / 62    44 / 51
+    //    96^3  60 / 79    57 / 70    62 / 76    60 / 69
+    //   128^3  78 / 95    75 / 90    75 / 90    84 / 92
+    //   192^3  136 / 160  134 / 150  133 / 149  163 / 174
+    //   256^3  240 / 250  238 / 251  235 / 251  305 / 321
+    //   384^3  830 / 877  818 / 866  788 / 829
+    //   512^3  1822 / 1936  1818 / 1899  1729 / 1792  2394 / 2520
+    //  1024^3  16.07 ms              15.75 ms
+    // FP64: 64^3 58, 50, 52, 48; 192^3 204, 195, 195, 244; 256^3 429, 423, 421, 527;
+    // 512^3 3532, 3480, 3445, 4559.
+    const bool wide = n >= 256 && n % 32 == 0, flat = n >= 96 && n % 16 == 0;
+    tx = wide ? 32 : flat ? 16 : 8;
+    ty = !wide && flat ? 16 : 8;
+    tz = 8;
   }
   if (!tile_shape_supported(tx, ty, tz) || n % tx || n % ty || n % tz) return g;  // not usable
   g.tx = tx;
@@ -1742,9 +1757,14 @@ hipError_t bins_scatter(const PState<R>& p, const Lattice& L, const TileGeom& G,
   if (after_gather && tile_scatter_on(G, B)) {
 #define PM_L(X, Y, Z)                                                                                           \
   do {                                                                                                          \
-    if constexpr ((X) * (Y) * (Z) >= kTileScatterCells)                                                         \
-      k_tile_scatter<R, X, Y, Z><<<G.ntiles, kScatterT, 0, st>>>(p.s, p.id, L, G, B.offsets, B.cursors,         \
-                                                                 B.entries, B.capacity, B.health, B.counts);    \
+    if constexpr ((X) * (Y) * (Z) >= kTileScatterCells) {                                                       \
+      if (G.ntiles < kScatterTiles)                                                                             \
+        k_tile_scatter<R, X, Y, Z, kScatterWide><<<G.ntiles, kScatterWide, 0, st>>>(                            \
+            p.s, p.id, L, G, B.offsets, B.cursors, B.entries, B.capacity, B.health, B.counts);                  \
+      else                                                                                                      \
+        k_tile_scatter<R, X, Y, Z, kScatterT><<<G.ntiles, kScatterT, 0, st>>>(                                  \
+            p.s, p.id, L, G, B.offsets, B.cursors, B.entries, B.capacity, B.health, B.counts);                  \
+    }                                                                                                           \
   } while (0)
     PM_TILE_DISPATCH(G, PM_L);
 #undef PM_L
@@ -1935,7 +1955,8 @@ hipError_t batch_scatter(const BatchDesc* d, long total, long total_tiles, hipSt
   }
   if (total_tiles > 0) {
     if (hipError_t e = batch_grid(total_tiles, g)) return e;
-    k_batch_tile_scatter<<<g, kScatterT, 0, st>>>(d);
+    if (total_tiles < kScatterTiles) k_batch_tile_scatter<kScatterWide><<<g, kScatterWide, 0, st>>>(d);
+    else k_batch_tile_scatter<kScatterT><<<g, kScatterT, 0, st>>>(d);
   }
   return hipGetLastError();
 }

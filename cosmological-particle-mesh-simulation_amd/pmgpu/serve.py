@@ -125,6 +125,7 @@ def _start(req: SimRequest, prepared) -> PMSim:
     sim = PMSim(req.n_cells, req.n_parts, 32, omega_m0=req.om, omega_lambda0=req.ol,
                 omega_k0=req.ok, h0=req.h)
     try:
+        sim.set_tiles(16, 16, 16)   # the ensemble's shape: joining it keeps the bins and the density
         sim.zeldovich(amp, scale, vfac, seed=req.seed)
         sim.deposit()
     except Exception:
