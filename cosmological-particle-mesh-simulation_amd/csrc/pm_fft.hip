@@ -422,7 +422,9 @@ __device__ __forceinline__ void pencil_load(const PencilAddr<R>& p, cpx<R>* lds,
 // after one exchange through LDS it takes, for each of its J = A / TT values ka = t + j TT, the TT
 // values Y[t'][ka] and does the TT-point DFT, giving X[ka + A kb].  The inverse of the fused z pass
 // runs the same steps backwards from there.
-// Shape: W columns per block (whole 128-byte row segments), NT = W * TT threads.  FP64 takes 16
+// Shape: W columns per block (whole 128-byte row segments), NT = W * TT threads.  FP32 at N = 1024
+// takes 16 columns with 512 threads: with 8 (64-byte segments, half a cache line) the y passes ran
+// 2.35 and 2.32 ms in registers and 2.16 and 1.94 as LDS passes, with 16 they run 1.73 and 1.84.  FP64 takes 16
 // threads per column like FP32 but half the columns, so a block of 128 threads holds A = 32 complex
 // values per thread (N = 512) in 256 registers and its exchange slice is 37 KB: four blocks per CU.
 // FP64 runs only the z pass this way.  As an LDS pass its pencil, tables and twiddles left one block
@@ -430,8 +432,8 @@ __device__ __forceinline__ void pencil_load(const PencilAddr<R>& p, cpx<R>* lds,
 // 1580 us (caller's grid) at 512^3 against 666 / 701 / 848, 72 / 71 against 58 / 62 at 256^3.  The y
 // passes have LDS for two blocks and stay there: 373 and 364 us, 393 and 391 in registers.
 template <typename R, int N> struct RegShape {
-  static constexpr int W = pencil_w<R, N>();
-  static constexpr int TT = sizeof(R) == 4 ? kThreads / W : 16;
+  static constexpr int W = sizeof(R) == 4 && N == 1024 ? 16 : pencil_w<R, N>();
+  static constexpr int TT = sizeof(R) == 8 ? 16 : N == 1024 ? 32 : kThreads / W;
   static constexpr int NT = W * TT;
 };
 template <typename R, int N> constexpr bool reg_transform() {
@@ -442,11 +444,9 @@ template <typename R, int N> constexpr bool reg_transform() {
          N / S::TT <= 32 && (sizeof(R) == 4 ? N <= 1024 : S::W == 8 && N <= 512);
 }
 
-// Passes that run the register transform: every y and z pass up to N = 512; above that only
-// the fused z pass (its LDS slice takes 82-90 KB, one workgroup per CU: the y passes are faster
-// as LDS Stockham passes there, the z pass with its 4 MiB column stride is not)
+// Passes that run the register transform: in FP32 every y and z pass it exists for, in FP64 the z pass
 template <typename R, int N, int MODE> constexpr bool reg_pass() {
-  return reg_transform<R, N>() && ((sizeof(R) == 4 && N <= 512) || MODE == 0);
+  return reg_transform<R, N>() && (sizeof(R) == 4 || MODE == 0);
 }
 
 // the transform(s) of a staged pencil, in LDS (ends with the LDS holding the result)
@@ -509,15 +509,12 @@ __device__ __forceinline__ void pencil_tables(const cpx<R>* __restrict__ twg, co
 
 // One pencil: fetch, transform, store.  MODE: -1 forward only, +1 inverse only, 0 forward +
 // k-space operator + inverse.
-// Hout / s0out (optional): the first segment's pencils are written to Hout with the layout s0out
-// instead of back in place (the passes at N >= 1024 move the spectrum between layouts).
 // TAB_LDS: the tables are copied to LDS (tw, s2, wd) or are the global tables themselves.
 template <typename R, int N, int MODE, bool TAB_LDS = true, int W = pencil_w<R, N>()>
 __device__ __forceinline__ void pencil_body(cpx<R>* H, cpx<R>* Q, const PencilSeg& s0, const PencilSeg& s1,
                                             const GreenArgs& g, const cpx<R>* __restrict__ twg,
                                             const R* __restrict__ s2g, const R* __restrict__ wdg, long blk,
-                                            cpx<R>* lds, const cpx<R>* tw, const R* s2, const R* wd,
-                                            cpx<R>* Hout = nullptr, const PencilSeg* s0out = nullptr) {
+                                            cpx<R>* lds, const cpx<R>* tw, const R* s2, const R* wd) {
   const int tid = threadIdx.x;
   if constexpr (TAB_LDS)
     pencil_tables<R, N, MODE>(twg, s2g, wdg, const_cast<cpx<R>*>(tw), const_cast<R*>(s2), const_cast<R*>(wd), tid);
@@ -526,20 +523,18 @@ __device__ __forceinline__ void pencil_body(cpx<R>* H, cpx<R>* Q, const PencilSe
   __syncthreads();
   const R coef = MODE == 0 ? R(g.table ? g.table[3 * (*g.step)] : g.coef) : R(0);
   pencil_transform<R, N, MODE, W>(p, g, coef, lds, tw, s2, wd, tid);
-  if (Hout && blk < s0.nblk) pencil_store<R, N, W>(pencil_addr<R, N, W>(Hout, Q, *s0out, s1, blk), lds, tid);
-  else pencil_store<R, N, W>(p, lds, tid);
+  pencil_store<R, N, W>(p, lds, tid);
 }
 
 template <typename R, int N, int MODE, int W = pencil_w<R, N>()>
 __global__ __launch_bounds__(kThreads) void k_pencil(cpx<R>* H, cpx<R>* Q, PencilSeg s0, PencilSeg s1, GreenArgs g,
                                                      const cpx<R>* __restrict__ twg, const R* __restrict__ s2g,
-                                                     const R* __restrict__ wdg, cpx<R>* Hout, PencilSeg s0out) {
+                                                     const R* __restrict__ wdg) {
   __shared__ cpx<R> lds[N * (W + 1)];
   __shared__ cpx<R> tw[N];  // (the Stockham passes read the twiddles in every stage: kept in LDS)
   __shared__ R s2[MODE == 0 ? N : 1];
   __shared__ R wd[MODE == 0 ? N : 1];
-  pencil_body<R, N, MODE, true, W>(H, Q, s0, s1, g, twg, s2g, wdg, xcd_block(blockIdx.x, gridDim.x), lds, tw, s2, wd,
-                                   Hout, &s0out);
+  pencil_body<R, N, MODE, true, W>(H, Q, s0, s1, g, twg, s2g, wdg, xcd_block(blockIdx.x, gridDim.x), lds, tw, s2, wd);
 }
 
 // Register pass: the four-step transform with the columns read from and written to global
@@ -547,11 +542,20 @@ __global__ __launch_bounds__(kThreads) void k_pencil(cpx<R>* H, cpx<R>* Q, Penci
 // slice of TT ka values at a time (TT*TT rows of W columns), so a block holds a fraction of its
 // pencil in LDS and more blocks stay resident.  Row r of a slice sits at r*SN + r/TT + w: the
 // extra word per TT rows spreads both the writers' and the readers' lanes over the banks.
-template <typename R, int N> constexpr int xslice_elems() {
+// SPLIT (FP32 N = 1024, one slice of 32 x 32 rows): the real and the imaginary parts take turns in the
+// slice, which halves the block's LDS to 76 KB, two blocks of 512 threads per CU; its rows sit at
+// r*SN + 48 (r/TT) + w, which gives the 64 lanes of a wavefront 64 banks both ways.
+constexpr int kSplitPad = 48;
+template <typename R, int N> constexpr bool reg_split() {
+  return sizeof(R) == 4 && RegShape<R, N>::TT == 32 && N == 1024;
+}
+template <typename R, int N> constexpr int xslice_elems() {  // in complex values
   constexpr int W = RegShape<R, N>::W, TT = RegShape<R, N>::TT;
-  return TT * TT * (W + 1) + TT;
+  return reg_split<R, N>() ? (TT * TT * (W + 1) + kSplitPad * TT) / 2 : TT * TT * (W + 1) + TT;
 }
 
+// Hout / s0out (optional): the first segment's pencils are written to Hout with the layout s0out
+// instead of back in place (the passes at N = 1024 move the spectrum between layouts).
 // TAB_LDS: the twiddle and k-space tables are copied to LDS (tw, s2, wd); otherwise tw, s2, wd
 // are the global tables themselves (read through the caches), which keeps the block's LDS to the
 // exchange slice
@@ -559,7 +563,8 @@ template <typename R, int N, int MODE, bool TAB_LDS = true>
 __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const PencilSeg& s0, const PencilSeg& s1,
                                                 const GreenArgs& g, const cpx<R>* __restrict__ twg,
                                                 const R* __restrict__ s2g, const R* __restrict__ wdg, long blk,
-                                                cpx<R>* xb, const cpx<R>* tw, const R* s2, const R* wd) {
+                                                cpx<R>* xb, const cpx<R>* tw, const R* s2, const R* wd,
+                                                cpx<R>* Hout = nullptr, const PencilSeg* s0out = nullptr) {
   using T = cpx<R>;
   constexpr int W = RegShape<R, N>::W, TT = RegShape<R, N>::TT;
   constexpr int SN = W + 1;
@@ -586,28 +591,65 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
   reg_dft<S1, A>(v);
   twiddle_row<S1, N, A, 8>(v, tw, t);
   T u[J][TT];
+  constexpr bool SPLIT = reg_split<R, N>();
+  // SPLIT: row (from, q) of one value array to row (t, q) of the other through the slice
+  auto split_exchange = [&](const T (&from)[TT], T (&to)[TT], bool out_rows) {
+    R* xs = reinterpret_cast<R*>(xb);
+    auto srow = [&](int r) { return r * SN + kSplitPad * (r / TT) + w; };
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    if (j) __syncthreads();
+    for (int part = 0; part < 2; ++part) {
+      if (part || out_rows) __syncthreads();
 #pragma unroll
-    for (int q = 0; q < TT; ++q) xb[xrow(q * TT + t)] = v[j * TT + q];
-    __syncthreads();
+      for (int q = 0; q < TT; ++q)
+        xs[out_rows ? srow(t * TT + q) : srow(q * TT + t)] = part ? from[q].y : from[q].x;
+      __syncthreads();
 #pragma unroll
-    for (int q = 0; q < TT; ++q) u[j][q] = xb[xrow(t * TT + q)];
-    reg_dft<S1, TT>(u[j]);  // u[j][kb] = X[ka + A kb], ka = j TT + t
+      for (int q = 0; q < TT; ++q) {
+        const R x = xs[out_rows ? srow(q * TT + t) : srow(t * TT + q)];
+        if (part) to[q].y = x;
+        else to[q].x = x;
+      }
+    }
+  };
+  if constexpr (SPLIT) {
+    split_exchange(v, u[0], false);
+    reg_dft<S1, TT>(u[0]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      if (j) __syncthreads();
+#pragma unroll
+      for (int q = 0; q < TT; ++q) xb[xrow(q * TT + t)] = v[j * TT + q];
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < TT; ++q) u[j][q] = xb[xrow(t * TT + q)];
+      reg_dft<S1, TT>(u[j]);  // u[j][kb] = X[ka + A kb], ka = j TT + t
+    }
   }
   if constexpr (MODE != 0) {
+    if (Hout && blk < s0.nblk) {  // the first segment goes to another array and layout
+      const PencilAddr<R> o = pencil_addr<R, N, W, TT>(Hout, Q, *s0out, s1, blk);
+      const __amdgpu_buffer_rsrc_t obuf = buffer_of(o.base, o.tail * (long)sizeof(T));
+      const int ovoff = (int)((uint32_t)t * (uint32_t)(o.stride_n * (long)sizeof(T)) + (uint32_t)w * (uint32_t)sizeof(T));
+      const uint32_t oblk8 = (uint32_t)(o.stride_blk * (long)sizeof(T));
 #pragma unroll
-    for (int j = 0; j < J; ++j)
+      for (int j = 0; j < J; ++j)
 #pragma unroll
-      for (int kb = 0; kb < TT; ++kb) buffer_store(buf, voff, roff(j * TT + A * kb), u[j][kb]);
+        for (int kb = 0; kb < TT; ++kb)
+          buffer_store(obuf, ovoff, (int)((uint32_t)((j * TT + A * kb) / TT) * oblk8), u[j][kb]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int kb = 0; kb < TT; ++kb) buffer_store(buf, voff, roff(j * TT + A * kb), u[j][kb]);
+    }
   } else {
     // k-space operator on X[k], k = ka + A kb the z mode, then the same steps backwards
     const int kx = p.kx0 + w * p.dkx, ky = p.ky0 + w * p.dky;
     const R coef = R(coef_of(g));
     // green_factor(), each of its forms in a loop of its own (factors that live across a branch
     // would cost the plain form's registers) with the loads of GB factors issued together
-    constexpr int GB = sizeof(R) == 8 ? 8 : TT;
+    constexpr int GB = 8;
     if (g.from_grid) {
       const uint32_t row = (uint32_t)N * N, g1 = (uint32_t)ky * N + kx;
       const uint32_t g2 = (uint32_t)((N - ky) % N) * N + (N - kx) % N;  // the mode's conjugate
@@ -656,16 +698,22 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
       const int ka = j * TT + t;
       reg_dft<+1, TT>(u[j]);
 #pragma unroll
-      for (int q = 1; q < TT; ++q) u[j][q] = cmulc(u[j][q], tw[(q * ka) % N]);
+      for (int q = 1; q < TT; ++q) {
+        u[j][q] = cmulc(u[j][q], tw[(q * ka) % N]);
+      }
     }
+    if constexpr (SPLIT) {
+      split_exchange(u[0], v, true);
+    } else {
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      __syncthreads();
+      for (int j = 0; j < J; ++j) {
+        __syncthreads();
 #pragma unroll
-      for (int q = 0; q < TT; ++q) xb[xrow(t * TT + q)] = u[j][q];
-      __syncthreads();
+        for (int q = 0; q < TT; ++q) xb[xrow(t * TT + q)] = u[j][q];
+        __syncthreads();
 #pragma unroll
-      for (int r = 0; r < TT; ++r) v[j * TT + r] = xb[xrow(r * TT + t)];
+        for (int r = 0; r < TT; ++r) v[j * TT + r] = xb[xrow(r * TT + t)];
+      }
     }
     reg_dft<+1, A>(v);
 #pragma unroll
@@ -674,9 +722,9 @@ __device__ __forceinline__ void pencil_reg_body(cpx<R>* H, cpx<R>* Q, const Penc
 }
 
 template <typename R, int N, int MODE>
-__global__ __launch_bounds__((RegShape<R, N>::NT), sizeof(R) == 8 ? 2 : 1) void k_pencil_reg(
+__global__ __launch_bounds__((RegShape<R, N>::NT), sizeof(R) == 8 || N == 1024 ? 2 : 1) void k_pencil_reg(
     cpx<R>* H, cpx<R>* Q, PencilSeg s0, PencilSeg s1, GreenArgs g, const cpx<R>* __restrict__ twg,
-    const R* __restrict__ s2g, const R* __restrict__ wdg) {
+    const R* __restrict__ s2g, const R* __restrict__ wdg, cpx<R>* Hout, PencilSeg s0out) {
   __shared__ cpx<R> xb[xslice_elems<R, N>()];
   // above N = 512, and in FP64, the tables stay in global memory: with them the block's LDS (90 KB
   // at N = 1024) allows one block per CU, without them two
@@ -689,7 +737,7 @@ __global__ __launch_bounds__((RegShape<R, N>::NT), sizeof(R) == 8 ? 2 : 1) void 
                                       wd);
   else
     pencil_reg_body<R, N, MODE, false>(H, Q, s0, s1, g, twg, s2g, wdg, xcd_block(blockIdx.x, gridDim.x), xb, twg,
-                                       s2g, wdg);
+                                       s2g, wdg, reg_split<R, N>() ? Hout : nullptr, &s0out);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -792,37 +840,33 @@ hipError_t launch_pencil(cpx<R>* H, cpx<R>* Q, bool zaxis, const GreenArgs& g, c
       PencilSeg a2, b2;
       if (zaxis) z_segments<R, N, W2>(a2, b2);
       else y_segments<R, N, W2>(a2, b2);
-      k_pencil<R, N, MODE, W2><<<(unsigned)(a2.nblk + b2.nblk), kThreads, 0, st>>>(H, Q, a2, b2, g, tw, s2, wd,
-                                                                                   nullptr, a2);
+      k_pencil<R, N, MODE, W2><<<(unsigned)(a2.nblk + b2.nblk), kThreads, 0, st>>>(H, Q, a2, b2, g, tw, s2, wd);
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;
     }
   }
   PencilSeg a, b;
-  if (zaxis) z_segments<R, N>(a, b);
-  else y_segments<R, N>(a, b);
+  constexpr int W = reg_pass<R, N, MODE>() ? RegShape<R, N>::W : pencil_w<R, N>();
+  if (zaxis) z_segments<R, N, W>(a, b);
+  else y_segments<R, N, W>(a, b);
   const unsigned nb = (unsigned)(a.nblk + b.nblk);
   if constexpr (tiled_spectrum<R, N>()) {
     if (work) {
-      if (zaxis) {  // in place on the tiled array
-        const PencilSeg at = z_tiled<R, N>(a);
-        if constexpr (reg_pass<R, N, MODE>())
-          k_pencil_reg<R, N, MODE><<<nb, RegShape<R, N>::NT, 0, st>>>(work, Q, at, b, g, tw, s2, wd);
-        else
-          k_pencil<R, N, MODE><<<nb, kThreads, 0, st>>>(work, Q, at, b, g, tw, s2, wd, nullptr, at);
-      } else if (MODE < 0) {  // plain H -> tiled work
-        k_pencil<R, N, MODE><<<nb, kThreads, 0, st>>>(H, Q, a, b, g, tw, s2, wd, work, y_tiled<R, N>(a));
-      } else {  // tiled work -> plain H
-        k_pencil<R, N, MODE><<<nb, kThreads, 0, st>>>(work, Q, y_tiled<R, N>(a), b, g, tw, s2, wd, H, a);
-      }
+      // z in place on the tiled array; forward y from plain H to it, inverse y back
+      const PencilSeg in = zaxis ? z_tiled<R, N>(a) : MODE < 0 ? a : y_tiled<R, N>(a);
+      const PencilSeg out = MODE < 0 ? y_tiled<R, N>(a) : a;
+      cpx<R>* src = !zaxis && MODE < 0 ? H : work;
+      cpx<R>* dst = zaxis ? nullptr : MODE < 0 ? work : H;
+      static_assert(reg_pass<R, N, MODE>() || sizeof(R) == 8, "the tiled spectrum is transformed in registers");
+      k_pencil_reg<R, N, MODE><<<nb, RegShape<R, N>::NT, 0, st>>>(src, Q, in, b, g, tw, s2, wd, dst, out);
       return hipGetLastError();
     }
   }
   if constexpr (reg_pass<R, N, MODE>()) {
-    k_pencil_reg<R, N, MODE><<<nb, RegShape<R, N>::NT, 0, st>>>(H, Q, a, b, g, tw, s2, wd);
+    k_pencil_reg<R, N, MODE><<<nb, RegShape<R, N>::NT, 0, st>>>(H, Q, a, b, g, tw, s2, wd, nullptr, a);
   } else {
-    k_pencil<R, N, MODE><<<nb, kThreads, 0, st>>>(H, Q, a, b, g, tw, s2, wd, nullptr, a);
+    k_pencil<R, N, MODE><<<nb, kThreads, 0, st>>>(H, Q, a, b, g, tw, s2, wd);
   }
   return hipGetLastError();
 }
