@@ -906,7 +906,10 @@ __global__ __launch_bounds__(kDrT) void k_deposit_r2c(const float* __restrict__ 
 // ------------------------------------------------------------------------------------------
 template <int TX, int TY, int TZ> constexpr int gkd_box_cells() { return (TX + 3) * (TY + 3) * (TZ + 3); }
 
-constexpr int kGkdE = 2;  // particles per thread and batch in the gather
+// particles per thread and batch in the gather (FP64: one, which leaves the registers for a fourth
+// wavefront per SIMD: 138 -> 124, gather 896 -> 788 us at 512^3, 116 -> 105 at 256^3; FP32 measures
+// the same with either)
+template <typename R> constexpr int gkd_e() { return sizeof(R) == 4 ? 2 : 1; }
 
 // own-entry range [beg, end) of a tile, and a thread's first batch of its slot entries
 __device__ __forceinline__ void tile_range(const uint32_t* __restrict__ offsets, uint32_t capacity, int tile,
@@ -914,10 +917,11 @@ __device__ __forceinline__ void tile_range(const uint32_t* __restrict__ offsets,
   end = min(offsets[tile + 1], capacity);
   beg = min(offsets[tile], end);
 }
+template <int E>
 __device__ __forceinline__ void first_entries(const uint32_t* __restrict__ entries, uint32_t beg, uint32_t end,
-                                              long np, uint32_t (&sl)[kGkdE]) {
+                                              long np, uint32_t (&sl)[E]) {
 #pragma unroll
-  for (int u = 0; u < kGkdE; ++u) {
+  for (int u = 0; u < E; ++u) {
     const uint32_t e = beg + u * kT + threadIdx.x;
     sl[u] = e < end ? min(entries[e], (uint32_t)(np - 1)) : kNone;
   }
@@ -941,14 +945,14 @@ template <typename R, int TX, int TY, int TZ, bool LOCAL_HIST, bool TS>
 __device__ __forceinline__ void gkd_tile(const GkdState<R>& ps, const R* __restrict__ phi, R kick, R drift,
                                          const Lattice& L, const TileGeom& G,
                                          const uint32_t* __restrict__ entries, uint32_t* __restrict__ counts,
-                                         int tile, uint32_t beg, uint32_t end, const uint32_t (&sl0)[kGkdE], R* box,
+                                         int tile, uint32_t beg, uint32_t end, const uint32_t (&sl0)[gkd_e<R>()], R* box,
                                          uint32_t* hist, const float4* __restrict__ edge) {
   constexpr int BX = TX + 3, BY = TY + 3, BZ = TZ + 3;
   constexpr int NW = kT / 64;                       // wavefronts per block
   constexpr int PLANE = BX * BY;                    // values per box plane
   constexpr int PL = (PLANE + 63) / 64;             // wavefront loads per plane
   constexpr int ZIT = (BZ + NW - 1) / NW;           // planes per wavefront
-  constexpr int E = kGkdE;
+  constexpr int E = gkd_e<R>();
   // hist: new-tile counts, offset (-1..2)^3 from this tile x {own, halo}
   static_assert(!TS || LOCAL_HIST, "the tile scatter needs the neighbourhood histogram");
   if (beg == end) return;  // empty tile: the whole block leaves together
@@ -1208,7 +1212,7 @@ __device__ __forceinline__ void gkd_body(const GkdState<R>& P, const R* __restri
                                          const uint32_t* __restrict__ entries, uint32_t* __restrict__ counts,
                                          uint32_t capacity, int tile, R* box, uint32_t* hist,
                                          const float4* __restrict__ edge = nullptr) {
-  uint32_t beg, end, sl[kGkdE];
+  uint32_t beg, end, sl[gkd_e<R>()];
   tile_range(offsets, capacity, tile, beg, end);
   first_entries(entries, beg, end, L.np, sl);
   gkd_tile<R, TX, TY, TZ, LOCAL_HIST, TS>(P, phi, kick, drift, L, G, entries, counts, tile, beg, end, sl, box,
