@@ -468,8 +468,7 @@ PM_API int pm_density_k(const float* rho, int n, void* rho_k) {
   Workspace* w;
   if (int rc = get_tables(n, 8, &t)) return rc;
   if (int rc = get_workspace(n, false, &w)) return rc;
-  PM_HIP((fft_r2c_x<double, float>(rho, w->H, w->Q, n, *t, g_stream)));
-  PM_HIP(fft_c2c_y<double>(w->H, w->Q, n, -1, *t, g_stream));
+  PM_HIP((fft_forward_xy<double, float>(rho, w->H, w->Q, n, *t, g_stream)));
   PM_HIP(fft_c2c_z<double>(w->H, w->Q, n, -1, *t, g_stream));
   PM_HIP(spec_expand_full(w->H, w->Q, (double2*)rho_k, n, g_stream));
   PM_HIP(hipStreamSynchronize(g_stream));
@@ -497,8 +496,7 @@ PM_API int pm_potential_real(const void* phi_k, int n, float* phi) {
   const double scale = 1.0 / ((double)n * n * n);  // pyFFTW normalise_idft=True
   PM_HIP(spec_hermitian_half((const double2*)phi_k, w->H, w->Q, n, scale, g_stream));
   PM_HIP(fft_c2c_z<double>(w->H, w->Q, n, +1, *t, g_stream));
-  PM_HIP(fft_c2c_y<double>(w->H, w->Q, n, +1, *t, g_stream));
-  PM_HIP((fft_c2r_x<double, float>(w->H, w->Q, phi, n, *t, g_stream)));
+  PM_HIP((fft_inverse_yx<double, float>(w->H, w->Q, phi, n, *t, g_stream)));
   PM_HIP(hipStreamSynchronize(g_stream));
   return PM_OK;
 }
@@ -512,11 +510,9 @@ static int potential_into(const float* rho, const float* fgrid, int n, double a,
   g.coef = (-3 * omega_m0 / 8 / a) / ((double)n * n * n);
   g.from_grid = 1;
   g.fgrid = fgrid;
-  PM_HIP((fft_r2c_x<double, float>(rho, w->H, w->Q, n, *t, g_stream)));
-  PM_HIP(fft_c2c_y<double>(w->H, w->Q, n, -1, *t, g_stream));
+  PM_HIP((fft_forward_xy<double, float>(rho, w->H, w->Q, n, *t, g_stream)));
   PM_HIP(fft_z_green<double>(w->H, w->Q, n, g, *t, g_stream));
-  PM_HIP(fft_c2c_y<double>(w->H, w->Q, n, +1, *t, g_stream));
-  PM_HIP((fft_c2r_x<double, float>(w->H, w->Q, phi, n, *t, g_stream)));
+  PM_HIP((fft_inverse_yx<double, float>(w->H, w->Q, phi, n, *t, g_stream)));
   return PM_OK;
 }
 
@@ -558,11 +554,9 @@ PM_API int pm_potential_static(const float* rho, const float* fgrid, int n, doub
   g.coef = (-3 * omega_m0 / 8 / a) / ((double)n * n * n);
   g.from_grid = 1;
   g.fgrid = fgrid;
-  PM_HIP((fft_r2c_x<double, float>(rho, H, Q, n, t, g_stream)));
-  PM_HIP(fft_c2c_y<double>(H, Q, n, -1, t, g_stream));
+  PM_HIP((fft_forward_xy<double, float>(rho, H, Q, n, t, g_stream)));
   PM_HIP(fft_z_green<double>(H, Q, n, g, t, g_stream));
-  PM_HIP(fft_c2c_y<double>(H, Q, n, +1, t, g_stream));
-  PM_HIP((fft_c2r_x<double, float>(H, Q, phi, n, t, g_stream)));
+  PM_HIP((fft_inverse_yx<double, float>(H, Q, phi, n, t, g_stream)));
   PM_HIP(hipStreamSynchronize(g_stream));
   return PM_OK;
 }
@@ -880,13 +874,17 @@ template <typename R> int sim_step_impl(pm_sim* s, double a, double da, bool tab
   // the spectrum: left in the density slot by the fused deposit, or the R2C pass of the density
   const bool in_rho_slot = s->spec_valid;
   cpx<R>* H = (cpx<R>*)(in_rho_slot ? rho_slot(s) : spec_slot(s));
+  // small grids: x and y in one plane pass (timed as the x pass), unless the caller chose a y pencil shape
+  const bool plane = fft_plane_supported(n, (int)sizeof(R));
+  const bool plane_fwd = plane && !in_rho_slot && !s->pencil_alt[0], plane_inv = plane && !s->pencil_alt[2];
   if (!in_rho_slot) {
     StageTimer t(s, ST_R2C);
-    PM_HIP((fft_r2c_x<R, R>((const R*)rho_slot(s), H, Q, n, *s->tab, s->stream, rev)));
+    if (plane_fwd) PM_HIP((fft_r2c_xy<R, R>((const R*)rho_slot(s), H, Q, n, *s->tab, s->stream)));
+    else PM_HIP((fft_r2c_x<R, R>((const R*)rho_slot(s), H, Q, n, *s->tab, s->stream, rev)));
   }
   // the other slot is the y / z passes' work array (the density it may hold has been consumed)
   cpx<R>* work = reinterpret_cast<cpx<R>*>(in_rho_slot ? spec_slot(s) : rho_slot(s));
-  {
+  if (!plane_fwd) {
     StageTimer t(s, ST_Y_FWD);
     PM_HIP(fft_c2c_y<R>(H, Q, n, -1, *s->tab, s->stream, work, s->pencil_alt[0]));
   }
@@ -894,7 +892,7 @@ template <typename R> int sim_step_impl(pm_sim* s, double a, double da, bool tab
     StageTimer t(s, ST_Z_GREEN);
     PM_HIP(fft_z_green<R>(H, Q, n, g, *s->tab, s->stream, work, s->pencil_alt[1]));
   }
-  {
+  if (!plane_inv) {
     StageTimer t(s, ST_Y_INV);
     PM_HIP(fft_c2c_y<R>(H, Q, n, +1, *s->tab, s->stream, work, s->pencil_alt[2]));
   }
@@ -902,7 +900,8 @@ template <typename R> int sim_step_impl(pm_sim* s, double a, double da, bool tab
   float4* edge = (s->edge && s->G.tx == 32) ? s->edge : nullptr;
   {
     StageTimer t(s, ST_C2R);
-    PM_HIP((fft_c2r_x<R, R>(H, Q, (R*)H, n, *s->tab, s->stream, edge, rev)));
+    if (plane_inv) PM_HIP((fft_c2r_yx<R, R>(H, Q, (R*)H, n, *s->tab, s->stream, edge)));
+    else PM_HIP((fft_c2r_x<R, R>(H, Q, (R*)H, n, *s->tab, s->stream, edge, rev)));
   }
   if (in_rho_slot) s->gb ^= 1;  // the potential now sits in the spectrum slot
   s->phi_valid = true;
@@ -1090,7 +1089,8 @@ template <typename R> int sim_autotune_impl(pm_sim* s, int reps, double* best_ms
   // by more than 2 %
   for (int p = 0; p < 3 && rc == PM_OK; ++p) {
     const int mode = p == 0 ? -1 : (p == 1 ? 0 : 1);
-    if (!fft_pencil_cols(n, s->prec, mode, true)) {
+    // (y passes that run within plane passes have no shape to tune)
+    if (!fft_pencil_cols(n, s->prec, mode, true) || (mode != 0 && fft_plane_supported(n, s->prec))) {
       s->pencil_alt[p] = false;
       continue;
     }
@@ -1615,16 +1615,14 @@ PM_API int pm_sim_power_spectrum(pm_sim* s, double box, int n_bins, double* k, d
       cpx<float>* H = (cpx<float>*)spec_slot(s);
       cpx<float>* Q = (cpx<float>*)s->Q;
       e = grid_sum<float>((const float*)rho_slot(s), cells, d, s->stream);
-      if (!e) e = fft_r2c_x<float, float>((const float*)rho_slot(s), H, Q, n, *s->tab, s->stream);
-      if (!e) e = fft_c2c_y<float>(H, Q, n, -1, *s->tab, s->stream);
+      if (!e) e = fft_forward_xy<float, float>((const float*)rho_slot(s), H, Q, n, *s->tab, s->stream);
       if (!e) e = fft_c2c_z<float>(H, Q, n, -1, *s->tab, s->stream);
       if (!e) e = shell_sums<float>(H, Q, n, n_bins, d + 1, s->stream);
     } else {
       cpx<double>* H = (cpx<double>*)spec_slot(s);
       cpx<double>* Q = (cpx<double>*)s->Q;
       e = grid_sum<double>((const double*)rho_slot(s), cells, d, s->stream);
-      if (!e) e = fft_r2c_x<double, double>((const double*)rho_slot(s), H, Q, n, *s->tab, s->stream);
-      if (!e) e = fft_c2c_y<double>(H, Q, n, -1, *s->tab, s->stream);
+      if (!e) e = fft_forward_xy<double, double>((const double*)rho_slot(s), H, Q, n, *s->tab, s->stream);
       if (!e) e = fft_c2c_z<double>(H, Q, n, -1, *s->tab, s->stream);
       if (!e) e = shell_sums<double>(H, Q, n, n_bins, d + 1, s->stream);
     }

@@ -19,12 +19,17 @@ template <typename T> __host__ __device__ __forceinline__ T cmake(decltype(T::x)
 }
 template <typename T> __host__ __device__ __forceinline__ T cadd(T a, T b) { return cmake<T>(a.x + b.x, a.y + b.y); }
 template <typename T> __host__ __device__ __forceinline__ T csub(T a, T b) { return cmake<T>(a.x - b.x, a.y - b.y); }
+// fused multiply-add a * b + c in the operands' precision
+__host__ __device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__host__ __device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// (written as fused multiply-adds: left to the compiler, which product is the fused one differs from
+// kernel to kernel, and passes that should give the same bits would not)
 template <typename T> __host__ __device__ __forceinline__ T cmul(T a, T b) {
-  return cmake<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return cmake<T>(fmadd(a.x, b.x, -(a.y * b.y)), fmadd(a.x, b.y, a.y * b.x));
 }
 // a * conj(b)
 template <typename T> __host__ __device__ __forceinline__ T cmulc(T a, T b) {
-  return cmake<T>(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
+  return cmake<T>(fmadd(a.x, b.x, a.y * b.y), fmadd(a.y, b.x, -(a.x * b.y)));
 }
 template <typename T> __host__ __device__ __forceinline__ T cconj(T a) { return cmake<T>(a.x, -a.y); }
 template <typename T, typename S> __host__ __device__ __forceinline__ T cscale(T a, S s) {

@@ -26,12 +26,12 @@ template <int S, typename T> __device__ __forceinline__ void dft3(T* v) {
   T t = cadd(v[1], v[2]);
   T d = csub(v[1], v[2]);
   T y0 = cadd(v[0], t);
-  T m = cmake<T>(v[0].x - R(0.5) * t.x, v[0].y - R(0.5) * t.y);
-  // S*i*h*d = (-S*h*d.y, S*h*d.x)
-  T r = cmake<T>(-R(S) * h * d.y, R(S) * h * d.x);
+  // (fused multiply-adds are written out, as in cmul, for the same bits in every kernel)
+  const R x = fmadd(R(-0.5), t.x, v[0].x), y = fmadd(R(-0.5), t.y, v[0].y);
   v[0] = y0;
-  v[1] = cadd(m, r);
-  v[2] = csub(m, r);
+  // S*i*h*d = (-S*h*d.y, S*h*d.x)
+  v[1] = cmake<T>(fmadd(-R(S) * h, d.y, x), fmadd(R(S) * h, d.x, y));
+  v[2] = cmake<T>(fmadd(R(S) * h, d.y, x), fmadd(-R(S) * h, d.x, y));
 }
 
 template <int S, typename T> __device__ __forceinline__ void dft4(T* v) {
@@ -52,18 +52,18 @@ template <int S, typename T> __device__ __forceinline__ void dft8(T* v) {
   T o[4] = {v[1], v[3], v[5], v[7]};
   dft4<S>(e);
   dft4<S>(o);
-  // o1 *= w8 = (1 + S i)/sqrt2 ; o2 *= S i ; o3 *= (-1 + S i)/sqrt2
-  T o1 = cmake<T>(c * (o[1].x - R(S) * o[1].y), c * (o[1].y + R(S) * o[1].x));
+  // o1 *= w8 = (1 + S i)/sqrt2 ; o2 *= S i ; o3 *= (-1 + S i)/sqrt2, the factors 1/sqrt2 in the sums
+  T o1 = cmake<T>(o[1].x - R(S) * o[1].y, o[1].y + R(S) * o[1].x);
   T o2 = cmul_si<S>(o[2]);
-  T o3 = cmake<T>(c * (-o[3].x - R(S) * o[3].y), c * (-o[3].y + R(S) * o[3].x));
+  T o3 = cmake<T>(-o[3].x - R(S) * o[3].y, -o[3].y + R(S) * o[3].x);
   v[0] = cadd(e[0], o[0]);
   v[4] = csub(e[0], o[0]);
-  v[1] = cadd(e[1], o1);
-  v[5] = csub(e[1], o1);
+  v[1] = cmake<T>(fmadd(c, o1.x, e[1].x), fmadd(c, o1.y, e[1].y));
+  v[5] = cmake<T>(fmadd(-c, o1.x, e[1].x), fmadd(-c, o1.y, e[1].y));
   v[2] = cadd(e[2], o2);
   v[6] = csub(e[2], o2);
-  v[3] = cadd(e[3], o3);
-  v[7] = csub(e[3], o3);
+  v[3] = cmake<T>(fmadd(c, o3.x, e[3].x), fmadd(c, o3.y, e[3].y));
+  v[7] = cmake<T>(fmadd(-c, o3.x, e[3].x), fmadd(-c, o3.y, e[3].y));
 }
 
 template <int RAD, int S, typename T> __device__ __forceinline__ void dftR(T* v) {
@@ -165,11 +165,11 @@ template <int L> struct fft_len_ok {
 
 // ------------------------------------------------------------------------------------------
 // One Stockham radix-RAD pass over W independent length-L sequences held in LDS.
-// Element (n, w) lives at lds[n*SN + w].  Butterfly b -> (w = b % W, j = b / W), so the
-// lanes of a wavefront walk along w (contiguous LDS addresses).
+// Element (n, w) lives at lds[n*SN + w*SW].  Butterfly b -> (w = b % W, j = b / W), so the
+// lanes of a wavefront walk along w (contiguous LDS addresses, or an odd stride SW).
 // tw[m*TS] = exp(-2 pi i m / L) for m in [0, L).
 // ------------------------------------------------------------------------------------------
-template <typename T, int L, int RAD, int NS, int S, int W, int SN, int NT, int TS>
+template <typename T, int L, int RAD, int NS, int S, int W, int SN, int NT, int TS, int SW>
 __device__ __forceinline__ void stockham_pass(T* lds, const T* tw, int tid) {
   constexpr int NB = L / RAD;
   constexpr int TOT = NB * W;
@@ -181,7 +181,7 @@ __device__ __forceinline__ void stockham_pass(T* lds, const T* tw, int tid) {
     if (TOT % NT == 0 || b < TOT) {
       const int w = b % W, j = b / W;
 #pragma unroll
-      for (int r = 0; r < RAD; ++r) v[i][r] = lds[(j + r * NB) * SN + w];
+      for (int r = 0; r < RAD; ++r) v[i][r] = lds[(j + r * NB) * SN + w * SW];
     }
   }
   __syncthreads();
@@ -202,19 +202,19 @@ __device__ __forceinline__ void stockham_pass(T* lds, const T* tw, int tid) {
       dftR<RAD, S>(v[i]);
       const int base = (j / NS) * NS * RAD + k;
 #pragma unroll
-      for (int r = 0; r < RAD; ++r) lds[(base + r * NS) * SN + w] = v[i][r];
+      for (int r = 0; r < RAD; ++r) lds[(base + r * NS) * SN + w * SW] = v[i][r];
     }
   }
   __syncthreads();
 }
 
-template <typename T, int L, int NS, int S, int W, int SN, int NT, int TS>
+template <typename T, int L, int NS, int S, int W, int SN, int NT, int TS, int SW = 1>
 __device__ __forceinline__ void fft_passes(T* lds, const T* tw, int tid) {
   if constexpr (NS < L) {
     constexpr int RAD = first_radix<L / NS>::value;
     static_assert(RAD != 0, "FFT length must be 2^a 3^b");
-    stockham_pass<T, L, RAD, NS, S, W, SN, NT, TS>(lds, tw, tid);
-    fft_passes<T, L, NS * RAD, S, W, SN, NT, TS>(lds, tw, tid);
+    stockham_pass<T, L, RAD, NS, S, W, SN, NT, TS, SW>(lds, tw, tid);
+    fft_passes<T, L, NS * RAD, S, W, SN, NT, TS, SW>(lds, tw, tid);
   }
 }
 
@@ -282,6 +282,14 @@ hipError_t fft_r2c_x(const Tin* rho, cpx<R>* H, cpx<R>* Q, int n, const FftTable
 template <typename R>
 hipError_t fft_c2c_y(cpx<R>* H, cpx<R>* Q, int n, int sign, const FftTables& t, hipStream_t st,
                      cpx<R>* work = nullptr, bool alt = false);
+// The x and y passes of one direction as one pass per z plane, held in LDS: the bits of the two passes.
+// For grids whose plane fits (fft_plane_supported); rho / out as in fft_r2c_x / fft_c2r_x.
+bool fft_plane_supported(int n, int prec);
+template <typename R, typename Tin>
+hipError_t fft_r2c_xy(const Tin* rho, cpx<R>* H, cpx<R>* Q, int n, const FftTables& t, hipStream_t st);
+template <typename R, typename Tout>
+hipError_t fft_c2r_yx(const cpx<R>* H, const cpx<R>* Q, Tout* out, int n, const FftTables& t, hipStream_t st,
+                      float4* edge = nullptr);
 template <typename R>
 hipError_t fft_c2c_z(cpx<R>* H, cpx<R>* Q, int n, int sign, const FftTables& t, hipStream_t st);
 template <typename R>
@@ -295,5 +303,19 @@ template <typename R, typename Tout>
 // edge (FP32 only, N % 32 == 0; may be null): also write the x margins of 32-wide tiles, see c2r_body
 hipError_t fft_c2r_x(cpx<R>* H, const cpx<R>* Q, Tout* out, int n, const FftTables& t, hipStream_t st,
                      float4* edge = nullptr, bool rev = false);
+
+// forward x and y / inverse y and x of a grid, as plane passes where they exist
+template <typename R, typename Tin>
+hipError_t fft_forward_xy(const Tin* rho, cpx<R>* H, cpx<R>* Q, int n, const FftTables& t, hipStream_t st) {
+  if (fft_plane_supported(n, (int)sizeof(R))) return fft_r2c_xy<R, Tin>(rho, H, Q, n, t, st);
+  if (hipError_t e = fft_r2c_x<R, Tin>(rho, H, Q, n, t, st)) return e;
+  return fft_c2c_y<R>(H, Q, n, -1, t, st);
+}
+template <typename R, typename Tout>
+hipError_t fft_inverse_yx(cpx<R>* H, cpx<R>* Q, Tout* out, int n, const FftTables& t, hipStream_t st) {
+  if (fft_plane_supported(n, (int)sizeof(R))) return fft_c2r_yx<R, Tout>(H, Q, out, n, t, st);
+  if (hipError_t e = fft_c2c_y<R>(H, Q, n, +1, t, st)) return e;
+  return fft_c2r_x<R, Tout>(H, Q, out, n, t, st);
+}
 
 }  // namespace pm

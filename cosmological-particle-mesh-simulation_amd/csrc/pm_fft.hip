@@ -43,6 +43,106 @@ template <typename R, int N> constexpr int rows_per_block() {
 // LDS of the x passes: M*(RB+1) complex for the rows plus N twiddles
 template <typename R, int N, int RB> constexpr int xpass_lds() { return ((N / 2) * (RB + 1) + N) * (int)sizeof(cpx<R>); }
 
+// R2C untangling of RB rows in LDS (element k of row w at lds[k*SN + w]): the M-point spectra Z of
+// x[2n] + i x[2n+1] become X[0 .. M) of the N reals; nyquist(w, X[M]) takes the real Nyquist value.
+// Ends with a barrier.
+template <typename R, int N, int RB, int SN, int NT, class F>
+__device__ __forceinline__ void untangle_rows(cpx<R>* lds, const cpx<R>* tw, int tid, F&& nyquist) {
+  using T = cpx<R>;
+  constexpr int M = N / 2;
+  constexpr int NPAIR = M / 2 + 1;
+  constexpr int TOTP = NPAIR * RB;
+  constexpr int PERP = (TOTP + NT - 1) / NT;
+  T zk[PERP], zm[PERP];
+#pragma unroll
+  for (int i = 0; i < PERP; ++i) {
+    const int b = tid + i * NT;
+    if (b < TOTP) {
+      const int w = b % RB, k = b / RB;
+      zk[i] = lds[k * SN + w];
+      zm[i] = lds[((M - k) % M) * SN + w];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PERP; ++i) {
+    const int b = tid + i * NT;
+    if (b < TOTP) {
+      const int w = b % RB, k = b / RB;
+      // E = (Z[k] + conj Z[M-k]) / 2 ; O = (Z[k] - conj Z[M-k]) / (2i)
+      const T a = zk[i], c = zm[i];
+      const T E = cmake<T>(R(0.5) * (a.x + c.x), R(0.5) * (a.y - c.y));
+      const T O = cmake<T>(R(0.5) * (a.y + c.y), R(-0.5) * (a.x - c.x));
+      const T wO = cmul(O, tw[k]);
+      if (k == 0) {
+        lds[w] = cmake<T>(E.x + wO.x, R(0));
+        nyquist(w, E.x - wO.x);
+      } else {
+        lds[k * SN + w] = cadd(E, wO);                       // X[k]
+        if (2 * k != M) lds[(M - k) * SN + w] = cconj(csub(E, wO));  // X[M-k]
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// The reverse for C2R: X[0 .. M) and nyquist(w) = X[M] become the spectra of the packed rows.
+template <typename R, int N, int RB, int SN, int NT, class F>
+__device__ __forceinline__ void tangle_rows(cpx<R>* lds, const cpx<R>* tw, int tid, F&& nyquist) {
+  using T = cpx<R>;
+  constexpr int M = N / 2;
+  constexpr int NPAIR = M / 2 + 1;
+  constexpr int TOTP = NPAIR * RB;
+  constexpr int PERP = (TOTP + NT - 1) / NT;
+  T xk[PERP], xm[PERP];
+#pragma unroll
+  for (int i = 0; i < PERP; ++i) {
+    const int b = tid + i * NT;
+    if (b < TOTP) {
+      const int w = b % RB, k = b / RB;
+      xk[i] = lds[k * SN + w];
+      xm[i] = (k == 0) ? nyquist(w) : lds[(M - k) * SN + w];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PERP; ++i) {
+    const int b = tid + i * NT;
+    if (b < TOTP) {
+      const int w = b % RB, k = b / RB;
+      const T A = cadd(xk[i], cconj(xm[i]));
+      const T B = csub(xk[i], cconj(xm[i]));
+      const T wk = tw[k];
+      // Z[k] = A + i conj(w^k) B
+      const T cb = cmulc(B, wk);
+      lds[k * SN + w] = cmake<T>(A.x - cb.y, A.y + cb.x);
+      if (k != 0 && 2 * k != M) {
+        // Z[M-k] = conj(A) + i w^k conj(B)
+        const T wb = cmul(cconj(B), wk);
+        lds[(M - k) * SN + w] = cmake<T>(A.x - wb.y, -A.y + wb.x);
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// x margins of the rows row0 .. row0 + RB in LDS (see c2r_body)
+template <int N, int RB, int SN, int NT>
+__device__ __forceinline__ void write_edge(const float2* lds, float4* __restrict__ edge, size_t row0, int tid) {
+  constexpr int NB = N / 32;
+  auto phi_at = [&](int x, int w) {
+    const float2 v = lds[(x >> 1) * SN + w];
+    return (x & 1) ? v.y : v.x;
+  };
+  for (int i = tid; i < RB * NB; i += NT) {
+    const int w = i % RB, b = i / RB;
+    const size_t row = row0 + w;
+    const size_t z = row / N, y = row - z * N;
+    const int x0 = 32 * b;
+    edge[(z * NB + b) * N + y] = make_float4(phi_at(x0 == 0 ? N - 1 : x0 - 1, w), phi_at(x0, w), phi_at(x0 + 1, w), 0.f);
+  }
+}
+
 template <typename R, typename Tin, int N, int RB>
 __device__ __forceinline__ void r2c_body(const Tin* __restrict__ rho, cpx<R>* __restrict__ H, cpx<R>* __restrict__ Q,
                                          const cpx<R>* __restrict__ twg, long blk, cpx<R>* lds, cpx<R>* tw) {
@@ -79,40 +179,7 @@ __device__ __forceinline__ void r2c_body(const Tin* __restrict__ rho, cpx<R>* __
   __syncthreads();
   fft_passes<T, M, 1, -1, RB, SN, NT, 2>(lds, tw, tid);
 
-  constexpr int NPAIR = M / 2 + 1;
-  constexpr int TOTP = NPAIR * RB;
-  constexpr int PERP = (TOTP + NT - 1) / NT;
-  T zk[PERP], zm[PERP];
-#pragma unroll
-  for (int i = 0; i < PERP; ++i) {
-    const int b = tid + i * NT;
-    if (b < TOTP) {
-      const int w = b % RB, k = b / RB;
-      zk[i] = lds[k * SN + w];
-      zm[i] = lds[((M - k) % M) * SN + w];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < PERP; ++i) {
-    const int b = tid + i * NT;
-    if (b < TOTP) {
-      const int w = b % RB, k = b / RB;
-      // E = (Z[k] + conj Z[M-k]) / 2 ; O = (Z[k] - conj Z[M-k]) / (2i)
-      const T a = zk[i], c = zm[i];
-      const T E = cmake<T>(R(0.5) * (a.x + c.x), R(0.5) * (a.y - c.y));
-      const T O = cmake<T>(R(0.5) * (a.y + c.y), R(-0.5) * (a.x - c.x));
-      const T wO = cmul(O, tw[k]);
-      if (k == 0) {
-        lds[w] = cmake<T>(E.x + wO.x, R(0));
-        Q[row0 + w] = cmake<T>(E.x - wO.x, R(0));
-      } else {
-        lds[k * SN + w] = cadd(E, wO);                       // X[k]
-        if (2 * k != M) lds[(M - k) * SN + w] = cconj(csub(E, wO));  // X[M-k]
-      }
-    }
-  }
-  __syncthreads();
+  untangle_rows<R, N, RB, SN, NT>(lds, tw, tid, [&](int w, R x) { Q[row0 + w] = cmake<T>(x, R(0)); });
   T* dst = H + row0 * M;
 #pragma unroll 4
   for (int e = tid; e < RB * M; e += NT) {
@@ -174,57 +241,10 @@ __device__ __forceinline__ void c2r_body(const cpx<R>* H, const cpx<R>* __restri
   }
   __syncthreads();
 
-  constexpr int NPAIR = M / 2 + 1;
-  constexpr int TOTP = NPAIR * RB;
-  constexpr int PERP = (TOTP + NT - 1) / NT;
-  T xk[PERP], xm[PERP];
-#pragma unroll
-  for (int i = 0; i < PERP; ++i) {
-    const int b = tid + i * NT;
-    if (b < TOTP) {
-      const int w = b % RB, k = b / RB;
-      xk[i] = lds[k * SN + w];
-      xm[i] = (k == 0) ? qx[w] : lds[(M - k) * SN + w];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < PERP; ++i) {
-    const int b = tid + i * NT;
-    if (b < TOTP) {
-      const int w = b % RB, k = b / RB;
-      const T A = cadd(xk[i], cconj(xm[i]));
-      const T B = csub(xk[i], cconj(xm[i]));
-      const T wk = tw[k];
-      // Z[k] = A + i conj(w^k) B
-      const T cb = cmulc(B, wk);
-      lds[k * SN + w] = cmake<T>(A.x - cb.y, A.y + cb.x);
-      if (k != 0 && 2 * k != M) {
-        // Z[M-k] = conj(A) + i w^k conj(B)
-        const T wb = cmul(cconj(B), wk);
-        lds[(M - k) * SN + w] = cmake<T>(A.x - wb.y, -A.y + wb.x);
-      }
-    }
-  }
-  __syncthreads();
+  tangle_rows<R, N, RB, SN, NT>(lds, tw, tid, [&](int w) { return qx[w]; });
   fft_passes<T, M, 1, +1, RB, SN, NT, 2>(lds, tw, tid);
-  if constexpr (sizeof(R) == 4 && sizeof(Tout) == 4 && N % 32 == 0) {
-    if (edge) {
-      constexpr int NB = N / 32;
-      auto phi_at = [&](int x, int w) {
-        const T v = lds[(x >> 1) * SN + w];
-        return (x & 1) ? v.y : v.x;
-      };
-      for (int i = tid; i < RB * NB; i += NT) {
-        const int w = i % RB, b = i / RB;
-        const size_t row = row0 + w;
-        const size_t z = row / N, y = row - z * N;
-        const int x0 = 32 * b;
-        edge[(z * NB + b) * N + y] = make_float4(phi_at(x0 == 0 ? N - 1 : x0 - 1, w), phi_at(x0, w),
-                                                 phi_at(x0 + 1, w), 0.f);
-      }
-    }
-  }
+  if constexpr (sizeof(R) == 4 && sizeof(Tout) == 4 && N % 32 == 0)
+    if (edge) write_edge<N, RB, SN, NT>(lds, edge, row0, tid);
   cpx<Tout>* dst = reinterpret_cast<cpx<Tout>*>(out) + row0 * M;
 #pragma unroll 4
   for (int e = tid; e < RB * M; e += NT) {
@@ -243,6 +263,85 @@ __global__ __launch_bounds__(kThreads) void k_c2r_x(const cpx<R>* H, const cpx<R
   __shared__ cpx<R> qx[RB];
   c2r_body<R, Tout, N, RB>(H, Q, out, twg, rev ? xcd_block(blockIdx.x, gridDim.x, 1) : (int)blockIdx.x, lds, tw,
                            qx, edge);
+}
+
+// ------------------------------------------------------------------------------------------
+// x and y passes of one z plane in LDS
+//
+// On small grids a pass is a few microseconds of latency: start, one round trip to memory, the
+// transform, stores, drain.  Where a plane's half spectrum fits in LDS, one block transforms it along
+// x and y (the same Stockham passes in the same order, so the same bits), two launches and a round
+// trip through memory less per transform.  Sequence k of the plane (kx = k, k = M the Nyquist column)
+// runs along y at lds[k*SN + y]; SN = N + 1 keeps both directions free of bank conflicts.
+// ------------------------------------------------------------------------------------------
+// Every size whose plane fits in LDS takes it.  Step of a resident run, separate / plane passes, us:
+// FP32 32^3 36.7 / 32.3, 64^3 44.3 / 38.8, 96^3 57.8 / 52.5, 128^3 76.5 / 70.1, 192^3 133 / 125 (one
+// block of 151 KB per CU); FP64 64^3 47.5 / 42.7, 96^3 68.2 / 65.6, 128^3 97.6 / 86.9.  A 64^3 Poisson
+// solve of float32 arrays 33.9 / 27.7.
+template <typename R, int N> constexpr bool plane_pass() { return N <= (sizeof(R) == 4 ? 192 : 128); }
+// one radix-8 butterfly per thread and pass or a little more
+template <int N> constexpr int plane_threads() { return N >= 96 ? 1024 : N >= 64 ? 512 : 256; }
+
+template <typename R, typename Tin, int N>
+__global__ __launch_bounds__(plane_threads<N>()) void k_plane_r2c(const Tin* __restrict__ rho, cpx<R>* __restrict__ H,
+                                                                  cpx<R>* __restrict__ Q,
+                                                                  const cpx<R>* __restrict__ twg) {
+  using T = cpx<R>;
+  constexpr int M = N / 2, SN = N + 1, NT = plane_threads<N>();
+  __shared__ T lds[(M + 1) * SN];
+  __shared__ T tw[N];
+  const int tid = threadIdx.x, z = blockIdx.x;
+  for (int i = tid; i < N; i += NT) tw[i] = twg[i];
+  const cpx<Tin>* src = reinterpret_cast<const cpx<Tin>*>(rho) + (size_t)z * N * M;
+#pragma unroll 8
+  for (int e = tid; e < N * M; e += NT) {
+    const int y = e / M, n = e - y * M;
+    const cpx<Tin> u = src[e];
+    lds[n * SN + y] = cmake<T>(R(u.x), R(u.y));
+  }
+  __syncthreads();
+  fft_passes<T, M, 1, -1, N, SN, NT, 2>(lds, tw, tid);
+  untangle_rows<R, N, N, SN, NT>(lds, tw, tid, [&](int w, R x) { lds[M * SN + w] = cmake<T>(x, R(0)); });
+  fft_passes<T, N, 1, -1, M + 1, 1, NT, 1, SN>(lds, tw, tid);
+  T* dst = H + (size_t)z * N * M;
+#pragma unroll 8
+  for (int e = tid; e < N * M; e += NT) {
+    const int y = e / M, k = e - y * M;
+    dst[e] = lds[k * SN + y];
+  }
+  for (int y = tid; y < N; y += NT) Q[(size_t)z * N + y] = lds[M * SN + y];
+}
+
+template <typename R, typename Tout, int N>
+__global__ __launch_bounds__(plane_threads<N>()) void k_plane_c2r(const cpx<R>* H, const cpx<R>* __restrict__ Q,
+                                                                  Tout* out, const cpx<R>* __restrict__ twg,
+                                                                  float4* __restrict__ edge) {
+  using T = cpx<R>;
+  constexpr int M = N / 2, SN = N + 1, NT = plane_threads<N>();
+  __shared__ T lds[(M + 1) * SN];
+  __shared__ T tw[N];
+  const int tid = threadIdx.x, z = blockIdx.x;
+  for (int i = tid; i < N; i += NT) tw[i] = twg[i];
+  const T* src = H + (size_t)z * N * M;
+#pragma unroll 8
+  for (int e = tid; e < N * M; e += NT) {
+    const int y = e / M, k = e - y * M;
+    lds[k * SN + y] = src[e];
+  }
+  for (int y = tid; y < N; y += NT) lds[M * SN + y] = Q[(size_t)z * N + y];
+  __syncthreads();
+  fft_passes<T, N, 1, +1, M + 1, 1, NT, 1, SN>(lds, tw, tid);
+  tangle_rows<R, N, N, SN, NT>(lds, tw, tid, [&](int w) { return lds[M * SN + w]; });
+  fft_passes<T, M, 1, +1, N, SN, NT, 2>(lds, tw, tid);
+  if constexpr (sizeof(R) == 4 && sizeof(Tout) == 4 && N % 32 == 0)
+    if (edge) write_edge<N, N, SN, NT>(lds, edge, (size_t)z * N, tid);
+  cpx<Tout>* dst = reinterpret_cast<cpx<Tout>*>(out) + (size_t)z * N * M;
+#pragma unroll 8
+  for (int e = tid; e < N * M; e += NT) {
+    const int y = e / M, n = e - y * M;
+    const T u = lds[n * SN + y];
+    dst[e] = cmake<cpx<Tout>>(Tout(u.x), Tout(u.y));
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -899,6 +998,59 @@ bool fft_size_supported(int n) {
       return false;
   }
 }
+
+bool fft_plane_supported(int n, int prec) {
+  switch (n) {
+#define PM_CASE(NN) case NN: return prec == 4 ? plane_pass<float, NN>() : plane_pass<double, NN>();
+    PM_FOR_EACH_N(PM_CASE)
+#undef PM_CASE
+  }
+  return false;
+}
+
+template <typename R, typename Tin>
+hipError_t fft_r2c_xy(const Tin* rho, cpx<R>* H, cpx<R>* Q, int n, const FftTables& t, hipStream_t st) {
+  switch (n) {
+#define PM_CASE(NN)                                                                                              \
+  case NN:                                                                                                       \
+    if constexpr (plane_pass<R, NN>()) {                                                                         \
+      k_plane_r2c<R, Tin, NN><<<NN, plane_threads<NN>(), 0, st>>>(rho, H, Q, (const cpx<R>*)t.tw);               \
+      return hipGetLastError();                                                                                  \
+    }                                                                                                            \
+    break;
+    PM_FOR_EACH_N(PM_CASE)
+#undef PM_CASE
+  }
+  return hipErrorInvalidValue;
+}
+template <typename R, typename Tout>
+hipError_t fft_c2r_yx(const cpx<R>* H, const cpx<R>* Q, Tout* out, int n, const FftTables& t, hipStream_t st,
+                      float4* edge) {
+  switch (n) {
+#define PM_CASE(NN)                                                                                              \
+  case NN:                                                                                                       \
+    if constexpr (plane_pass<R, NN>()) {                                                                         \
+      k_plane_c2r<R, Tout, NN><<<NN, plane_threads<NN>(), 0, st>>>(H, Q, out, (const cpx<R>*)t.tw, edge);        \
+      return hipGetLastError();                                                                                  \
+    }                                                                                                            \
+    break;
+    PM_FOR_EACH_N(PM_CASE)
+#undef PM_CASE
+  }
+  return hipErrorInvalidValue;
+}
+
+template hipError_t fft_r2c_xy<float, float>(const float*, cpx<float>*, cpx<float>*, int, const FftTables&, hipStream_t);
+template hipError_t fft_r2c_xy<double, double>(const double*, cpx<double>*, cpx<double>*, int, const FftTables&,
+                                               hipStream_t);
+template hipError_t fft_r2c_xy<double, float>(const float*, cpx<double>*, cpx<double>*, int, const FftTables&,
+                                              hipStream_t);
+template hipError_t fft_c2r_yx<float, float>(const cpx<float>*, const cpx<float>*, float*, int, const FftTables&,
+                                             hipStream_t, float4*);
+template hipError_t fft_c2r_yx<double, double>(const cpx<double>*, const cpx<double>*, double*, int, const FftTables&,
+                                               hipStream_t, float4*);
+template hipError_t fft_c2r_yx<double, float>(const cpx<double>*, const cpx<double>*, float*, int, const FftTables&,
+                                              hipStream_t, float4*);
 
 template <typename R, typename Tin>
 hipError_t fft_r2c_x(const Tin* rho, cpx<R>* H, cpx<R>* Q, int n, const FftTables& t, hipStream_t st, bool rev) {

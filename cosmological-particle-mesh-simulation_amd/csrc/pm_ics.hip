@@ -189,8 +189,7 @@ hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, cons
   // 2. its half spectrum in wbuf (H part, then the Nyquist plane)
   cpx<R>* WH = reinterpret_cast<cpx<R>*>(wbuf);
   cpx<R>* WQ = WH + (long)n * n * (n / 2);
-  if (hipError_t e = fft_r2c_x<R, R>(hbuf, WH, WQ, n, t, st)) return e;
-  if (hipError_t e = fft_c2c_y<R>(WH, WQ, n, -1, t, st)) return e;
+  if (hipError_t e = fft_forward_xy<R, R>(hbuf, WH, WQ, n, t, st)) return e;
   if (hipError_t e = fft_c2c_z<R>(WH, WQ, n, -1, t, st)) return e;
   // 3. per component: k-space operator, inverse transform, particles
   cpx<R>* H = reinterpret_cast<cpx<R>*>(hbuf);
@@ -199,8 +198,7 @@ hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, cons
     k_zeldovich_component<R><<<grid_for(total), kB, 0, st>>>(WH, WQ, H, qbuf, d_amp, n, d, scale);
     if (hipError_t e = hipGetLastError()) return e;
     if (hipError_t e = fft_c2c_z<R>(H, qbuf, n, +1, t, st)) return e;
-    if (hipError_t e = fft_c2c_y<R>(H, qbuf, n, +1, t, st)) return e;
-    if (hipError_t e = fft_c2r_x<R, R>(H, qbuf, hbuf, n, t, st)) return e;
+    if (hipError_t e = fft_inverse_yx<R, R>(H, qbuf, hbuf, n, t, st)) return e;
     k_zeldovich_particles<R><<<grid_for(L.np), kB, 0, st>>>(hbuf, s, v, L, d, vel_factor);
     if (hipError_t e = hipGetLastError()) return e;
   }
