@@ -1138,9 +1138,11 @@ PM_API int pm_sim_set_tiles(pm_sim* s, int tx, int ty, int tz) {
   if (!s) return fail(PM_E_INVALID, "null sim");
   if ((tx || ty || tz) && !tile_shape_supported(tx, ty, tz))
     return fail(PM_E_UNSUPPORTED, "tile shape %dx%dx%d is not instantiated", tx, ty, tz);
-  if (s->ens && !(tx == 16 && ty == 16 && tz == 16) && (tx || ty || tz))
-    return fail(PM_E_STATE, "ensemble members keep 16^3 tiles");
-  if (s->ens) tx = ty = tz = 16;  // the default of a member is the ensemble's shape
+  if (s->ens) {  // 16^3 and the default both leave a member in its ensemble's shape
+    if (!(tx == 16 && ty == 16 && tz == 16) && (tx || ty || tz))
+      return fail(PM_E_STATE, "ensemble members keep the ensemble's tile shape");
+    return PM_OK;
+  }
   return sim_use_tiles(s, make_tiles(s->L.n, s->prec, tx, ty, tz));
 }
 
@@ -1183,7 +1185,7 @@ PM_API int pm_sim_get_tiles(pm_sim* s, int* tx, int* ty, int* tz) {
 PM_API int pm_sim_autotune(pm_sim* s, int reps, int* tx, int* ty, int* tz, double* best_ms) {
   if (!s) return fail(PM_E_INVALID, "null sim");
   if (!s->has_state) return fail(PM_E_STATE, "state was never set");
-  if (s->ens) return fail(PM_E_STATE, "ensemble members keep 16^3 tiles");
+  if (s->ens) return fail(PM_E_STATE, "ensemble members keep the ensemble's tile shape");
   int rc = s->prec == 4 ? sim_autotune_impl<float>(s, std::max(reps, 1), best_ms)
                         : sim_autotune_impl<double>(s, std::max(reps, 1), best_ms);
   if (rc) return rc;
@@ -1725,6 +1727,8 @@ void ens_describe(pm_ensemble* e) {
     m.fgrid = s->fgrid;
     m.local_hist = (s->G.ntx >= 4 && s->G.nty >= 4 && s->G.ntz >= 4) ? 1 : 0;
     m.tile_scatter = (s->B.tile_scatter && tile_scatter_ok(s->G)) ? 1 : 0;
+    m.wide = s->G.tx == 32 ? 1 : 0;
+    m.edge = m.wide ? s->edge : nullptr;
     for (int b = 0; b < 2; ++b) {
       m.s[b] = (float*)s->sb[b];
       m.v[b] = (float*)s->vb[b];
@@ -1850,8 +1854,6 @@ int ens_check_member(const pm_sim* s) {
   if (!batch_size_supported(s->L.n))
     return fail(PM_E_UNSUPPORTED, "N_CELLS=%d is not a batched grid size (32, 48, 64, 96, 128, 192, 256, 384, 512)",
                 s->L.n);
-  if (s->G.tx != 16 || s->G.ty != 16 || s->G.tz != 16)
-    return fail(PM_E_UNSUPPORTED, "ensemble members need 16^3 tiles");
   return PM_OK;
 }
 
@@ -1903,9 +1905,10 @@ PM_API int pm_ensemble_add(pm_ensemble* e, pm_sim* s) {
   if (s->ens == e) return fail(PM_E_INVALID, "the sim is already a member");
   if (s->ens) return fail(PM_E_STATE, "the sim is a member of another ensemble");
   if ((int)e->members.size() >= kBatchMax) return fail(PM_E_UNSUPPORTED, "an ensemble holds at most %d sims", kBatchMax);
-  if (s->G.tx != 16 || s->G.ty != 16 || s->G.tz != 16)  // members share the 16^3 tile kernels
-    if (int rc = sim_use_tiles(s, make_tiles(s->L.n, s->prec, 16, 16, 16))) return rc;
   if (int rc = ens_check_member(s)) return rc;
+  const TileGeom g = batch_tiles(s->L.n);
+  if (s->G.tx != g.tx || s->G.ty != g.ty || s->G.tz != g.tz)
+    if (int rc = sim_use_tiles(s, g)) return rc;
   PM_HIP(hipStreamSynchronize(e->stream));
   e->members.push_back(s);
   s->ens = e;

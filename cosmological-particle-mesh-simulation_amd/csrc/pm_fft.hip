@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_c2r(const BatchDesc* __restr
   case NN: {                                                                                     \
     cpx<float>* tw = lds + (NN / 2) * (x_rb<NN>() + 1);                                          \
     c2r_body<float, float, NN, x_rb<NN>()>(gmem(m.H), gmem(m.Q), gmem(reinterpret_cast<float*>(m.H)), \
-                                           gmem(m.tw), blk, lds, tw, tw + NN);                   \
+                                           gmem(m.tw), blk, lds, tw, tw + NN, gmem(m.edge));     \
     break;                                                                                       \
   }
   PM_BATCH_CLASS_SWITCH(CLS, m.n, PM_CASE)

@@ -1239,17 +1239,27 @@ __global__ __launch_bounds__(kT, sizeof(R) == 4 && LOCAL_HIST ? 7 : 1) void k_gk
 }
 
 // ------------------------------------------------------------------------------------------
-// batched tile kernels: the tiles (or particle blocks) of every member in one launch, FP32,
-// 16^3 tiles.  The XCD remap is applied to the ensemble-wide block index, so every XCD works
+// batched tile kernels: the tiles (or particle blocks) of every member in one launch, FP32, in
+// 32x8x8 or 16x16x8 tiles (batch_tiles).  The XCD remap is applied to the ensemble-wide block index, so every XCD works
 // on one contiguous run of tiles.
 // ------------------------------------------------------------------------------------------
-constexpr int kBT = 16;
+// runs CALL(X, Y, Z) with the member's tile shape
+#define PM_BATCH_TILES(m, CALL) \
+  do {                          \
+    if ((m).wide) CALL(32, 8, 8); \
+    else CALL(16, 16, 8);       \
+  } while (0)
+constexpr int kBatchBox = gkd_box_cells<32, 8, 8>() > gkd_box_cells<16, 16, 8>() ? gkd_box_cells<32, 8, 8>()
+                                                                                 : gkd_box_cells<16, 16, 8>();
+constexpr int kBatchAcc = deposit_lds_cells<32, 8, 8>() > deposit_lds_cells<16, 16, 8>()
+                              ? deposit_lds_cells<32, 8, 8>()
+                              : deposit_lds_cells<16, 16, 8>();
 
 // TS: the members with the tile scatter (stage BS_GKD_TS), otherwise the others (BS_GKD); each
 // launch holds one code path, so the tile scatter's reservations cost the others no registers
 template <bool TS>
-__global__ __launch_bounds__(kT, TS ? 5 : 1) void k_batch_gkd(const BatchDesc* __restrict__ D) {
-  __shared__ float box[gkd_box_cells<kBT, kBT, kBT>()];
+__global__ __launch_bounds__(kT, TS ? 7 : 1) void k_batch_gkd(const BatchDesc* __restrict__ D) {
+  __shared__ float box[kBatchBox];
   __shared__ uint32_t hist[kBins];
   constexpr int stage = TS ? BS_GKD_TS : BS_GKD;
   const long b = xcd_tile(blockIdx.x, gridDim.x);
@@ -1263,15 +1273,20 @@ __global__ __launch_bounds__(kT, TS ? 5 : 1) void k_batch_gkd(const BatchDesc* _
   const GkdState<float> ps{gmem(m.s[in]),     gmem(m.v[in]),     gmem(m.id[in]),
                            gmem(m.s[in ^ 1]), gmem(m.v[in ^ 1]), gmem(m.id[in ^ 1])};
   const float* phi = gmem(reinterpret_cast<const float*>(m.H));
-  if (TS)
-    gkd_body<float, kBT, kBT, kBT, true, true>(ps, phi, kick, drift, m.L, m.G, gmem(m.offsets), gmem(m.entries),
-                                               gmem(m.counts), m.capacity, tile, box, hist);
-  else if (m.local_hist)
-    gkd_body<float, kBT, kBT, kBT, true>(ps, phi, kick, drift, m.L, m.G, gmem(m.offsets), gmem(m.entries),
-                                         gmem(m.counts), m.capacity, tile, box, hist);
-  else
-    gkd_body<float, kBT, kBT, kBT, false>(ps, phi, kick, drift, m.L, m.G, gmem(m.offsets), gmem(m.entries),
-                                          gmem(m.counts), m.capacity, tile, box, hist);
+#define PM_L(X, Y, Z)                                                                                              \
+  do {                                                                                                             \
+    if (TS)                                                                                                        \
+      gkd_body<float, X, Y, Z, true, true>(ps, phi, kick, drift, m.L, m.G, gmem(m.offsets), gmem(m.entries),       \
+                                           gmem(m.counts), m.capacity, tile, box, hist, gmem(m.edge));             \
+    else if (m.local_hist)                                                                                         \
+      gkd_body<float, X, Y, Z, true>(ps, phi, kick, drift, m.L, m.G, gmem(m.offsets), gmem(m.entries),             \
+                                     gmem(m.counts), m.capacity, tile, box, hist, gmem(m.edge));                   \
+    else                                                                                                           \
+      gkd_body<float, X, Y, Z, false>(ps, phi, kick, drift, m.L, m.G, gmem(m.offsets), gmem(m.entries),            \
+                                      gmem(m.counts), m.capacity, tile, box, hist, gmem(m.edge));                  \
+  } while (0)
+  PM_BATCH_TILES(m, PM_L);
+#undef PM_L
 }
 
 // state buffer the binning and the deposit read: the gather's output (the scan has advanced
@@ -1281,20 +1296,24 @@ __device__ __forceinline__ int batch_state(const BatchDesc* D, const BatchMember
 }
 
 __global__ __launch_bounds__(kT) void k_batch_deposit(const BatchDesc* __restrict__ D) {
-  __shared__ double acc[deposit_lds_cells<kBT, kBT, kBT>()];
+  __shared__ double acc[kBatchAcc];
   const long b = xcd_tile(blockIdx.x, gridDim.x);
   const int k = batch_member(D, BS_TILES, b);
   const BatchMember& m = D->m[k];
   const int cur = batch_state(D, m);
   const int tile = (int)(b - D->off[BS_TILES][k]);
-  if (m.det_fix > 0.0)
-    deposit_body<float, kBT, kBT, kBT, true>(gmem(m.s[cur]), gmem(m.id[cur]), gmem(m.rho), m.mass, m.L, m.G,
-                                             gmem(m.offsets), gmem(m.entries), m.capacity, tile, acc, gmem(m.health),
-                                             m.det_fix);
-  else
-    deposit_body<float, kBT, kBT, kBT, false>(gmem(m.s[cur]), gmem(m.id[cur]), gmem(m.rho), m.mass, m.L, m.G,
-                                              gmem(m.offsets), gmem(m.entries), m.capacity, tile, acc,
-                                              gmem(m.health));
+#define PM_L(X, Y, Z)                                                                                              \
+  do {                                                                                                             \
+    if (m.det_fix > 0.0)                                                                                           \
+      deposit_body<float, X, Y, Z, true>(gmem(m.s[cur]), gmem(m.id[cur]), gmem(m.rho), m.mass, m.L, m.G,           \
+                                         gmem(m.offsets), gmem(m.entries), m.capacity, tile, acc, gmem(m.health),  \
+                                         m.det_fix);                                                               \
+    else                                                                                                           \
+      deposit_body<float, X, Y, Z, false>(gmem(m.s[cur]), gmem(m.id[cur]), gmem(m.rho), m.mass, m.L, m.G,          \
+                                          gmem(m.offsets), gmem(m.entries), m.capacity, tile, acc, gmem(m.health)); \
+  } while (0)
+  PM_BATCH_TILES(m, PM_L);
+#undef PM_L
 }
 
 // particle-parallel scatter of the members without the tile scatter (BS_SCATTER has no blocks
@@ -1305,9 +1324,11 @@ __global__ __launch_bounds__(kT) void k_batch_scatter(const BatchDesc* __restric
   const int k = batch_member(D, BS_SCATTER, b);
   const BatchMember& m = D->m[k];
   const int cur = batch_state(D, m);
-  bin_scatter_body<float, kBT, kBT, kBT>(gmem(m.s[cur]), gmem(m.id[cur]), m.L, m.G, gmem(m.offsets),
-                                         gmem(m.cursors), gmem(m.entries), m.capacity, b - D->off[BS_SCATTER][k],
-                                         gmem(m.health));
+#define PM_L(X, Y, Z)                                                                                               \
+  bin_scatter_body<float, X, Y, Z>(gmem(m.s[cur]), gmem(m.id[cur]), m.L, m.G, gmem(m.offsets), gmem(m.cursors),    \
+                                   gmem(m.entries), m.capacity, b - D->off[BS_SCATTER][k], gmem(m.health))
+  PM_BATCH_TILES(m, PM_L);
+#undef PM_L
 }
 
 template <int NT>
@@ -1317,9 +1338,12 @@ __global__ __launch_bounds__(NT) void k_batch_tile_scatter(const BatchDesc* __re
   const int k = batch_member(D, BS_TILE_SCATTER, b);
   const BatchMember& m = D->m[k];
   const int cur = batch_state(D, m);
-  tile_scatter_body<float, kBT, kBT, kBT, NT>(gmem(m.s[cur]), gmem(m.id[cur]), m.L, m.G, gmem(m.offsets),
-                                          gmem(m.cursors), gmem(m.entries), m.capacity, gmem(m.health),
-                                          gmem(m.counts), (int)(b - D->off[BS_TILE_SCATTER][k]), cur_bins, lim_bins);
+#define PM_L(X, Y, Z)                                                                                                \
+  tile_scatter_body<float, X, Y, Z, NT>(gmem(m.s[cur]), gmem(m.id[cur]), m.L, m.G, gmem(m.offsets),                 \
+                                        gmem(m.cursors), gmem(m.entries), m.capacity, gmem(m.health),               \
+                                        gmem(m.counts), (int)(b - D->off[BS_TILE_SCATTER][k]), cur_bins, lim_bins)
+  PM_BATCH_TILES(m, PM_L);
+#undef PM_L
 }
 
 __global__ __launch_bounds__(kT) void k_batch_scan_reduce(const BatchDesc* __restrict__ D) {

@@ -17,6 +17,11 @@ MAX_MEMBERS = 64
 BATCH_SIZES = (32, 48, 64, 96, 128, 192, 256, 384, 512)
 
 
+def ensemble_tiles(n_cells: int) -> tuple[int, int, int]:
+    """Tile shape of a member on an n_cells^3 grid (a sim takes it when it joins)."""
+    return (32, 8, 8) if n_cells >= 128 else (16, 16, 8)
+
+
 class PMEnsemble:
     def __init__(self, sims=()):
         _lib.init()

@@ -28,7 +28,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from .ensemble import MAX_MEMBERS, PMEnsemble
+from .ensemble import MAX_MEMBERS, PMEnsemble, ensemble_tiles
 from .sim import PMSim
 
 
@@ -125,7 +125,7 @@ def _start(req: SimRequest, prepared) -> PMSim:
     sim = PMSim(req.n_cells, req.n_parts, 32, omega_m0=req.om, omega_lambda0=req.ol,
                 omega_k0=req.ok, h0=req.h)
     try:
-        sim.set_tiles(16, 16, 16)   # the ensemble's shape: joining it keeps the bins and the density
+        sim.set_tiles(*ensemble_tiles(req.n_cells))   # joining keeps the bins and the density
         sim.zeldovich(amp, scale, vfac, seed=req.seed)
         sim.deposit()
     except Exception:
@@ -399,7 +399,7 @@ class PMServer:
 def run_alone(req: SimRequest, keep_state: bool = False, tiles=None) -> SimResult:
     """One request by itself: its own sim, device initial conditions, the graph-replayed
     step loop and the final power spectrum (the one-at-a-time way of serving).  ``tiles``
-    fixes the tile shape (the ensemble's 16^3 makes the run use the served kernels)."""
+    fixes the tile shape (``ensemble_tiles(n_cells)`` makes the run use the served kernels)."""
     t0 = time.perf_counter()
     sim = _start(req, _prepare(req))
     try:

@@ -41,12 +41,18 @@ def test_default_tiles_give_the_bits_of_8_cubed(n, prec):
 def test_member_keeps_the_ensemble_shape():
     from pmgpu.ensemble import PMEnsemble
     from pmgpu.sim import PMSim
-    s = PMSim(64, 32, 32, **KW)
-    ens = PMEnsemble([s])
-    assert s.tiles() == (16, 16, 16)
-    s.set_tiles(0, 0, 0)
-    x, v = _state(64, 32, 1)
-    s.set_state(x, v)
-    ens.run([0.5], [0.001], 2)
-    assert s.tiles() == (16, 16, 16)
-    ens.close()
+    from pmgpu.ensemble import ensemble_tiles
+    for n in (48, 64, 128, 256):
+        s = PMSim(n, 32, 32, **KW)
+        s.set_tiles(16, 16, 16)
+        ens = PMEnsemble([s])
+        assert s.tiles() == ensemble_tiles(n)
+        for tiles in ((0, 0, 0), (16, 16, 16)):      # both leave a member where it is
+            s.set_tiles(*tiles)
+            x, v = _state(n, 32, 1)
+            s.set_state(x, v)
+            ens.run([0.5], [0.001], 2)
+            assert s.tiles() == ensemble_tiles(n)
+        with pytest.raises(RuntimeError):
+            s.set_tiles(8, 8, 8)
+        ens.close()
