@@ -1574,7 +1574,7 @@ PM_API int pm_sim_zeldovich(pm_sim* s, const double* amp, int64_t n_amp, double 
   FftTables* t;
   if (int rc = get_tables(n, s->prec, &t)) return rc;
   double* d_amp = nullptr;
-  if (dev_malloc(&d_amp, sizeof(double) * need) != hipSuccess) return fail(PM_E_NOMEM, "amplitude table allocation failed");
+  if (pool_alloc((void**)&d_amp, sizeof(double) * need) != hipSuccess) return fail(PM_E_NOMEM, "amplitude table allocation failed");
   hipError_t e = hipMemcpyAsync(d_amp, amp, sizeof(double) * need, hipMemcpyHostToDevice, s->stream);
   if (e == hipSuccess) {
     if (s->prec == 4)
@@ -1588,7 +1588,7 @@ PM_API int pm_sim_zeldovich(pm_sim* s, const double* amp, int64_t n_amp, double 
     if (e == hipSuccess) e = ids_identity(s->idb[s->cur], s->L, s->stream);  // the state is in slot order
   }
   hipError_t es = hipStreamSynchronize(s->stream);
-  (void)hipFree(d_amp);
+  (void)pool_free(d_amp);
   if (e != hipSuccess || es != hipSuccess)
     return fail(PM_E_HIP, "device initial conditions failed: %s", hipGetErrorString(e ? e : es));
   s->has_state = s->slot_order = true;
@@ -1609,7 +1609,8 @@ PM_API int pm_sim_power_spectrum(pm_sim* s, double box, int n_bins, double* k, d
   const long cells = (long)n * n * n;
   double* d = nullptr;  // [0]: sum of rho, then 3 (n_bins + 1) shell sums
   const size_t nd = 1 + 3 * (size_t)(n_bins + 1);
-  if (dev_malloc(&d, sizeof(double) * nd) != hipSuccess) return fail(PM_E_NOMEM, "spectrum scratch allocation failed");
+  if (pool_alloc((void**)&d, sizeof(double) * nd) != hipSuccess)
+    return fail(PM_E_NOMEM, "spectrum scratch allocation failed");
   std::vector<double> h(nd);
   hipError_t e = hipMemsetAsync(d, 0, sizeof(double) * nd, s->stream);
   if (e == hipSuccess) {
@@ -1631,7 +1632,7 @@ PM_API int pm_sim_power_spectrum(pm_sim* s, double box, int n_bins, double* k, d
   }
   if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d, sizeof(double) * nd, hipMemcpyDeviceToHost, s->stream);
   hipError_t es = hipStreamSynchronize(s->stream);
-  (void)hipFree(d);
+  (void)pool_free(d);
   s->phi_valid = false;  // the potential buffer held the spectrum
   if (e != hipSuccess || es != hipSuccess)
     return fail(PM_E_HIP, "power spectrum failed: %s", hipGetErrorString(e ? e : es));
