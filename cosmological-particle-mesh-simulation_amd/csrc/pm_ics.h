@@ -35,10 +35,13 @@ __host__ __device__ inline void white4(long g, uint64_t seed, double z[4]) {
   const double two_pi = 6.283185307179586;
   const double r0 = sqrt(-2.0 * log(((double)u.x + 0.5) * s)), t0 = two_pi * (((double)u.y + 0.5) * s);
   const double r1 = sqrt(-2.0 * log(((double)u.z + 0.5) * s)), t1 = two_pi * (((double)u.w + 0.5) * s);
-  z[0] = r0 * cos(t0);
-  z[1] = r0 * sin(t0);
-  z[2] = r1 * cos(t1);
-  z[3] = r1 * sin(t1);
+  double s0, c0, s1, c1;
+  sincos(t0, &s0, &c0);
+  sincos(t1, &s1, &c1);
+  z[0] = r0 * c0;
+  z[1] = r0 * s0;
+  z[2] = r1 * c1;
+  z[3] = r1 * s1;
 }
 
 // n3 normal deviates (element e from white4(e / 4)) into out (float or double per prec)
@@ -46,11 +49,11 @@ hipError_t white_noise(void* out, int prec, long n3, uint64_t seed, hipStream_t 
 
 // Zel'dovich displacements and velocities of a lattice (L.np_side must be a supported FFT
 // size): noise = caller field (noise_bytes 4/8, device pointer) or NULL for white_noise(seed);
-// d_amp[m2] = sqrt(P(k) n^3 / V) D(a) for m2 = 0 .. 3 (n/2)^2; Psi = scale * IDFT(i m / m^2 A W),
+// d_amp[m2] = sqrt(P(k) n^3 / V) D(a) for m2 = 0 .. 3 (n/2)^2 (scaled in place); Psi = scale * IDFT(i m / m^2 A W),
 // scale = (N_CELLS / box) / (k_f n^3); s = Psi, v = vel_factor * Psi.  Scratch: wbuf holds
 // n^3 + 2 n^2 reals, hbuf n^3 reals, qbuf n^2 complex.
 template <typename R>
-hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, const double* d_amp, double scale,
+hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, double* d_amp, double scale,
                          double vel_factor, const Lattice& L, const FftTables& t, R* s, R* v, R* wbuf, R* hbuf,
                          cpx<R>* qbuf, hipStream_t st);
 

@@ -46,41 +46,48 @@ __global__ __launch_bounds__(kB) void k_copy_field(const Tin* __restrict__ in, R
 // signed mode number of index i on an n-point axis (numpy.fft.fftfreq order)
 __device__ __forceinline__ int signed_mode(int i, int n) { return i < n / 2 ? i : i - n; }
 
-// one displacement component's half spectrum from the noise spectrum W (H part + Nyquist plane)
+// amp[m2] -> scale * amp[m2] / m2 (0 for m2 = 0), in place: one division per |m|^2 instead of one per
+// mode and component
+__global__ __launch_bounds__(kB) void k_amplitude_scale(double* __restrict__ amp, long count, double scale) {
+  const long i = blockIdx.x * (long)kB + threadIdx.x;
+  if (i < count) amp[i] = i ? scale * amp[i] / (double)i : 0.0;
+}
+
+// one displacement component's half spectrum from the noise spectrum W (H part + Nyquist plane); a
+// thread takes two neighbouring modes of a row, the last blocks the Nyquist plane.  With 64-bit
+// divisions, an FP64 one and one mode per thread: 46 us at 256^3 for 134 MB of traffic, now 40 (one
+// thread for the four mirrored modes of a table value: 52).
 template <typename R>
 __global__ __launch_bounds__(kB) void k_zeldovich_component(const cpx<R>* __restrict__ WH, const cpx<R>* __restrict__ WQ,
                                                            cpx<R>* __restrict__ H, cpx<R>* __restrict__ Q,
-                                                           const double* __restrict__ amp, int n, int d,
-                                                           double scale) {
-  const long half = (long)n * n * (n / 2);
-  const long total = half + (long)n * n;
-  const long idx = blockIdx.x * (long)kB + threadIdx.x;
-  if (idx >= total) return;
-  int z, y, kx;
-  cpx<R> w;
-  if (idx < half) {
-    kx = (int)(idx % (n / 2));
-    y = (int)((idx / (n / 2)) % n);
-    z = (int)(idx / ((long)n * (n / 2)));
-    w = WH[idx];
+                                                           const double* __restrict__ amp, int n, FastDiv by_n,
+                                                           FastDiv by_pairs, uint32_t main_blocks, int d) {
+  struct alignas(2 * sizeof(cpx<R>)) Pair {
+    cpx<R> v[2];
+  };
+  const uint32_t pairs = by_pairs.d, rows = (uint32_t)n * (uint32_t)n;
+  const bool main = blockIdx.x < main_blocks;
+  const uint32_t idx = (main ? blockIdx.x : blockIdx.x - main_blocks) * (uint32_t)kB + threadIdx.x;
+  if (idx >= (main ? rows * pairs : rows)) return;
+  const uint32_t row = main ? by_pairs.div(idx) : idx;
+  const int kx = main ? 2 * (int)(idx - row * pairs) : n / 2;
+  const int z = (int)by_n.div(row), y = (int)(row - (uint32_t)z * (uint32_t)n);
+  const int mz = signed_mode(z, n), my = signed_mode(y, n);
+  auto mode = [&](int mx, cpx<R> w) {
+    // component d: derivative along lattice axis d = spectrum axis z, y, x for d = 0, 1, 2; its Nyquist
+    // plane is zero
+    const int md = d == 0 ? mz : (d == 1 ? my : mx);
+    const double f = (d == 0 ? z : d == 1 ? y : mx) == n / 2 ? 0.0 : amp[mx * mx + my * my + mz * mz] * (double)md;
+    return cmake<cpx<R>>(R(-f * (double)w.y), R(f * (double)w.x));  // i f w
+  };
+  if (main) {
+    Pair p = reinterpret_cast<const Pair*>(WH)[idx];
+    p.v[0] = mode(kx, p.v[0]);
+    p.v[1] = mode(kx + 1, p.v[1]);
+    reinterpret_cast<Pair*>(H)[idx] = p;
   } else {
-    const long j = idx - half;
-    kx = n / 2;
-    y = (int)(j % n);
-    z = (int)(j / n);
-    w = WQ[j];
+    Q[row] = mode(kx, WQ[row]);
   }
-  const int mz = signed_mode(z, n), my = signed_mode(y, n), mx = kx;
-  const long m2 = (long)mx * mx + (long)my * my + (long)mz * mz;
-  // component d: derivative along lattice axis d = spectrum axis z, y, x for d = 0, 1, 2
-  const int md = d == 0 ? mz : (d == 1 ? my : mx);
-  const int id = d == 0 ? z : (d == 1 ? y : kx);
-  double f = 0.0;
-  if (m2 > 0 && id != n / 2) f = scale * amp[m2] * (double)md / (double)m2;
-  // i * f * w
-  const cpx<R> out = cmake<cpx<R>>(R(-f * (double)w.y), R(f * (double)w.x));
-  if (idx < half) H[idx] = out;
-  else Q[idx - half] = out;
 }
 
 // particles of the lattice take component d of the displacement field (real [i][j][k] grid)
@@ -95,6 +102,32 @@ __global__ __launch_bounds__(kB) void k_zeldovich_particles(const R* __restrict_
   const R x = psi[p];
   s[d * L.np + slot] = wrap_disp<R>(x, R(L.n));
   v[d * L.np + slot] = R(vel_factor * (double)x);
+}
+
+// the same for lattices of 4^3 blocks, through LDS in whole cache lines (see kSlotK; 48 -> 30 us at 256^3)
+template <typename R>
+__global__ __launch_bounds__(kB) void k_zeldovich_slots(const R* __restrict__ psi, R* __restrict__ s, R* __restrict__ v,
+                                                        Lattice L, int d, double vel_factor) {
+  constexpr int PER = 16 * kSlotK / kB;
+  __shared__ R t[kSlotK * kSlotPitch];
+  const SlotRegion r = slot_region(L, blockIdx.x);
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    int ijk[3], at;
+    long p;
+    if (slot_ref(L, r, u * kB + threadIdx.x, ijk, p, at)) t[at] = psi[p];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    int at;
+    long slot;
+    if (slot_dev(L, r, u * kB + threadIdx.x, slot, at)) {
+      const R x = t[at];
+      s[d * L.np + slot] = wrap_disp<R>(x, R(L.n));
+      v[d * L.np + slot] = R(vel_factor * (double)x);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- power spectrum
@@ -193,7 +226,7 @@ hipError_t white_noise(void* out, int prec, long n3, uint64_t seed, hipStream_t 
 }
 
 template <typename R>
-hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, const double* d_amp, double scale,
+hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, double* d_amp, double scale,
                          double vel_factor, const Lattice& L, const FftTables& t, R* s, R* v, R* wbuf, R* hbuf,
                          cpx<R>* qbuf, hipStream_t st) {
   const int n = L.np_side;
@@ -213,13 +246,17 @@ hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, cons
   if (hipError_t e = fft_c2c_z<R>(WH, WQ, n, -1, t, st)) return e;
   // 3. per component: k-space operator, inverse transform, particles
   cpx<R>* H = reinterpret_cast<cpx<R>*>(hbuf);
-  const long total = (long)n * n * (n / 2) + (long)n * n;
+  const unsigned main_blocks = grid_for((long)n * n * (n / 4));  // (n is a multiple of 8)
+  const long n_amp = 3L * (n / 2) * (n / 2) + 1;
+  k_amplitude_scale<<<grid_for(n_amp), kB, 0, st>>>(d_amp, n_amp, scale);
   for (int d = 0; d < 3; ++d) {
-    k_zeldovich_component<R><<<grid_for(total), kB, 0, st>>>(WH, WQ, H, qbuf, d_amp, n, d, scale);
+    k_zeldovich_component<R><<<main_blocks + grid_for((long)n * n), kB, 0, st>>>(
+        WH, WQ, H, qbuf, d_amp, n, FastDiv((uint32_t)n), FastDiv((uint32_t)n / 4), main_blocks, d);
     if (hipError_t e = hipGetLastError()) return e;
     if (hipError_t e = fft_c2c_z<R>(H, qbuf, n, +1, t, st)) return e;
     if (hipError_t e = fft_inverse_yx<R, R>(H, qbuf, hbuf, n, t, st)) return e;
-    k_zeldovich_particles<R><<<grid_for(L.np), kB, 0, st>>>(hbuf, s, v, L, d, vel_factor);
+    if (L.lb == 2) k_zeldovich_slots<R><<<slot_blocks(L), kB, 0, st>>>(hbuf, s, v, L, d, vel_factor);
+    else k_zeldovich_particles<R><<<grid_for(L.np), kB, 0, st>>>(hbuf, s, v, L, d, vel_factor);
     if (hipError_t e = hipGetLastError()) return e;
   }
   return hipSuccess;
@@ -241,7 +278,7 @@ hipError_t shell_sums(const cpx<R>* H, const cpx<R>* Q, int n, int nb, double* d
 }
 
 #define PM_INST(R)                                                                                                \
-  template hipError_t zeldovich_ics<R>(const void*, int, uint64_t, const double*, double, double, const Lattice&, \
+  template hipError_t zeldovich_ics<R>(const void*, int, uint64_t, double*, double, double, const Lattice&, \
                                        const FftTables&, R*, R*, R*, R*, cpx<R>*, hipStream_t);                   \
   template hipError_t grid_sum<R>(const R*, long, double*, hipStream_t);                                          \
   template hipError_t shell_sums<R>(const cpx<R>*, const cpx<R>*, int, int, double*, hipStream_t);
