@@ -1421,15 +1421,15 @@ PM_API int pm_sim_get_state(pm_sim* s, void* pos, void* vel, int dtype_bytes, in
   }
   hipError_t e;
   const bool slots = s->slot_order;
-  const int nz = s->G.ntz;
+  uint32_t* work = (uint32_t*)s->sb[s->cur ^ 1];  // the next gather's output, unused until then
   const hipStream_t st = s->stream;
   if (s->prec == 4) {
-    e = dtype_bytes == 4 ? sim_get_state<float, float>(cur_state<float>(s), (float*)dp, (float*)dv, s->L, slots, nz, st)
-                         : sim_get_state<float, double>(cur_state<float>(s), (double*)dp, (double*)dv, s->L, slots, nz, st);
+    e = dtype_bytes == 4 ? sim_get_state<float, float>(cur_state<float>(s), (float*)dp, (float*)dv, s->L, slots, work, st)
+                         : sim_get_state<float, double>(cur_state<float>(s), (double*)dp, (double*)dv, s->L, slots, work, st);
   } else {
     e = dtype_bytes == 4
-            ? sim_get_state<double, float>(cur_state<double>(s), (float*)dp, (float*)dv, s->L, slots, nz, st)
-            : sim_get_state<double, double>(cur_state<double>(s), (double*)dp, (double*)dv, s->L, slots, nz, st);
+            ? sim_get_state<double, float>(cur_state<double>(s), (float*)dp, (float*)dv, s->L, slots, work, st)
+            : sim_get_state<double, double>(cur_state<double>(s), (double*)dp, (double*)dv, s->L, slots, work, st);
   }
   if (e == hipSuccess && !on_device) {
     e = hipMemcpyAsync(pos, dp, bytes, hipMemcpyDeviceToHost, s->stream);

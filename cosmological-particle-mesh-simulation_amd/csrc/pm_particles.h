@@ -175,10 +175,9 @@ template <typename R> struct PState {
 template <typename R, typename Tin>
 hipError_t sim_set_state(const Tin* pos, const Tin* vel, const PState<R>& p, const Lattice& L, hipStream_t st,
                          uint32_t* health = nullptr);
-// slot_order: the state is in slot order (id = storage index); otherwise it follows the tile bins of
-// some step, `layers` tiles along z (an order to walk it in: any value gives the same result)
+// slot_order: the state is in slot order (id = storage index); otherwise work holds N_p words of scratch
 template <typename R, typename Tout>
-hipError_t sim_get_state(const PState<R>& p, Tout* pos, Tout* vel, const Lattice& L, bool slot_order, int layers,
+hipError_t sim_get_state(const PState<R>& p, Tout* pos, Tout* vel, const Lattice& L, bool slot_order, uint32_t* work,
                          hipStream_t st);
 // id = storage index (slot order)
 hipError_t ids_identity(uint32_t* id, const Lattice& L, hipStream_t st);

@@ -98,13 +98,34 @@ __device__ __forceinline__ Tout state_pos(R q, R s, const Lattice& L) {
   return x >= Tout(L.n) ? Tout(0) : x;
 }
 
-// state in slot order (id = storage index)
+// where[slot] = storage index of that particle (ids outside the lattice are skipped)
+__global__ __launch_bounds__(kBlock) void k_where(const uint32_t* __restrict__ id, uint32_t* __restrict__ where, long np) {
+  const long e = blockIdx.x * (long)kBlock + threadIdx.x;
+  if (e >= np) return;
+  const uint32_t slot = id[e];
+  if (slot < (uint64_t)np) where[slot] = (uint32_t)e;
+}
+
+// State at storage index where[slot] (null: in slot order).  A wavefront's 64 slots are a 4^3 block of
+// the lattice, which a tile-ordered state keeps within a few cache lines of one or two tiles; writing
+// the reference's arrays straight from tile order instead, 4 bytes here and there, took 706 us at 256^3
+// particles (5.45 ms at 512^3) against 265 us (2.13 ms) for the two kernels.
 template <typename R, typename Tout>
 __global__ __launch_bounds__(kBlock) void k_get_slots(const R* __restrict__ s, const R* __restrict__ v,
-                                                      Tout* __restrict__ pos, Tout* __restrict__ vel, Lattice L) {
+                                                      const uint32_t* __restrict__ where, Tout* __restrict__ pos,
+                                                      Tout* __restrict__ vel, Lattice L) {
   constexpr int PER = 16 * kSlotK / kBlock;
   __shared__ R t[kSlotK * kSlotPitch];
   const SlotRegion r = slot_region(L, blockIdx.x);
+  uint32_t from[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    int at;
+    long slot;
+    from[u] = 0u;
+    if (slot_dev(L, r, u * kBlock + threadIdx.x, slot, at))
+      from[u] = where ? min(where[slot], (uint32_t)(L.np - 1)) : (uint32_t)slot;
+  }
 #pragma unroll 1
   for (int d = 0; d < 6; ++d) {
     const R* src = (d < 3 ? s : v) + (d % 3) * L.np;
@@ -113,7 +134,7 @@ __global__ __launch_bounds__(kBlock) void k_get_slots(const R* __restrict__ s, c
     for (int u = 0; u < PER; ++u) {
       int at;
       long slot;
-      if (slot_dev(L, r, u * kBlock + threadIdx.x, slot, at)) t[at] = src[slot];
+      if (slot_dev(L, r, u * kBlock + threadIdx.x, slot, at)) t[at] = src[from[u]];
     }
     __syncthreads();
 #pragma unroll
@@ -128,17 +149,12 @@ __global__ __launch_bounds__(kBlock) void k_get_slots(const R* __restrict__ s, c
   }
 }
 
-// storage index e holds particle id[e]; ids outside the lattice are skipped.  Storage follows the
-// tiles of an earlier step, x fastest, so a block's writes are short runs along k of the reference's
-// arrays, and the rest of their cache lines belongs to the tiles above and below.  The blocks are
-// walked with the tile layers fastest (`layers` of them, `per` blocks each; exact for evenly spread
-// particles, nearly so otherwise), so the runs of a line meet in one L2 (256^3 particles after a run: 880 -> 706 us).
+// storage index e holds particle id[e]; ids outside the lattice are skipped (lattices without 4^3 blocks)
 template <typename R, typename Tout>
 __global__ __launch_bounds__(kBlock) void k_get_state(const R* __restrict__ s, const R* __restrict__ v,
                                                       const uint32_t* __restrict__ id, Tout* __restrict__ pos,
-                                                      Tout* __restrict__ vel, Lattice L, int layers, long per) {
-  const long c = xcd_block(blockIdx.x, gridDim.x);
-  const long e = ((c % layers) * per + c / layers) * kBlock + threadIdx.x;
+                                                      Tout* __restrict__ vel, Lattice L) {
+  const long e = blockIdx.x * (long)kBlock + threadIdx.x;
   if (e >= L.np) return;
   const uint32_t slot = id[e];
   if (slot >= (uint64_t)L.np) return;
@@ -382,14 +398,14 @@ hipError_t sim_set_state(const Tin* pos, const Tin* vel, const PState<R>& p, con
   return hipGetLastError();
 }
 template <typename R, typename Tout>
-hipError_t sim_get_state(const PState<R>& p, Tout* pos, Tout* vel, const Lattice& L, bool slot_order, int layers,
+hipError_t sim_get_state(const PState<R>& p, Tout* pos, Tout* vel, const Lattice& L, bool slot_order, uint32_t* work,
                          hipStream_t st) {
-  if (slot_order && L.lb == 2) {
-    k_get_slots<R, Tout><<<slot_blocks(L), kBlock, 0, st>>>(p.s, p.v, pos, vel, L);
-  } else {
-    const long per = (grid_for(L.np) + layers - 1) / layers;
-    k_get_state<R, Tout><<<(unsigned)(per * layers), kBlock, 0, st>>>(p.s, p.v, p.id, pos, vel, L, layers, per);
+  if (L.lb != 2) {
+    k_get_state<R, Tout><<<grid_for(L.np), kBlock, 0, st>>>(p.s, p.v, p.id, pos, vel, L);
+    return hipGetLastError();
   }
+  if (!slot_order) k_where<<<grid_for(L.np), kBlock, 0, st>>>(p.id, work, L.np);
+  k_get_slots<R, Tout><<<slot_blocks(L), kBlock, 0, st>>>(p.s, p.v, slot_order ? nullptr : work, pos, vel, L);
   return hipGetLastError();
 }
 hipError_t ids_identity(uint32_t* id, const Lattice& L, hipStream_t st) {
@@ -399,7 +415,7 @@ hipError_t ids_identity(uint32_t* id, const Lattice& L, hipStream_t st) {
 #define PM_INST(R, T)                                                                                  \
   template hipError_t sim_set_state<R, T>(const T*, const T*, const PState<R>&, const Lattice&, hipStream_t,   \
                                           uint32_t*);                                                          \
-  template hipError_t sim_get_state<R, T>(const PState<R>&, T*, T*, const Lattice&, bool, int, hipStream_t);
+  template hipError_t sim_get_state<R, T>(const PState<R>&, T*, T*, const Lattice&, bool, uint32_t*, hipStream_t);
 PM_INST(float, float)
 PM_INST(float, double)
 PM_INST(double, float)
