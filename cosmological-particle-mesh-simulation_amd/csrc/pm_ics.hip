@@ -255,7 +255,7 @@ hipError_t zeldovich_ics(const void* noise, int noise_bytes, uint64_t seed, doub
     if (hipError_t e = hipGetLastError()) return e;
     if (hipError_t e = fft_c2c_z<R>(H, qbuf, n, +1, t, st)) return e;
     if (hipError_t e = fft_inverse_yx<R, R>(H, qbuf, hbuf, n, t, st)) return e;
-    if (L.lb == 2) k_zeldovich_slots<R><<<slot_blocks(L), kB, 0, st>>>(hbuf, s, v, L, d, vel_factor);
+    if (slot_regions(L)) k_zeldovich_slots<R><<<slot_blocks(L), kB, 0, st>>>(hbuf, s, v, L, d, vel_factor);
     else k_zeldovich_particles<R><<<grid_for(L.np), kB, 0, st>>>(hbuf, s, v, L, d, vel_factor);
     if (hipError_t e = hipGetLastError()) return e;
   }

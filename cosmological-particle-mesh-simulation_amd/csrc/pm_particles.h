@@ -77,6 +77,10 @@ __host__ __device__ __forceinline__ void slot_to_ijk(long slot, const Lattice& L
 // through the 4 x 4 x 4 sites of a block with i first: a thread per slot touches 16 reference lines per
 // wavefront and uses 16 bytes of each.  Here a block of threads takes 4 x 4 rows of kSlotK sites and
 // turns them in LDS: 256-byte runs on both sides (256^3 particles: set 488 -> 218 us, get 568 -> 207).
+// Below kSlotMin particles the thread-per-particle kernels run: a region's six arrays in turn are a
+// longer chain than one thread's six accesses (32^3: set 4.2 against 10.5 us, get 5.1 against 12; 96^3:
+// set 16.1 and 17.5, get 27.2 and 22.8).
+constexpr long kSlotMin = 1 << 19;
 constexpr int kSlotK = 64;
 constexpr int kSlotPitch = 17;  // 16 rows + 1: both sides' lanes spread over the banks
 
@@ -93,6 +97,7 @@ __device__ __forceinline__ SlotRegion slot_region(const Lattice& L, int blk) {
   r.bj = blk / L.nb;
   return r;
 }
+inline bool slot_regions(const Lattice& L) { return L.lb == 2 && L.np >= kSlotMin; }
 inline unsigned slot_blocks(const Lattice& L) {
   return (unsigned)((long)((L.np_side + kSlotK - 1) / kSlotK) * L.nb * L.nb);
 }

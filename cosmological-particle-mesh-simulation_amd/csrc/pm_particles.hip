@@ -149,7 +149,8 @@ __global__ __launch_bounds__(kBlock) void k_get_slots(const R* __restrict__ s, c
   }
 }
 
-// storage index e holds particle id[e]; ids outside the lattice are skipped (lattices without 4^3 blocks)
+// storage index e holds particle id[e]; ids outside the lattice are skipped (lattices without slot
+// regions)
 template <typename R, typename Tout>
 __global__ __launch_bounds__(kBlock) void k_get_state(const R* __restrict__ s, const R* __restrict__ v,
                                                       const uint32_t* __restrict__ id, Tout* __restrict__ pos,
@@ -393,14 +394,14 @@ __global__ __launch_bounds__(kBlock) void k_convert(const Tin* __restrict__ in, 
 template <typename R, typename Tin>
 hipError_t sim_set_state(const Tin* pos, const Tin* vel, const PState<R>& p, const Lattice& L, hipStream_t st,
                          uint32_t* health) {
-  if (L.lb == 2) k_set_slots<R, Tin><<<slot_blocks(L), kBlock, 0, st>>>(pos, vel, p.s, p.v, p.id, L, health);
+  if (slot_regions(L)) k_set_slots<R, Tin><<<slot_blocks(L), kBlock, 0, st>>>(pos, vel, p.s, p.v, p.id, L, health);
   else k_set_state<R, Tin><<<grid_for(L.np), kBlock, 0, st>>>(pos, vel, p.s, p.v, p.id, L, health);
   return hipGetLastError();
 }
 template <typename R, typename Tout>
 hipError_t sim_get_state(const PState<R>& p, Tout* pos, Tout* vel, const Lattice& L, bool slot_order, uint32_t* work,
                          hipStream_t st) {
-  if (L.lb != 2) {
+  if (!slot_regions(L)) {
     k_get_state<R, Tout><<<grid_for(L.np), kBlock, 0, st>>>(p.s, p.v, p.id, pos, vel, L);
     return hipGetLastError();
   }

@@ -2,7 +2,7 @@
 lattices of 4^3 blocks and others, sides at and off the edges of the 64-site runs) and tile order
 (after steps, replayed graphs and ensemble runs).  With a zero time step every particle keeps its
 position and velocity, so what comes out is what went in, each at its reference index: float64 sims
-hold the displacement x - q to 2^-53 (positions within 1e-13 of a cell at N <= 72), float32 sims to
+hold the displacement x - q to 2^-53 (positions within 1e-13 of a cell at N <= 192), float32 sims to
 2^-24 of the largest displacement plus the float32 position's own rounding."""
 import numpy as np
 import pytest
@@ -28,11 +28,11 @@ def _check(got, want, prec):
     assert np.abs(periodic_diff(x, x0, N)).max() <= bar
 
 
-@pytest.mark.parametrize("side", [4, 5, 16, 20, 33, 34, 36])
+@pytest.mark.parametrize("side", [4, 5, 16, 20, 33, 34, 36, 80, 81, 84, 92])
 @pytest.mark.parametrize("prec", [32, 64])
 def test_state_comes_back_at_its_reference_index(side, prec):
     from pmgpu.sim import PMSim
-    n = 48 if side < 20 else 96
+    n = 48 if side < 20 else 96 if side < 80 else 192
     global N
     N = n
     dt = np.float32 if prec == 32 else np.float64
@@ -55,8 +55,8 @@ def test_state_after_ensemble_runs():
     from pmgpu.sim import PMSim
     global N
     N = 96
-    sims = [PMSim(96, p, 32, omega_m0=0.3, omega_lambda0=0.7, h0=0.7) for p in (32, 36)]
-    states = [_state(p, 7, np.float32) for p in (32, 36)]
+    sims = [PMSim(96, p, 32, omega_m0=0.3, omega_lambda0=0.7, h0=0.7) for p in (32, 84)]
+    states = [_state(p, 7, np.float32) for p in (32, 84)]
     ens = PMEnsemble(sims)
     for steps in (1, 64, 8):
         for s, (x, v) in zip(sims, states):
@@ -71,7 +71,7 @@ def test_non_finite_values_are_counted_once_per_particle():
     from pmgpu.sim import PMSim
     global N
     N = 96
-    for side in (20, 33):
+    for side in (20, 33, 84):
         x, v = _state(side, 3, np.float32)
         x[1, 17] = np.nan
         v[2, 17] = np.inf
