@@ -1526,6 +1526,69 @@ __global__ __launch_bounds__(kT) void k_ref_bin_lds(const float* __restrict__ po
   });
 }
 
+// The same for up to kRefWideKeys keys (147 KB of LDS, one block per CU): 1024 threads take 16 particles
+// each, so the passes over the table are few per particle, and read the positions again to place them.
+// For particle counts that are no cube, whose wavefronts run along the slowest axis through eight tiles
+// and more: count + scatter of 7.65 M clustered particles on 384^3 250 -> 177 us.  From kRefWideMin
+// particles on (whole density calls with / without, us: 1.0 M on 272^3 129 / 113, 2.1 M on 384^3
+// 179 / 183, 4.1 M 202 / 265, 8.0 M on 416^3 371 / 453): fewer are too few blocks.
+constexpr int kRefWideT = 1024, kRefWideP = 16;
+constexpr int kRefWideKeys = 36864;
+constexpr long kRefWideMin = 1 << 21;
+
+template <int TX, int TY, int TZ, bool HALO, bool SCATTER>
+__global__ __launch_bounds__(kRefWideT) void k_ref_bin_wide(const float* __restrict__ pos, long np, int n, TileGeom G,
+                                                            uint32_t* __restrict__ counts,
+                                                            const uint32_t* __restrict__ offsets,
+                                                            uint32_t* __restrict__ entries, uint32_t capacity) {
+  extern __shared__ uint32_t table[];
+  const int keys = (HALO ? 2 : 1) * G.ntiles;
+  const long first = blockIdx.x * (long)(kRefWideT * kRefWideP) + threadIdx.x;
+  auto each = [&](auto&& f) {
+#pragma unroll 1
+    for (int u0 = 0; u0 < kRefWideP; u0 += 4) {
+      float x[4][3];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const long p = first + (long)(u0 + u) * kRefWideT;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) x[u][a] = p < np ? pos[a * np + p] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const long p = first + (long)(u0 + u) * kRefWideT;
+        if (p >= np) continue;
+        int c[3], t[3], up[3];
+        float d[3];
+        abs_cell_and_frac(x[u][0], x[u][1], x[u][2], n, c, d);
+        tile_of<TX, TY, TZ>(c, G, t, up);
+        f(target_key(t, 0, G), (uint32_t)p);
+        if (HALO && (up[0] | up[1] | up[2])) {
+#pragma unroll 1
+          for (int o = 1; o < 8; ++o)
+            if (target_active(up, o)) f(target_key(t, o, G), (uint32_t)p);
+        }
+      }
+    }
+  };
+  for (int k = threadIdx.x; k < keys; k += kRefWideT) table[k] = 0u;
+  __syncthreads();
+  each([&](uint32_t key, uint32_t) { atomicAdd(&table[key], 1u); });
+  __syncthreads();
+  for (int k = threadIdx.x; k < keys; k += kRefWideT) {
+    const uint32_t cnt = table[k];
+    if (!cnt) continue;
+    if (SCATTER) table[k] = offsets[k] + atomicAdd(&counts[k], cnt);
+    else atomicAdd(&counts[k], cnt);
+  }
+  if (!SCATTER) return;
+  __syncthreads();
+  each([&](uint32_t key, uint32_t p) {
+    const uint32_t at = atomicAdd(&table[key], 1u);
+    if (at < capacity) entries[at] = p;
+  });
+}
+
 // More keys: device atomics from every wavefront, one per run of equal keys
 template <int TX, int TY, int TZ, bool HALO, bool SCATTER>
 __global__ __launch_bounds__(kT) void k_ref_bin(const float* __restrict__ pos, long np, int side, int n, TileGeom G,
@@ -1844,7 +1907,8 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
   const long nb = ref_blocks(np, side);
   const long nbl = (nb + kRefP - 1) / kRefP;
   const int keys = (halo ? 2 : 1) * G.ntiles;
-  const bool lds = keys <= kRefLdsKeys;
+  const bool lds = keys <= kRefLdsKeys, wide = !lds && side == 0 && np >= kRefWideMin && keys <= kRefWideKeys;
+  const unsigned nbw = (unsigned)((np + kRefWideT * kRefWideP - 1) / (kRefWideT * kRefWideP));
   // the counts and the scan's ticket after them (never captured: the callers synchronise)
   if (hipError_t e = hipMemsetAsync(B.counts, 0, (2 * (size_t)G.ntiles + 1) * sizeof(uint32_t), st)) return e;
 #define PM_ONE(X, Y, Z, HALO, SCATTER, CTR)                                                                          \
@@ -1852,7 +1916,15 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
     if (lds)                                                                                                         \
       k_ref_bin_lds<X, Y, Z, HALO, SCATTER>                                                                          \
           <<<nbl, kT, keys * sizeof(uint32_t), st>>>(pos, np, side, n, G, CTR, B.offsets, B.entries, B.capacity);    \
-    else                                                                                                             \
+    else if (wide) {                                                                                                 \
+      /* (blocks above 64 KiB of LDS have to be allowed) */                                                          \
+      static const hipError_t allowed =                                                                              \
+          hipFuncSetAttribute((const void*)k_ref_bin_wide<X, Y, Z, HALO, SCATTER>,                                   \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kRefWideKeys * sizeof(uint32_t));          \
+      if (allowed != hipSuccess) return allowed;                                                                     \
+      k_ref_bin_wide<X, Y, Z, HALO, SCATTER><<<nbw, kRefWideT, keys * sizeof(uint32_t), st>>>(                       \
+          pos, np, n, G, CTR, B.offsets, B.entries, B.capacity);                                                     \
+    } else                                                                                                           \
       k_ref_bin<X, Y, Z, HALO, SCATTER><<<nb, kT, 0, st>>>(pos, np, side, n, G, CTR, B.offsets, B.entries, B.capacity); \
   } while (0)
 #define PM_L(X, Y, Z)                                        \

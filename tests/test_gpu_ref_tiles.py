@@ -1,9 +1,9 @@
 """The tiled density() and integrate() of the reference-layout entry points against the oracle.
 
-Sizes at the edges of the tiles (8^3 and 16^3, one tile per axis, an odd number of them), of the two
-forms of the binning (up to 8192 tile keys and above), of the particle mapping (cubes of odd sides,
-counts that are no cube) and of the rule that takes them (the smallest counts; a grid no tile
-divides), in lattice and in random order, with particles on tile faces and on the box's edge.
+Sizes at the edges of the tiles (8^3 and 16^3, one tile per axis, an odd number of them), of the three
+forms of the binning (up to 8192 tile keys, up to 36864 from 2^21 particles on, above), of the
+particle mapping (cubes of odd sides, counts that are no cube) and of the rule that takes them (the
+smallest counts; a grid no tile divides), in lattice and in random order, with particles on tile faces and on the box's edge.
 
 Bars: the density of a cell is summed in float64 and rounded once (2^-24 relative, 1e-7 asserted).
 The gradient is eight float32 products of weights (2^-24 each) and differences of float32
@@ -43,7 +43,8 @@ def _positions(n, n_p, order, seed):
 
 DENSITY = [(8, 65536, "random"), (16, 65536, "random"), (24, 65537, "random"), (20, 65537, "random"),
            (48, 41 ** 3, "lattice"), (96, 51 ** 3, "lattice"), (128, 64 ** 3, "lattice"),
-           (256, 65536, "random"), (264, 80 ** 3, "lattice"), (272, 300001, "random"), (288, 100 ** 3, "lattice")]
+           (256, 65536, "random"), (264, 80 ** 3, "lattice"), (272, 300001, "random"), (288, 100 ** 3, "lattice"),
+           (272, 2 ** 21, "random"), (416, 2 ** 21 + 1, "random"), (432, 2 ** 21 + 1, "random")]
 
 
 @pytest.mark.parametrize("n,n_p,order", DENSITY)
@@ -59,7 +60,8 @@ def test_density(n, n_p, order):
 
 
 PUSH = [(16, 1 << 19, "random"), (24, (1 << 19) + 1, "random"), (96, 81 ** 3, "lattice"),
-        (160, 81 ** 3, "random"), (168, 83 ** 3, "lattice"), (336, 700001, "random"), (352, 81 ** 3, "lattice")]
+        (160, 81 ** 3, "random"), (168, 83 ** 3, "lattice"), (336, 700001, "random"), (352, 81 ** 3, "lattice"),
+        (336, 2 ** 21, "random"), (416, 2 ** 21 + 1, "random")]
 
 
 @pytest.mark.parametrize("n,n_p,order", PUSH)
