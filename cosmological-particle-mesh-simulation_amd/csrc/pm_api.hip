@@ -1982,6 +1982,7 @@ PM_API int pm_ensemble_run(pm_ensemble* e, double* a, const double* da, int n_st
     PM_HIP(hipMemcpyAsync(e->d_table, e->table.data(), sizeof(double) * 3 * (size_t)chunk * nm,
                           hipMemcpyHostToDevice, e->stream));
     PM_HIP(hipMemcpyAsync(e->d_step, &zero, sizeof(int), hipMemcpyHostToDevice, e->stream));
+    for (pm_sim* s : e->members) s->slot_order = false;  // from the first launch on, also if a later chunk fails
     int k = 0;
     if (use_graph)
       for (; k + e->graph_steps <= chunk; k += e->graph_steps) PM_HIP(hipGraphLaunch(e->graph, e->stream));
@@ -2001,7 +2002,6 @@ PM_API int pm_ensemble_run(pm_ensemble* e, double* a, const double* da, int n_st
     a[i] = acur[i];
     pm_sim* s = e->members[i];
     s->cur ^= done & 1;  // every step's gather switched the member's state buffer
-    if (done) s->slot_order = false;
     s->rho_valid = s->bins_valid = s->phi_valid = true;
     s->spec_valid = false;
   }
