@@ -14,6 +14,7 @@
 #include "pm_fft.h"
 #include "pm_ics.h"
 #include "pm_particles.h"
+#include "pm_pool.h"
 
 using namespace pm;
 
@@ -69,83 +70,19 @@ int ensure_init() {
 // ------------------------------------------------------------------------------------------
 // device memory
 // ------------------------------------------------------------------------------------------
-// pm_malloc / pm_free keep freed blocks for the next allocation of the same size.  Every density or
-// potential on device arrays allocates its result: hipMalloc + hipFree of a 384^3 grid cost 0.3 ms
-// a call, and the driver clears freed memory at about 35 GB/s, so a loop that allocates faster
-// than that ends up waiting for it (6.4 ms per 384^3 density, 0.5 ms of which are kernels).
-// A block is put back only when the device is idle, as hipFree would have waited too, so no stream
-// can still use it when it is handed out again.  The pool holds at most kPoolBytes (the oldest blocks
-// go first), and everything is given back before an allocation fails and before free memory is
-// reported.
-constexpr size_t kPoolBytes = (size_t)4 << 30;
-constexpr size_t kPoolGrain = (size_t)64 << 10;  // blocks are whole multiples of this
-
-constexpr int kPoolBlocks = 64;
-
-struct PoolBlock {
-  void* ptr;
-  size_t bytes;
+struct HipRuntime {
+  using Error = hipError_t;
+  static constexpr Error ok = hipSuccess, out_of_memory = hipErrorOutOfMemory, invalid = hipErrorInvalidValue;
+  static Error malloc(void** ptr, size_t bytes) { return hipMalloc(ptr, bytes); }
+  static Error free(void* ptr) { return hipFree(ptr); }
+  static Error range(void** base, size_t* bytes, void* ptr) { return hipMemGetAddressRange(base, bytes, ptr); }
+  static Error synchronize() { return hipDeviceSynchronize(); }
+  static void clear_error() { (void)hipGetLastError(); }
 };
-std::mutex g_pool_mu;
-PoolBlock g_pool[kPoolBlocks];  // free blocks, oldest first
-int g_pool_n = 0;
-size_t g_pool_bytes = 0;  // their bytes
+DevicePool<HipRuntime> g_pool;
 
-// (callers hold g_pool_mu)
-void* pool_take(int i) {
-  void* p = g_pool[i].ptr;
-  g_pool_bytes -= g_pool[i].bytes;
-  --g_pool_n;
-  for (; i < g_pool_n; ++i) g_pool[i] = g_pool[i + 1];
-  return p;
-}
-void pool_empty() {
-  std::lock_guard<std::mutex> lk(g_pool_mu);
-  while (g_pool_n) (void)hipFree(pool_take(0));
-}
-
-// hipMalloc that gives the pool's free blocks back before it fails (every allocation of the library)
-hipError_t dev_malloc(void** ptr, size_t bytes) {
-  hipError_t e = hipMalloc(ptr, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    pool_empty();
-    e = hipMalloc(ptr, bytes);
-  }
-  return e;
-}
+hipError_t dev_malloc(void** ptr, size_t bytes) { return g_pool.plain_alloc(ptr, bytes); }
 template <class T> hipError_t dev_malloc(T** ptr, size_t bytes) { return dev_malloc((void**)ptr, bytes); }
-
-hipError_t pool_alloc(void** ptr, size_t bytes) {
-  bytes = std::max((bytes + kPoolGrain - 1) / kPoolGrain, (size_t)1) * kPoolGrain;
-  {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    for (int i = g_pool_n - 1; i >= 0; --i)  // the one freed last
-      if (g_pool[i].bytes == bytes) {
-        *ptr = pool_take(i);
-        return hipSuccess;
-      }
-  }
-  return dev_malloc(ptr, bytes);
-}
-
-hipError_t pool_free(void* ptr) {
-  hipDeviceptr_t base = nullptr;
-  size_t bytes = 0;
-  // pointers that do not start an allocation go to hipFree, which names the error
-  if (hipMemGetAddressRange(&base, &bytes, ptr) != hipSuccess || base != ptr || bytes % kPoolGrain ||
-      bytes > kPoolBytes || hipDeviceSynchronize() != hipSuccess) {
-    (void)hipGetLastError();
-    return hipFree(ptr);
-  }
-  std::lock_guard<std::mutex> lk(g_pool_mu);
-  for (int i = 0; i < g_pool_n; ++i)
-    if (g_pool[i].ptr == ptr) return hipErrorInvalidValue;  // freed twice
-  while (g_pool_n == kPoolBlocks || g_pool_bytes + bytes > kPoolBytes) (void)hipFree(pool_take(0));
-  g_pool[g_pool_n++] = {ptr, bytes};
-  g_pool_bytes += bytes;
-  return hipSuccess;
-}
 
 // ------------------------------------------------------------------------------------------
 // per-size FFT tables and complex128 workspaces
@@ -396,12 +333,12 @@ PM_API int pm_supported_grid(int n_cells) { return fft_size_supported(n_cells) ?
 PM_API int pm_malloc(void** ptr, size_t bytes) {
   PM_INIT();
   if (!ptr) return fail(PM_E_INVALID, "null output pointer");
-  if (pool_alloc(ptr, bytes) != hipSuccess) return fail(PM_E_NOMEM, "hipMalloc(%zu) failed", bytes);
+  if (g_pool.alloc(ptr, bytes) != hipSuccess) return fail(PM_E_NOMEM, "hipMalloc(%zu) failed", bytes);
   return PM_OK;
 }
 PM_API int pm_free(void* ptr) {
   PM_INIT();
-  if (ptr) PM_HIP(pool_free(ptr));
+  if (ptr) PM_HIP(g_pool.free(ptr));
   return PM_OK;
 }
 PM_API int pm_memcpy_htod(void* dst, const void* src, size_t bytes) {
@@ -427,7 +364,7 @@ PM_API int pm_memset(void* dst, int value, size_t bytes) {
 PM_API int pm_mem_info(size_t* free_bytes, size_t* total_bytes) {
   PM_INIT();
   if (!free_bytes || !total_bytes) return fail(PM_E_INVALID, "null argument");
-  pool_empty();
+  g_pool.give_back();
   PM_HIP(hipMemGetInfo(free_bytes, total_bytes));
   return PM_OK;
 }
@@ -1574,7 +1511,7 @@ PM_API int pm_sim_zeldovich(pm_sim* s, const double* amp, int64_t n_amp, double 
   FftTables* t;
   if (int rc = get_tables(n, s->prec, &t)) return rc;
   double* d_amp = nullptr;
-  if (pool_alloc((void**)&d_amp, sizeof(double) * need) != hipSuccess) return fail(PM_E_NOMEM, "amplitude table allocation failed");
+  if (g_pool.alloc((void**)&d_amp, sizeof(double) * need) != hipSuccess) return fail(PM_E_NOMEM, "amplitude table allocation failed");
   hipError_t e = hipMemcpyAsync(d_amp, amp, sizeof(double) * need, hipMemcpyHostToDevice, s->stream);
   if (e == hipSuccess) {
     if (s->prec == 4)
@@ -1588,7 +1525,7 @@ PM_API int pm_sim_zeldovich(pm_sim* s, const double* amp, int64_t n_amp, double 
     if (e == hipSuccess) e = ids_identity(s->idb[s->cur], s->L, s->stream);  // the state is in slot order
   }
   hipError_t es = hipStreamSynchronize(s->stream);
-  (void)pool_free(d_amp);
+  (void)g_pool.free(d_amp);
   if (e != hipSuccess || es != hipSuccess)
     return fail(PM_E_HIP, "device initial conditions failed: %s", hipGetErrorString(e ? e : es));
   s->has_state = s->slot_order = true;
@@ -1609,7 +1546,7 @@ PM_API int pm_sim_power_spectrum(pm_sim* s, double box, int n_bins, double* k, d
   const long cells = (long)n * n * n;
   double* d = nullptr;  // [0]: sum of rho, then 3 (n_bins + 1) shell sums
   const size_t nd = 1 + 3 * (size_t)(n_bins + 1);
-  if (pool_alloc((void**)&d, sizeof(double) * nd) != hipSuccess)
+  if (g_pool.alloc((void**)&d, sizeof(double) * nd) != hipSuccess)
     return fail(PM_E_NOMEM, "spectrum scratch allocation failed");
   std::vector<double> h(nd);
   hipError_t e = hipMemsetAsync(d, 0, sizeof(double) * nd, s->stream);
@@ -1632,7 +1569,7 @@ PM_API int pm_sim_power_spectrum(pm_sim* s, double box, int n_bins, double* k, d
   }
   if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d, sizeof(double) * nd, hipMemcpyDeviceToHost, s->stream);
   hipError_t es = hipStreamSynchronize(s->stream);
-  (void)pool_free(d);
+  (void)g_pool.free(d);
   s->phi_valid = false;  // the potential buffer held the spectrum
   if (e != hipSuccess || es != hipSuccess)
     return fail(PM_E_HIP, "power spectrum failed: %s", hipGetErrorString(e ? e : es));
