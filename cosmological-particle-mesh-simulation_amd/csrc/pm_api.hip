@@ -76,7 +76,19 @@ struct HipRuntime {
   static Error malloc(void** ptr, size_t bytes) { return hipMalloc(ptr, bytes); }
   static Error free(void* ptr) { return hipFree(ptr); }
   static Error range(void** base, size_t* bytes, void* ptr) { return hipMemGetAddressRange(base, bytes, ptr); }
-  static Error synchronize() { return hipDeviceSynchronize(); }
+  static Error device_of(int* device, void* ptr) {
+    hipPointerAttribute_t at;
+    const Error e = hipPointerGetAttributes(&at, ptr);
+    if (e == ok) *device = at.device;
+    return e;
+  }
+  static int current_device() {
+    int device = 0;
+    (void)hipGetDevice(&device);
+    return device;
+  }
+  static Error set_device(int device) { return hipSetDevice(device); }
+  static Error synchronize() { return hipDeviceSynchronize(); }  // the current device
   static void clear_error() { (void)hipGetLastError(); }
 };
 DevicePool<HipRuntime> g_pool;

@@ -4,8 +4,9 @@
 // arrays allocates its result: hipMalloc + hipFree of a 384^3 grid cost 0.3 ms a call, and the driver
 // clears freed memory at about 35 GB/s, so a loop that allocates faster than that ends up waiting for it
 // (6.4 ms per 384^3 density, 0.5 ms of which are kernels).
-// A block is put back only when the device is idle, as hipFree would have waited too, so no stream can
-// still use it when it is handed out again.  The pool holds at most kPoolBytes (the oldest blocks go
+// A block is put back only when its device is idle, as hipFree would have waited too, so no stream can
+// still use it when it is handed out again, and only to callers whose current device is its own (the
+// freeing thread's current device may be another).  The pool holds at most kPoolBytes (the oldest blocks go
 // first), and everything is given back before an allocation fails and before free memory is reported.
 //
 // Api is the device runtime (a CPU stand-in in tests): Error and its values Api::ok, Api::out_of_memory
@@ -40,10 +41,11 @@ template <class Api> class DevicePool {
   Error alloc(void** ptr, size_t bytes) {
     if (bytes > kPoolBytes) return plain_alloc(ptr, bytes);  // never kept: no rounding, which could overflow
     bytes = (bytes > kPoolGrain ? (bytes + kPoolGrain - 1) / kPoolGrain : 1) * kPoolGrain;
+    const int device = Api::current_device();
     {
       std::lock_guard<std::mutex> lk(mu_);
       for (int i = n_ - 1; i >= 0; --i)  // the one freed last
-        if (blocks_[i].bytes == bytes) {
+        if (blocks_[i].bytes == bytes && blocks_[i].device == device) {
           *ptr = take(i);
           return Api::ok;
         }
@@ -54,9 +56,10 @@ template <class Api> class DevicePool {
   Error free(void* ptr) {
     void* base = nullptr;
     size_t bytes = 0;
+    int device = 0;
     // pointers that do not start an allocation go to Api::free, which names the error
     if (Api::range(&base, &bytes, ptr) != Api::ok || base != ptr || bytes % kPoolGrain || bytes > kPoolBytes ||
-        Api::synchronize() != Api::ok) {
+        Api::device_of(&device, ptr) != Api::ok || synchronize(device) != Api::ok) {
       Api::clear_error();
       return Api::free(ptr);
     }
@@ -64,7 +67,7 @@ template <class Api> class DevicePool {
     for (int i = 0; i < n_; ++i)
       if (blocks_[i].ptr == ptr) return Api::invalid;  // freed twice
     while (n_ == kPoolBlocks || bytes_ + bytes > kPoolBytes) (void)Api::free(take(0));
-    blocks_[n_++] = {ptr, bytes};
+    blocks_[n_++] = {ptr, bytes, device};
     bytes_ += bytes;
     return Api::ok;
   }
@@ -78,7 +81,18 @@ template <class Api> class DevicePool {
   struct Block {
     void* ptr;
     size_t bytes;
+    int device;
   };
+
+  // waits for everything on `device`, whichever device the thread has current
+  static Error synchronize(int device) {
+    const int current = Api::current_device();
+    if (device == current) return Api::synchronize();
+    Error e = Api::set_device(device);
+    if (e == Api::ok) e = Api::synchronize();
+    const Error back = Api::set_device(current);
+    return e != Api::ok ? e : back;
+  }
 
   // (callers hold mu_)
   void* take(int i) {

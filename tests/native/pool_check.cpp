@@ -15,7 +15,10 @@ struct FakeRuntime {
   static constexpr Error ok = 0, out_of_memory = 2, invalid = 1;
   struct Live {
     size_t bytes;
+    int device;
   };
+  static thread_local int device;
+  static thread_local std::vector<int> waited;  // devices synchronised by this thread
   static std::mutex mu;
   static std::map<char*, Live> live;
   static size_t capacity, held;
@@ -26,7 +29,7 @@ struct FakeRuntime {
     std::lock_guard<std::mutex> lk(mu);
     if (bytes > capacity - held) return out_of_memory;
     *ptr = next;
-    live[next] = {bytes};
+    live[next] = {bytes, device};
     held += bytes;
     next += (bytes / 4096 + 2) * 4096;
     return ok;
@@ -49,9 +52,26 @@ struct FakeRuntime {
     *bytes = it->second.bytes;
     return ok;
   }
-  static Error synchronize() { return ok; }
+  static Error device_of(int* d, void* ptr) {
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = live.find((char*)ptr);
+    if (it == live.end()) return invalid;
+    *d = it->second.device;
+    return ok;
+  }
+  static int current_device() { return device; }
+  static Error set_device(int d) {
+    device = d;
+    return ok;
+  }
+  static Error synchronize() {
+    waited.push_back(device);
+    return ok;
+  }
   static void clear_error() {}
 };
+thread_local int FakeRuntime::device = 0;
+thread_local std::vector<int> FakeRuntime::waited;
 std::mutex FakeRuntime::mu;
 std::map<char*, FakeRuntime::Live> FakeRuntime::live;
 size_t FakeRuntime::capacity = (size_t)64 << 30, FakeRuntime::held = 0;
@@ -109,6 +129,34 @@ int pressure() {
   return 0;
 }
 
+// a block waits for its own device, is handed out on that device alone, and the thread's current device
+// stays what it was
+int devices() {
+  Pool p;
+  void* a = get(p, MiB);  // on device 0
+  void *other = nullptr, *wrong = nullptr;
+  int at = -1, rc = 1;
+  std::vector<int> waited;
+  std::thread([&] {  // a thread whose current device is another frees it
+    FakeRuntime::device = 1;
+    rc = p.free(a);
+    waited = FakeRuntime::waited;
+    at = FakeRuntime::device;
+    wrong = get(p, MiB);
+    other = get(p, MiB);
+    (void)p.free(other);
+  }).join();
+  CHECK(rc == FakeRuntime::ok && at == 1);
+  CHECK(waited == std::vector<int>{0});
+  CHECK(wrong != a && other != a);
+  CHECK(FakeRuntime::live[(char*)wrong].device == 1);
+  CHECK(get(p, MiB) == a);                        // back on its own device, past the other's newer block
+  CHECK(p.free(a) == 0 && p.free(wrong) == 0);
+  p.give_back();                                  // both devices' blocks
+  CHECK(FakeRuntime::held == 0);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -116,6 +164,7 @@ int main(int argc, char** argv) {
   int rc = 2;
   if (!std::strcmp(name, "sizes")) rc = sizes();
   if (!std::strcmp(name, "pressure")) rc = pressure();
+  if (!std::strcmp(name, "devices")) rc = devices();
   if (rc == 0) std::printf("%s: ok\n", name);
   return rc;
 }
