@@ -169,16 +169,33 @@ int get_workspace(int n, bool need_phi, Workspace** out) {
 }
 
 // The reference-layout entry points share the workspaces of this section: each holds this mutex
-// from its first launch to its synchronisation, so calls from several threads take turns.
+// from its first launch to its synchronisation, so calls from several threads take turns.  The pool's
+// scratch buffer (the tile bins of density and integrate) is a call's own for that time.
 std::mutex g_ref_mu;
+class RefCall {
+ public:
+  ~RefCall() {
+    if (!scratch_) return;  // finished, or nothing to wait for
+    (void)hipStreamSynchronize(g_stream);
+    g_pool.scratch_done();
+  }
+  void* scratch(size_t bytes) {
+    scratch_ = true;
+    return g_pool.scratch(bytes);
+  }
+  int finish() {
+    PM_HIP(hipStreamSynchronize(g_stream));
+    if (scratch_) g_pool.scratch_done();
+    scratch_ = false;
+    return PM_OK;
+  }
 
-// Tile bins of the reference-layout density and integrate (callers hold g_ref_mu): one slab grown to
-// the largest call so far; a slab above kRefKeepBytes is given back when its call ends.
-struct RefBins {
-  void* slab = nullptr;
-  size_t bytes = 0;
-} g_ref_bins;
-constexpr size_t kRefKeepBytes = (size_t)1 << 30;
+ private:
+  std::lock_guard<std::mutex> turn_{g_ref_mu};
+  bool scratch_ = false;
+};
+
+// Tile bins of the reference-layout density and integrate.
 // Below these many particles the kernels without bins run: five short launches cost more than the
 // atomics or line fetches that the tiles save.  Whole calls at 2 cells per particle and axis, evenly
 // spread / clustered particles, in us, without and with bins:
@@ -192,27 +209,17 @@ constexpr int64_t kRefPushMin = 1 << 19;
 // tile deposit's pass over the empty cells costs more than the atomics).
 constexpr int64_t kRefTileCells = 256;
 
-// The bins for a call with n_p particles on an n^3 grid; false: the call runs without (a grid that
+// The bins for a call with n_p particles on an n^3 grid, in its scratch buffer; false: the call runs without (a grid that
 // no tile divides, fewer than `least` or too many particles, or no memory for the entries).
-bool ref_bins_begin(int64_t n_p, int64_t least, int n, TileGeom& G, Bins& B) {
+bool ref_bins(RefCall& call, int64_t n_p, int64_t least, int n, TileGeom& G, Bins& B) {
   if (n_p < least || n % 8 || kRefTileCells * n_p < (int64_t)n * n * n) return false;
   const int t = n % 16 ? 8 : 16;
   G = make_tiles(n, 4, t, t, t);
   if (!ref_tiles_ok(n_p, G)) return false;
   const size_t m = 2 * (size_t)G.ntiles, nb = (size_t)scan_blocks(G);
   const size_t words = m + 1 + (m + 1) + m + nb + 8 * (size_t)n_p;
-  RefBins& r = g_ref_bins;
-  if (words * 4 > r.bytes) {
-    if (r.slab) (void)hipFree(r.slab);
-    r = RefBins{};
-    if (dev_malloc(&r.slab, words * 4) != hipSuccess) {
-      (void)hipGetLastError();
-      r.slab = nullptr;
-      return false;
-    }
-    r.bytes = words * 4;
-  }
-  uint32_t* w = (uint32_t*)r.slab;
+  uint32_t* w = (uint32_t*)call.scratch(words * 4);
+  if (!w) return false;
   B = Bins{};
   B.counts = w;
   B.done = w + m;  // cleared together with the counts
@@ -223,18 +230,11 @@ bool ref_bins_begin(int64_t n_p, int64_t least, int n, TileGeom& G, Bins& B) {
   B.capacity = (uint32_t)(8 * (size_t)n_p);
   return true;
 }
-// the work is done (the stream is idle): a large slab goes back
-void ref_bins_end() {
-  RefBins& r = g_ref_bins;
-  if (r.bytes <= kRefKeepBytes) return;
-  (void)hipFree(r.slab);
-  r = RefBins{};
-}
 
-int density_into(const float* pos, int64_t n_p, int n, double mass, float* rho, hipStream_t st) {
+int density_into(RefCall& call, const float* pos, int64_t n_p, int n, double mass, float* rho, hipStream_t st) {
   TileGeom G;
   Bins B;
-  if (!ref_bins_begin(n_p, kRefDepositMin, n, G, B)) {
+  if (!ref_bins(call, n_p, kRefDepositMin, n, G, B)) {
     PM_HIP(ref_density(pos, n_p, n, mass, rho, st));
     return PM_OK;
   }
@@ -242,11 +242,11 @@ int density_into(const float* pos, int64_t n_p, int n, double mass, float* rho, 
   return PM_OK;
 }
 
-int integrate_into(float* pos, float* vel, int64_t n_p, int n, double a, double fa1, double da, const float* phi,
-                   hipStream_t st) {
+int integrate_into(RefCall& call, float* pos, float* vel, int64_t n_p, int n, double a, double fa1, double da,
+                   const float* phi, hipStream_t st) {
   TileGeom G;
   Bins B;
-  if (!ref_bins_begin(n_p, kRefPushMin, n, G, B)) {
+  if (!ref_bins(call, n_p, kRefPushMin, n, G, B)) {
     PM_HIP(ref_integrate(pos, vel, n_p, n, a, fa1, da, phi, st));
     return PM_OK;
   }
@@ -393,11 +393,9 @@ PM_API int pm_synchronize(void) {
 PM_API int pm_density(const float* pos, int64_t n_p, int n, double mass, float* rho) {
   PM_INIT();
   if (n <= 0 || n_p < 0 || !rho || (n_p > 0 && !pos)) return fail(PM_E_INVALID, "pm_density: bad arguments");
-  std::lock_guard<std::mutex> turn(g_ref_mu);
-  if (int rc = density_into(pos, n_p, n, mass, rho, g_stream)) return rc;
-  PM_HIP(hipStreamSynchronize(g_stream));
-  ref_bins_end();
-  return PM_OK;
+  RefCall call;
+  if (int rc = density_into(call, pos, n_p, n, mass, rho, g_stream)) return rc;
+  return call.finish();
 }
 
 PM_API int pm_fourier_grid(int n, float* g) {
@@ -541,11 +539,9 @@ PM_API int pm_integrate(float* pos, float* vel, int64_t n_p, int n, double a_val
                         const float* phi) {
   PM_INIT();
   if (n <= 0 || n_p < 0 || (n_p && (!pos || !vel || !phi))) return fail(PM_E_INVALID, "pm_integrate: bad arguments");
-  std::lock_guard<std::mutex> turn(g_ref_mu);
-  if (int rc = integrate_into(pos, vel, n_p, n, a_val, f_a1, da, phi, g_stream)) return rc;
-  PM_HIP(hipStreamSynchronize(g_stream));
-  ref_bins_end();
-  return PM_OK;
+  RefCall call;
+  if (int rc = integrate_into(call, pos, vel, n_p, n, a_val, f_a1, da, phi, g_stream)) return rc;
+  return call.finish();
 }
 
 PM_API int pm_advance_time(const float* rho, float* pos, float* vel, const float* fgrid, int64_t n_p, int n,
@@ -555,15 +551,13 @@ PM_API int pm_advance_time(const float* rho, float* pos, float* vel, const float
   if (int rc = check_grid(n)) return rc;
   if (n_p < 0 || !rho || !fgrid || (n_p && (!pos || !vel)) || a == 0.0)
     return fail(PM_E_INVALID, "pm_advance_time: bad arguments");
-  std::lock_guard<std::mutex> turn(g_ref_mu);
+  RefCall call;
   Workspace* w;
   if (int rc = get_workspace(n, true, &w)) return rc;
   if (int rc = potential_into(rho, fgrid, n, a, omega_m0, w->phi)) return rc;
   const double fa1 = f_of_a(a + da, h0, omega_lambda0, omega_k0);  // integrate.py:12 (Q1)
-  if (int rc = integrate_into(pos, vel, n_p, n, a, fa1, da, w->phi, g_stream)) return rc;
-  PM_HIP(hipStreamSynchronize(g_stream));
-  ref_bins_end();
-  return PM_OK;
+  if (int rc = integrate_into(call, pos, vel, n_p, n, a, fa1, da, w->phi, g_stream)) return rc;
+  return call.finish();
 }
 
 PM_API double pm_f(double a, double c0, double c1, double c2) { return f_of_a(a, c0, c1, c2); }

@@ -9,6 +9,9 @@
 // freeing thread's current device may be another).  The pool holds at most kPoolBytes (the oldest blocks go
 // first), and everything is given back before an allocation fails and before free memory is reported.
 //
+// A scratch buffer that calls of the library take in turns is kept the same way: grown to the largest
+// request, up to kScratchBytes between calls, and given back with the rest while no call uses it.
+//
 // Api is the device runtime (a CPU stand-in in tests): Error and its values Api::ok, Api::out_of_memory
 // and Api::invalid, and the calls used below.
 #pragma once
@@ -21,12 +24,13 @@ namespace pm {
 constexpr size_t kPoolBytes = (size_t)4 << 30;
 constexpr size_t kPoolGrain = (size_t)64 << 10;  // blocks are whole multiples of this
 constexpr int kPoolBlocks = 64;
+constexpr size_t kScratchBytes = (size_t)1 << 30;
 
 template <class Api> class DevicePool {
  public:
   using Error = typename Api::Error;
 
-  // Api::malloc that gives the pool's free blocks back before it fails (every allocation of the library)
+  // Api::malloc that gives back what the pool keeps before it fails (every allocation of the library)
   Error plain_alloc(void** ptr, size_t bytes) {
     Error e = Api::malloc(ptr, bytes);
     if (e == Api::out_of_memory) {
@@ -72,9 +76,31 @@ template <class Api> class DevicePool {
     return Api::ok;
   }
 
+  // The scratch buffer with room for `bytes` (null: no memory); the caller's until scratch_done().  One
+  // caller at a time.
+  void* scratch(size_t bytes) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      scratch_busy_ = true;
+    }
+    if (bytes > scratch_bytes_) {
+      drop_scratch();
+      if (plain_alloc(&scratch_, bytes) == Api::ok) scratch_bytes_ = bytes;
+      else scratch_ = nullptr;
+    }
+    return scratch_;
+  }
+  // no work uses the scratch buffer any more
+  void scratch_done() {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (scratch_bytes_ > kScratchBytes) drop_scratch();
+    scratch_busy_ = false;
+  }
+
   void give_back() {
     std::lock_guard<std::mutex> lk(mu_);
     while (n_) (void)Api::free(take(0));
+    if (!scratch_busy_) drop_scratch();
   }
 
  private:
@@ -103,10 +129,20 @@ template <class Api> class DevicePool {
     return p;
   }
 
+  // (by the scratch buffer's user, or with mu_ held while it has none)
+  void drop_scratch() {
+    if (scratch_) (void)Api::free(scratch_);
+    scratch_ = nullptr;
+    scratch_bytes_ = 0;
+  }
+
   std::mutex mu_;
   Block blocks_[kPoolBlocks];  // free blocks, oldest first
   int n_ = 0;
   size_t bytes_ = 0;  // their bytes
+  void* scratch_ = nullptr;
+  size_t scratch_bytes_ = 0;
+  bool scratch_busy_ = false;
 };
 
 }  // namespace pm

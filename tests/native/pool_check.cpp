@@ -157,6 +157,34 @@ int devices() {
   return 0;
 }
 
+// the scratch buffer grows to the largest request, is kept between calls up to its bound, and goes back
+// under pressure and on request unless a call uses it
+int scratch() {
+  Pool p;
+  FakeRuntime::capacity = 4 * GiB;
+  void* a = p.scratch(300 * MiB);
+  CHECK(a && FakeRuntime::held == 300 * MiB);
+  p.give_back();
+  CHECK(FakeRuntime::held == 300 * MiB);           // in use
+  void* big = nullptr;
+  CHECK(p.plain_alloc(&big, 4 * GiB) != FakeRuntime::ok && FakeRuntime::held == 300 * MiB);
+  p.scratch_done();
+  CHECK(p.scratch(200 * MiB) == a);                // kept, large enough
+  p.scratch_done();
+  CHECK(p.plain_alloc(&big, 4 * GiB) == FakeRuntime::ok && FakeRuntime::held == 4 * GiB);  // idle: given back
+  CHECK(p.scratch(MiB) == nullptr);                // no memory: the call does without
+  p.scratch_done();
+  CHECK(FakeRuntime::free(big) == FakeRuntime::ok);
+  CHECK(p.scratch(2 * GiB) && FakeRuntime::held == 2 * GiB);
+  p.scratch_done();
+  CHECK(FakeRuntime::held == 0);                   // above the bound: not kept
+  CHECK(p.scratch(500 * MiB) && p.scratch(600 * MiB) && FakeRuntime::held == 600 * MiB);
+  p.scratch_done();
+  p.give_back();
+  CHECK(FakeRuntime::held == 0);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -165,6 +193,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(name, "sizes")) rc = sizes();
   if (!std::strcmp(name, "pressure")) rc = pressure();
   if (!std::strcmp(name, "devices")) rc = devices();
+  if (!std::strcmp(name, "scratch")) rc = scratch();
   if (rc == 0) std::printf("%s: ok\n", name);
   return rc;
 }

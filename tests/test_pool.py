@@ -22,7 +22,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["sizes", "pressure", "devices"])
+@pytest.mark.parametrize("case", ["sizes", "pressure", "devices", "scratch"])
 def test_pool(check, case):
     p = subprocess.run([str(check), case], capture_output=True, text=True, timeout=60)
     assert p.returncode == 0 and p.stdout == f"{case}: ok\n", p.stdout + p.stderr
