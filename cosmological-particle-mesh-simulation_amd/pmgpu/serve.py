@@ -120,18 +120,26 @@ def _prepare(req: SimRequest):
     return ic.amplitude_table(p), scale, ic.velocity_factor(p)
 
 
-def _start(req: SimRequest, prepared) -> PMSim:
+def _new_sim(req: SimRequest, prepared, tiles=None) -> PMSim:
+    """The request's sim with its device initial conditions and first density, in tiles of the
+    given shape (None: the grid's default)."""
     amp, scale, vfac = prepared
     sim = PMSim(req.n_cells, req.n_parts, 32, omega_m0=req.om, omega_lambda0=req.ol,
                 omega_k0=req.ok, h0=req.h)
     try:
-        sim.set_tiles(*ensemble_tiles(req.n_cells))   # joining keeps the bins and the density
+        if tiles:
+            sim.set_tiles(*tiles)
         sim.zeldovich(amp, scale, vfac, seed=req.seed)
         sim.deposit()
     except Exception:
         sim.close()
         raise
     return sim
+
+
+def _start(req: SimRequest, prepared) -> PMSim:
+    """A sim to be served, in its ensemble's tile shape: joining then keeps the bins and the density."""
+    return _new_sim(req, prepared, ensemble_tiles(req.n_cells))
 
 
 class PMServer:
@@ -399,12 +407,11 @@ class PMServer:
 def run_alone(req: SimRequest, keep_state: bool = False, tiles=None) -> SimResult:
     """One request by itself: its own sim, device initial conditions, the graph-replayed
     step loop and the final power spectrum (the one-at-a-time way of serving).  ``tiles``
-    fixes the tile shape (``ensemble_tiles(n_cells)`` makes the run use the served kernels)."""
+    fixes the tile shape (``ensemble_tiles(n_cells)`` makes the run use the served kernels; by default
+    the grid's own)."""
     t0 = time.perf_counter()
-    sim = _start(req, _prepare(req))
+    sim = _new_sim(req, _prepare(req), tiles)
     try:
-        if tiles:
-            sim.set_tiles(*tiles)
         n = req.loop_steps
         a = sim.run(req.a_init, req.da, n)
         k, pk, _ = sim.power_spectrum(req.box)
