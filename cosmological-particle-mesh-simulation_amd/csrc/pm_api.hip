@@ -209,36 +209,47 @@ constexpr int64_t kRefPushMin = 1 << 19;
 // tile deposit's pass over the empty cells costs more than the atomics).
 constexpr int64_t kRefTileCells = 256;
 
-// The bins for a call with n_p particles on an n^3 grid, in its scratch buffer; false: the call runs without (a grid that
-// no tile divides, fewer than `least` or too many particles, or no memory for the entries).
-bool ref_bins(RefCall& call, int64_t n_p, int64_t least, int n, TileGeom& G, Bins& B) {
-  if (n_p < least || n % 8 || kRefTileCells * n_p < (int64_t)n * n * n) return false;
+// The bins for a call with n_p particles on an n^3 grid, in its scratch buffer, with halo keys (the
+// deposit) or without; false: the call runs without (a grid that no tile divides, too few or too many
+// particles, or no memory for the entries).
+bool ref_bins(RefCall& call, int64_t n_p, int n, bool halo, TileGeom& G, Bins& B, RefPieces& P) {
+  if (n % 8 || kRefTileCells * n_p < (int64_t)n * n * n) return false;
+  if (n_p < (halo ? kRefDepositMin : kRefPushMin)) return false;
   const int t = n % 16 ? 8 : 16;
   G = make_tiles(n, 4, t, t, t);
   if (!ref_tiles_ok(n_p, G)) return false;
+  P = ref_pieces(n_p, G, halo);
   const size_t m = 2 * (size_t)G.ntiles, nb = (size_t)scan_blocks(G);
-  const size_t words = m + 1 + (m + 1) + m + nb + 8 * (size_t)n_p;
-  uint32_t* w = (uint32_t*)call.scratch(words * 4);
-  if (!w) return false;
   B = Bins{};
-  B.counts = w;
-  B.done = w + m;  // cleared together with the counts
+  B.capacity = (uint32_t)((halo ? 8 : 1) * (size_t)n_p);
+  // counters, counts and ticket (cleared together), offsets, cursors, sums, entries; 8-byte values; tickets
+  const size_t head = kRefCounters + m + 1 + (m + 1) + m + nb + B.capacity, pad = head & 1;
+  const size_t list = 2 * (size_t)P.max, part = 2 * (size_t)P.parts * P.cells;
+  uint32_t* w = (uint32_t*)call.scratch(4 * (head + pad + list + part + P.parts));
+  if (!w) return false;
+  P.n = w;
+  B.counts = P.n + kRefCounters;
+  B.done = B.counts + m;
   B.offsets = B.done + 1;
   B.cursors = B.offsets + m + 1;
   B.block_sums = B.cursors + m;
   B.entries = B.block_sums + nb;
-  B.capacity = (uint32_t)(8 * (size_t)n_p);
+  w += head + pad;
+  P.list = (uint2*)w;
+  P.part = part ? (double*)(w + list) : nullptr;
+  P.tickets = w + list + part;
   return true;
 }
 
 int density_into(RefCall& call, const float* pos, int64_t n_p, int n, double mass, float* rho, hipStream_t st) {
   TileGeom G;
   Bins B;
-  if (!ref_bins(call, n_p, kRefDepositMin, n, G, B)) {
+  RefPieces P;
+  if (!ref_bins(call, n_p, n, true, G, B, P)) {
     PM_HIP(ref_density(pos, n_p, n, mass, rho, st));
     return PM_OK;
   }
-  PM_HIP(ref_density_tiles(pos, n_p, n, mass, rho, G, B, st));
+  PM_HIP(ref_density_tiles(pos, n_p, n, mass, rho, G, B, P, st));
   return PM_OK;
 }
 
@@ -246,11 +257,12 @@ int integrate_into(RefCall& call, float* pos, float* vel, int64_t n_p, int n, do
                    const float* phi, hipStream_t st) {
   TileGeom G;
   Bins B;
-  if (!ref_bins(call, n_p, kRefPushMin, n, G, B)) {
+  RefPieces P;
+  if (!ref_bins(call, n_p, n, false, G, B, P)) {
     PM_HIP(ref_integrate(pos, vel, n_p, n, a, fa1, da, phi, st));
     return PM_OK;
   }
-  PM_HIP(ref_integrate_tiles(pos, vel, n_p, n, a, fa1, da, phi, G, B, st));
+  PM_HIP(ref_integrate_tiles(pos, vel, n_p, n, a, fa1, da, phi, G, B, P, st));
   return PM_OK;
 }
 

@@ -223,14 +223,40 @@ hipError_t gkd_tiles(const PState<R>& in, const PState<R>& out, const R* phi, do
 
 // ---- reference-layout kernels (absolute float32 positions, reference order) ------------------
 hipError_t ref_density(const float* pos, long np, int n, double mass, float* rho, hipStream_t st);
+// Dense tiles of a reference-layout call.  A key (own or halo segment of a tile) of at least `dense`
+// entries is cut into pieces of `per` (64 longer ones at most): the tile's block takes the first,
+// the others are listed by the scan and shared out to further blocks.  The deposit's blocks of one tile
+// leave FP64 partial sums; the last to do so (ticket) adds them up, about 1 us each, and rounds.
+// per is 4096 entries, four batches of a deposit block (about 15 us, what the meeting of a tile's blocks
+// costs), or N_p / 512: at most 256 tiles have own pieces, and a block's share of a call stays small.
+// dense is 2 per, and on 64 tiles or more twice their mean: evenly filled, they keep the chip busy by
+// themselves (density of 2.1 M random particles on 96^3, whole / in pieces of 4096: 248 / 336 us; on
+// 48^3, 27 tiles, 650 / 429).  Keys beyond the room for partial sums run whole.
+struct RefPieces {
+  uint32_t per = 0, dense = 0;
+  uint32_t max = 0;             // capacity of the list: all keys' count / per
+  uint32_t parts = 0;           // partial sums (deposit; the push needs none)
+  uint32_t cells = 0;           // values of each
+  uint32_t* n = nullptr;        // kRefCounters: pieces listed, partial sums taken
+  uint2* list = nullptr;        // {key, piece}
+  double* part = nullptr;
+  uint32_t* tickets = nullptr;  // one per partial sum (a tile uses that of its first)
+};
+constexpr long kRefPiece = 4096, kRefPieces = 512;
+constexpr int kRefTilePieces = 64;  // of one key
+constexpr int kRefCounters = 32;  // (two are used: the counts that follow start a cache line)
+RefPieces ref_pieces(long np, const TileGeom& G, bool halo);  // sizes; the caller sets the pointers
+
 // The same through tile bins (own + halo entries of the tiles G, at most 8 N_p): the sums of a cell
-// meet in FP64 in LDS.  B: entries of 8 N_p words, the scan's ticket right after the 2*ntiles counts;
-// ref_tiles_ok tells whether G and N_p allow it.
+// meet in FP64 in LDS.  B: entries of 8 N_p words; the pieces' counters right before the 2*ntiles counts,
+// the scan's ticket right after.  ref_tiles_ok tells whether G and N_p allow it.
 bool ref_tiles_ok(long np, const TileGeom& G);
+int cube_side(long np);  // s where np = s^3, otherwise 0
 hipError_t ref_density_tiles(const float* pos, long np, int n, double mass, float* rho, const TileGeom& G,
-                             const Bins& B, hipStream_t st);
+                             const Bins& B, const RefPieces& P, hipStream_t st);
 hipError_t ref_integrate_tiles(float* pos, float* vel, long np, int n, double a, double fa1, double da,
-                               const float* phi, const TileGeom& G, const Bins& B, hipStream_t st);
+                               const float* phi, const TileGeom& G, const Bins& B, const RefPieces& P,
+                               hipStream_t st);
 hipError_t ref_cell_centers(const float* pos, long np, int n, int64_t* cells, hipStream_t st);
 hipError_t ref_weights(const int64_t* cells, const float* pos, long np, float* t, hipStream_t st);
 hipError_t ref_sweep(const int64_t* cells, float* xd, float* vd, const float* t, const float* phi, long np,

@@ -539,11 +539,42 @@ __global__ __launch_bounds__(kT) void k_scan_reduce_spine(const uint32_t* __rest
   scan_reduce_spine_body(counts, m, bsum, nb, done, blockIdx.x, sh, &last, far);
 }
 
-// offsets of one chunk whose counts start at `start` entries; PER counts per thread
-template <int PER, int NT>
+// pieces of a key beyond its first
+__device__ __forceinline__ uint32_t pieces_of(const RefPieces& P, bool dense, uint32_t count) {
+  return dense ? min(count / P.per, (uint32_t)kRefTilePieces) - 1 : 0u;
+}
+// entries of piece i of the key with entries [beg, end); i = 0: what the tile's own block takes
+__device__ __forceinline__ void piece_range(const RefPieces& P, bool dense, uint32_t i, uint32_t& beg, uint32_t& end) {
+  if (!dense) return;
+  const uint32_t last = pieces_of(P, true, end - beg), len = (end - beg) / (last + 1);
+  beg += i * len;
+  if (i < last) end = beg + len;
+}
+
+// Lists the pieces of a dense key of a reference-layout call (see RefPieces) and returns what the scan
+// leaves in its count: 1 + the first of its partial sums (1 where pieces need none), 0 for a key that one
+// block takes whole.
+__device__ __forceinline__ uint32_t list_pieces(const RefPieces& P, uint32_t key, uint32_t count) {
+  if (count < P.dense) return 0u;
+  const uint32_t extra = pieces_of(P, true, count);
+  uint32_t slot = 0u;
+  if (P.part) {
+    slot = atomicAdd(&P.n[1], extra + 1);
+    if (slot + extra >= P.parts) return 0u;
+    P.tickets[slot] = 0u;
+  }
+  const uint32_t at = atomicAdd(&P.n[0], extra);
+  for (uint32_t i = 0; i < extra && at + i < P.max; ++i) P.list[at + i] = make_uint2(key, i + 1);
+  return slot + 1;
+}
+
+// offsets of one chunk whose counts start at `start` entries; PER counts per thread.  PIECES: a
+// reference-layout call, whose counts become list_pieces (otherwise they are cleared for the next step).
+template <int PER, int NT, bool PIECES = false>
 __device__ __forceinline__ void scan_chunk(uint32_t* __restrict__ counts, long m, long first, uint32_t start,
                                            uint32_t* __restrict__ offsets, uint32_t* __restrict__ cursors,
-                                           uint32_t* sh, uint32_t* __restrict__ far, uint32_t* __restrict__ old) {
+                                           uint32_t* sh, uint32_t* __restrict__ far, uint32_t* __restrict__ old,
+                                           const RefPieces* P = nullptr) {
   const long base = first + (long)threadIdx.x * PER;
   uint32_t v[PER], near[PER];
   uint32_t sum = 0;
@@ -562,7 +593,7 @@ __device__ __forceinline__ void scan_chunk(uint32_t* __restrict__ counts, long m
     if (j < m) {
       if (old && j <= m / 2) old[j] = offsets[j];  // own offsets of the binning being replaced
       offsets[j] = run;
-      counts[j] = 0u;
+      counts[j] = PIECES ? list_pieces(*P, (uint32_t)j, v[i]) : 0u;
       cursors[j] = far ? near[i] : 0u;
       if (far) far[j] = 0u;
     }
@@ -571,12 +602,13 @@ __device__ __forceinline__ void scan_chunk(uint32_t* __restrict__ counts, long m
   }
 }
 
+template <bool PIECES = false>
 __device__ __forceinline__ void scan_apply_body(uint32_t* __restrict__ counts, long m,
                                                 const uint32_t* __restrict__ bsum, uint32_t* __restrict__ offsets,
                                                 uint32_t* __restrict__ cursors, long blk, uint32_t* sh,
                                                 uint32_t* __restrict__ far = nullptr,
-                                                uint32_t* __restrict__ old = nullptr) {
-  scan_chunk<kScanPer, kT>(counts, m, blk * (long)kScanChunk, bsum[blk], offsets, cursors, sh, far, old);
+                                                uint32_t* __restrict__ old = nullptr, const RefPieces* P = nullptr) {
+  scan_chunk<kScanPer, kT, PIECES>(counts, m, blk * (long)kScanChunk, bsum[blk], offsets, cursors, sh, far, old, P);
 }
 
 // The whole scan in one block, for up to 2 counts per thread: one launch instead of two on small grids
@@ -584,21 +616,22 @@ __device__ __forceinline__ void scan_apply_body(uint32_t* __restrict__ counts, l
 // With 8 per thread (192^3, 6912 counts) one CU's scattered accesses take 22 us against 4.8 + 4.7.
 constexpr int kScanSmallT = 1024;
 constexpr long kScanSmall = 2 * kScanSmallT;
-template <int PER>
+template <int PER, bool PIECES>
 __global__ __launch_bounds__(kScanSmallT) void k_scan_small(uint32_t* __restrict__ counts, long m,
                                                             uint32_t* __restrict__ offsets,
                                                             uint32_t* __restrict__ cursors, uint32_t* __restrict__ far,
-                                                            uint32_t* __restrict__ old) {
+                                                            uint32_t* __restrict__ old, RefPieces P) {
   __shared__ uint32_t sh[kScanSmallT / 64];
-  scan_chunk<PER, kScanSmallT>(counts, m, 0, 0u, offsets, cursors, sh, far, old);
+  scan_chunk<PER, kScanSmallT, PIECES>(counts, m, 0, 0u, offsets, cursors, sh, far, old, &P);
 }
 
+template <bool PIECES>
 __global__ __launch_bounds__(kT) void k_scan_apply(uint32_t* __restrict__ counts, long m,
                                                    const uint32_t* __restrict__ bsum, uint32_t* __restrict__ offsets,
                                                    uint32_t* __restrict__ cursors, uint32_t* __restrict__ far,
-                                                   uint32_t* __restrict__ old) {
+                                                   uint32_t* __restrict__ old, RefPieces P) {
   __shared__ uint32_t sh[kT];
-  scan_apply_body(counts, m, bsum, offsets, cursors, blockIdx.x, sh, far, old);
+  scan_apply_body<PIECES>(counts, m, bsum, offsets, cursors, blockIdx.x, sh, far, old, &P);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -615,15 +648,15 @@ template <int TX, int TY, int TZ> constexpr int deposit_lds_cells() { return (TX
 // by the host so that the whole mass fits in 62 bits); integer adds are associative, so the
 // cell values do not depend on the order the atomics land in.
 // ABS: s holds absolute positions and there are no ids (only L.n and L.np are read).
+// Sums of the tile's cells over the own entries [ob, ob + n_own) and the halo entries [hb, hb +
+// total - n_own), read as one list of `total`; ends with a barrier.
 template <typename R, int TX, int TY, int TZ, bool DET = false, bool ABS = false>
-__device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint32_t* __restrict__ id,
-                                             R* __restrict__ rho, double mass, const Lattice& L, const TileGeom& G,
-                                             const uint32_t* __restrict__ offsets,
-                                             const uint32_t* __restrict__ entries, uint32_t capacity, int tile,
-                                             double* acc, uint32_t* __restrict__ health, double fix = 0.0) {
+__device__ __forceinline__ void deposit_sums(const R* __restrict__ s, const uint32_t* __restrict__ id, double mass,
+                                             const Lattice& L, const TileGeom& G,
+                                             const uint32_t* __restrict__ entries, int tile, uint32_t ob,
+                                             uint32_t n_own, uint32_t hb, uint32_t total, double* acc,
+                                             uint32_t* __restrict__ health, double fix = 0.0) {
   unsigned long long* iacc = reinterpret_cast<unsigned long long*>(acc);
-  constexpr int CELLS = TX * TY * TZ;
-  static_assert(CELLS % kT == 0, "tile must hold a multiple of the block size");
   constexpr int E = 4;
   constexpr int PX = TX + 3, PLANE = PX * TY, PADDED = deposit_lds_cells<TX, TY, TZ>();
   const int tix = tile % G.ntx, tiy = (tile / G.ntx) % G.nty, tiz = tile / (G.ntx * G.nty);
@@ -631,11 +664,6 @@ __device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint
   const int T[3] = {TX, TY, TZ};
   const int n = L.n;
   const long np = L.np;
-  // own entries [ob, oe) and halo entries [hb, he), read as one list of n_own + n_halo
-  const uint32_t nt = (uint32_t)G.ntiles;
-  const uint32_t oe = min(offsets[tile + 1], capacity), ob = min(offsets[tile], oe);
-  const uint32_t he = min(offsets[nt + tile + 1], capacity), hb = min(offsets[nt + tile], he);
-  const uint32_t n_own = oe - ob, total = n_own + (he - hb);
   uint32_t sl[E], pid[E];
   R sv[E][3];
   auto load = [&](uint32_t base) {
@@ -719,15 +747,44 @@ __device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint
   if (bad && health) atomicAdd(&health[PM_HEALTH_BINS], bad);
   if (nonfinite && health) atomicAdd(&health[PM_HEALTH_NONFINITE], nonfinite);
   __syncthreads();
+}
+
+// f(i, index in the grid, index in the accumulator) for every cell i of the tile, U per thread unrolled
+template <int TX, int TY, int TZ, int U = TX * TY * TZ / kT, class F>
+__device__ __forceinline__ void each_tile_cell(int n, const TileGeom& G, int tile, F&& f) {
+  constexpr int CELLS = TX * TY * TZ, PX = TX + 3, PLANE = PX * TY;
+  static_assert(CELLS % kT == 0, "tile must hold a multiple of the block size");
+  const int tix = tile % G.ntx, tiy = (tile / G.ntx) % G.nty, tiz = tile / (G.ntx * G.nty);
   const size_t nn = (size_t)n;
-#pragma unroll
+#pragma unroll U
   for (int i0 = 0; i0 < CELLS / kT; ++i0) {
     const int i = i0 * kT + threadIdx.x;
     const int rx = i % TX, ry = (i / TX) % TY, rz = i / (TX * TY);
-    const int li = rz * PLANE + ry * PX + rx;
-    rho[((size_t)(o0[2] + rz) * nn + (o0[1] + ry)) * nn + (o0[0] + rx)] =
-        DET ? R((double)iacc[li] / fix) : R(acc[li]);
+    f(i, ((size_t)(tiz * TZ + rz) * nn + (tiy * TY + ry)) * nn + (tix * TX + rx), rz * PLANE + ry * PX + rx);
   }
+}
+
+// own entries [ob, oe) and halo entries [hb, he) of a tile
+__device__ __forceinline__ void tile_entries(const uint32_t* __restrict__ offsets, uint32_t capacity, uint32_t nt,
+                                             int tile, uint32_t& ob, uint32_t& oe, uint32_t& hb, uint32_t& he) {
+  oe = min(offsets[tile + 1], capacity), ob = min(offsets[tile], oe);
+  he = min(offsets[nt + tile + 1], capacity), hb = min(offsets[nt + tile], he);
+}
+
+template <typename R, int TX, int TY, int TZ, bool DET = false>
+__device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint32_t* __restrict__ id,
+                                             R* __restrict__ rho, double mass, const Lattice& L, const TileGeom& G,
+                                             const uint32_t* __restrict__ offsets,
+                                             const uint32_t* __restrict__ entries, uint32_t capacity, int tile,
+                                             double* acc, uint32_t* __restrict__ health, double fix = 0.0) {
+  uint32_t ob, oe, hb, he;
+  tile_entries(offsets, capacity, (uint32_t)G.ntiles, tile, ob, oe, hb, he);
+  deposit_sums<R, TX, TY, TZ, DET>(s, id, mass, L, G, entries, tile, ob, oe - ob, hb, oe - ob + (he - hb), acc, health,
+                                   fix);
+  const unsigned long long* iacc = reinterpret_cast<const unsigned long long*>(acc);
+  each_tile_cell<TX, TY, TZ>(L.n, G, tile, [&](int, size_t at, int li) {
+    rho[at] = DET ? R((double)iacc[li] / fix) : R(acc[li]);
+  });
 }
 
 // step: when set, the last kernel of a table-driven step advances the table's step counter
@@ -1427,7 +1484,7 @@ inline long ref_blocks(long np, int side) {
 // block -> tile with z fastest: the tiles of one (x, y) column hold the particles of the same
 // cache lines of the reference's arrays, so they share them in one L2
 __device__ __forceinline__ int ref_tile(const TileGeom& G) {
-  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const int b = xcd_block((int)blockIdx.x, G.ntiles);
   const int tz = b % G.ntz, r = b / G.ntz, tx = r % G.ntx, ty = r / G.ntx;
   return (tz * G.nty + ty) * G.ntx + tx;
 }
@@ -1632,29 +1689,99 @@ __global__ __launch_bounds__(kT) void k_ref_bin(const float* __restrict__ pos, l
   }
 }
 
+// Dense tiles.  The first ntiles blocks of the deposit and the push take a tile each, the first piece of a
+// key that has pieces; `extra` further ones take the listed pieces in turn.  Without pieces a block's time
+// is its tile's entries (density / integrate): 2.1 M particles on 16^3, one tile, 7.35 / 10.1 -> 0.41 / 0.28 ms;
+// half of 2.1 M in one clump on 256^3 2.92 / 4.08 -> 0.43 / 0.49.
+// dense: 1 + first partial sum of a key with pieces, else 0 (the scan leaves it in the counts)
 template <int TX, int TY, int TZ>
 __global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ pos, float* __restrict__ rho, double mass,
                                                     Lattice L, TileGeom G, const uint32_t* __restrict__ offsets,
-                                                    const uint32_t* __restrict__ entries, uint32_t capacity) {
+                                                    const uint32_t* __restrict__ entries, uint32_t capacity,
+                                                    const uint32_t* __restrict__ dense, RefPieces P, uint32_t extra) {
+  constexpr int CELLS = TX * TY * TZ;
   __shared__ double acc[deposit_lds_cells<TX, TY, TZ>()];
-  deposit_body<float, TX, TY, TZ, false, true>(pos, nullptr, rho, mass, L, G, offsets, entries, capacity, ref_tile(G),
-                                               acc, nullptr);
+  __shared__ uint32_t last;
+  const uint32_t nt = (uint32_t)G.ntiles;
+  const bool piece = blockIdx.x >= nt;
+  uint32_t x = piece ? blockIdx.x - nt : blockIdx.x;
+  const uint32_t n = piece ? min(P.n[0], P.max) : 0u;
+  if (piece && x >= n) return;
+  int tile = piece ? 0 : ref_tile(G);
+  do {
+    bool halo = false;
+    uint32_t i = 0u;
+    if (piece) {
+      const uint2 e = P.list[x];
+      halo = e.x >= nt;
+      tile = (int)(halo ? e.x - nt : e.x);
+      i = e.y;
+    }
+    uint32_t ob, oe, hb, he;
+    tile_entries(offsets, capacity, nt, tile, ob, oe, hb, he);
+    const uint32_t d_own = dense[tile], d_halo = dense[nt + tile];
+    const uint32_t p_own = pieces_of(P, d_own, oe - ob), p_halo = pieces_of(P, d_halo, he - hb);
+    piece_range(P, d_own, halo ? 0 : i, ob, oe);
+    piece_range(P, d_halo, halo ? i : 0, hb, he);
+    if (piece) {
+      if (halo) oe = ob;
+      else he = hb;
+    }
+    deposit_sums<float, TX, TY, TZ, false, true>(pos, nullptr, mass, L, G, entries, tile, ob, oe - ob, hb,
+                                                 oe - ob + (he - hb), acc, nullptr);
+    if (!(d_own | d_halo)) {
+      each_tile_cell<TX, TY, TZ>(L.n, G, tile, [&](int, size_t at, int li) { rho[at] = float(acc[li]); });
+      break;
+    }
+    // each block of the tile leaves its sums; the one that leaves them last adds them all up in FP64 and
+    // rounds.  The tile's own block uses the first place of the own (or else the halo) key.
+    const uint32_t s_own = d_own - 1, s_halo = d_halo - 1;
+    const uint32_t place = halo ? s_halo + i : (d_own ? s_own : s_halo) + i;
+    double* mine = P.part + (size_t)place * CELLS;
+    each_tile_cell<TX, TY, TZ, 4>(L.n, G, tile, [&](int c, size_t, int li) { mine[c] = acc[li]; });
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0)
+      last = atomicAdd(&P.tickets[d_own ? s_own : s_halo], 1u) == p_own + p_halo ? 1u : 0u;
+    __syncthreads();
+    if (last) {
+      __threadfence();
+      auto add = [&](uint32_t first, uint32_t count) {
+        for (uint32_t k = first; k < first + count; ++k) {
+          if (k == place) continue;  // (in the LDS sums already)
+          const double* part = gmem(P.part) + (size_t)k * CELLS;
+          constexpr int U = CELLS / kT < 8 ? CELLS / kT : 8;
+          for (int q = 0; q < CELLS / kT; q += U) {
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = part[(q + u) * kT + threadIdx.x];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int c = (q + u) * kT + threadIdx.x, rx = c % TX, ry = (c / TX) % TY, rz = c / (TX * TY);
+              acc[(rz * TY + ry) * (TX + 3) + rx] += v[u];
+            }
+          }
+        }
+      };
+      if (d_own) add(s_own, 1 + p_own);
+      if (d_halo) add(d_own ? s_halo + 1 : s_halo, d_own ? p_halo : 1 + p_halo);
+      each_tile_cell<TX, TY, TZ, 4>(L.n, G, tile, [&](int, size_t at, int li) { rho[at] = float(acc[li]); });
+    }
+    __syncthreads();  // (the accumulator and `last` are used again)
+    x += extra;
+  } while (piece && x < n);
 }
 
-// integrate.py:15-97 for the particles of one tile, in place: the potential of the tile and its
+// integrate.py:15-97 for entries [beg, end) of one tile, in place: the potential of the tile and its
 // -1/+2 stencil margin staged in LDS, the arithmetic of k_ref_integrate term by term
+template <int TX, int TY, int TZ> constexpr int push_box_cells() { return (TX + 3) * (TY + 3) * (TZ + 3); }
 template <int TX, int TY, int TZ>
-__global__ __launch_bounds__(kT) void k_ref_push(float* __restrict__ pos, float* __restrict__ vel, long np, int n,
-                                                 double a, double fa1, double da, const float* __restrict__ phi,
-                                                 TileGeom G, const uint32_t* __restrict__ offsets,
-                                                 const uint32_t* __restrict__ entries, uint32_t capacity) {
+__device__ __forceinline__ void push_entries(float* __restrict__ pos, float* __restrict__ vel, long np, int n, double a,
+                                             double fa1, double da, const float* __restrict__ phi, const TileGeom& G,
+                                             const uint32_t* __restrict__ entries, int tile, uint32_t beg,
+                                             uint32_t end, float* box) {
   constexpr int BX = TX + 3, BY = TY + 3, BZ = TZ + 3, PLANE = BX * BY;
   constexpr int NW = kT / 64, PL = (PLANE + 63) / 64, ZIT = (BZ + NW - 1) / NW, E = 2;
-  __shared__ float box[BX * BY * BZ];
-  const int tile = ref_tile(G);
-  uint32_t beg, end;
-  tile_range(offsets, capacity, tile, beg, end);
-  if (beg == end) return;
   const int tix = tile % G.ntx, tiy = (tile / G.ntx) % G.nty, tiz = tile / (G.ntx * G.nty);
   const int o0[3] = {tix * TX, tiy * TY, tiz * TZ};
   const size_t nn = (size_t)n;
@@ -1756,6 +1883,36 @@ __global__ __launch_bounds__(kT) void k_ref_push(float* __restrict__ pos, float*
   }
 }
 
+template <int TX, int TY, int TZ>
+__global__ __launch_bounds__(kT) void k_ref_push(float* __restrict__ pos, float* __restrict__ vel, long np, int n,
+                                                 double a, double fa1, double da, const float* __restrict__ phi,
+                                                 TileGeom G, const uint32_t* __restrict__ offsets,
+                                                 const uint32_t* __restrict__ entries, uint32_t capacity,
+                                                 const uint32_t* __restrict__ dense, RefPieces P, uint32_t extra) {
+  __shared__ float box[push_box_cells<TX, TY, TZ>()];
+  const uint32_t nt = (uint32_t)G.ntiles;
+  const bool piece = blockIdx.x >= nt;
+  uint32_t x = piece ? blockIdx.x - nt : blockIdx.x;
+  const uint32_t n_pieces = piece ? min(P.n[0], P.max) : 0u;
+  if (piece && x >= n_pieces) return;
+  int tile = piece ? 0 : ref_tile(G);
+  do {
+    uint32_t i = 0u;
+    if (piece) {
+      const uint2 e = P.list[x];
+      tile = (int)e.x;  // (own keys only)
+      i = e.y;
+    }
+    uint32_t beg, end;
+    tile_range(offsets, capacity, tile, beg, end);
+    piece_range(P, dense[tile], i, beg, end);
+    if (beg == end) return;
+    push_entries<TX, TY, TZ>(pos, vel, np, n, a, fa1, da, phi, G, entries, tile, beg, end, box);
+    __syncthreads();  // (the box is used again)
+    x += extra;
+  } while (piece && x < n_pieces);
+}
+
 }  // namespace
 
 
@@ -1854,6 +2011,16 @@ hipError_t bins_count(const PState<R>& p, const Lattice& L, const TileGeom& G, c
   return hipGetLastError();
 }
 
+template <bool PIECES>
+static hipError_t launch_scan_small(long m, const Bins& B, uint32_t* far, uint32_t* old, const RefPieces& P,
+                                    hipStream_t st) {
+  if (m <= kScanSmallT)
+    k_scan_small<1, PIECES><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old, P);
+  else
+    k_scan_small<2, PIECES><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old, P);
+  return hipGetLastError();
+}
+
 hipError_t bins_scan(const TileGeom& G, const Bins& B, hipStream_t st, bool after_gather) {
   const long m = 2L * G.ntiles;
   const int nb = scan_blocks(G);
@@ -1861,12 +2028,10 @@ hipError_t bins_scan(const TileGeom& G, const Bins& B, hipStream_t st, bool afte
   uint32_t* far = ts ? B.counts + ts_far_at(G.ntiles) : nullptr;
   uint32_t* old = ts ? B.counts + ts_old_at(G.ntiles) : nullptr;
   if (m <= kScanSmall) {
-    if (m <= kScanSmallT) k_scan_small<1><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old);
-    else k_scan_small<2><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old);
-    return hipGetLastError();
+    return launch_scan_small<false>(m, B, far, old, RefPieces{}, st);
   }
   k_scan_reduce_spine<<<nb, kT, 0, st>>>(B.counts, m, B.block_sums, nb, B.done, far);
-  k_scan_apply<<<nb, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, far, old);
+  k_scan_apply<false><<<nb, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, far, old, RefPieces{});
   return hipGetLastError();
 }
 
@@ -1897,20 +2062,25 @@ hipError_t bins_scatter(const PState<R>& p, const Lattice& L, const TileGeom& G,
   return hipGetLastError();
 }
 
+int cube_side(long np) {
+  const long s = std::lround(std::cbrt((double)np));
+  return s * s * s == np ? (int)s : 0;
+}
+
 bool ref_tiles_ok(long np, const TileGeom& G) { return G.ntiles > 0 && 8 * (uint64_t)np < (uint64_t)UINT32_MAX; }
 
 // bins the particles of one call (own entries, and the halo ones the deposit needs)
 static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const TileGeom& G, const Bins& B,
-                          hipStream_t st) {
-  int side = (int)std::lround(std::cbrt((double)np));
-  if ((long)side * side * side != np) side = 0;
+                          const RefPieces& P, hipStream_t st) {
+  const int side = cube_side(np);
   const long nb = ref_blocks(np, side);
   const long nbl = (nb + kRefP - 1) / kRefP;
+  const long m = 2L * G.ntiles;
   const int keys = (halo ? 2 : 1) * G.ntiles;
   const bool lds = keys <= kRefLdsKeys, wide = !lds && side == 0 && np >= kRefWideMin && keys <= kRefWideKeys;
   const unsigned nbw = (unsigned)((np + kRefWideT * kRefWideP - 1) / (kRefWideT * kRefWideP));
-  // the counts and the scan's ticket after them (never captured: the callers synchronise)
-  if (hipError_t e = hipMemsetAsync(B.counts, 0, (2 * (size_t)G.ntiles + 1) * sizeof(uint32_t), st)) return e;
+  // the pieces' counters, the counts and the scan's ticket (never captured: the callers synchronise)
+  if (hipError_t e = hipMemsetAsync(P.n, 0, (kRefCounters + (size_t)m + 1) * sizeof(uint32_t), st)) return e;
 #define PM_ONE(X, Y, Z, HALO, SCATTER, CTR)                                                                          \
   do {                                                                                                               \
     if (lds)                                                                                                         \
@@ -1934,7 +2104,13 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
   } while (0)
   PM_REF_TILE_DISPATCH(G, PM_L);
 #undef PM_L
-  if (hipError_t e = bins_scan(G, B, st)) return e;
+  if (m <= kScanSmall) {
+    if (hipError_t e = launch_scan_small<true>(m, B, nullptr, nullptr, P, st)) return e;
+  } else {
+    const int nbs = scan_blocks(G);
+    k_scan_reduce_spine<<<nbs, kT, 0, st>>>(B.counts, m, B.block_sums, nbs, B.done, nullptr);
+    k_scan_apply<true><<<nbs, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, nullptr, nullptr, P);
+  }
 #define PM_L(X, Y, Z)                                        \
   do {                                                       \
     if (halo) PM_ONE(X, Y, Z, true, true, B.cursors);        \
@@ -1946,25 +2122,44 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
   return hipGetLastError();
 }
 
+RefPieces ref_pieces(long np, const TileGeom& G, bool halo) {
+  RefPieces P;
+  P.per = (uint32_t)std::max(kRefPiece, (np + kRefPieces - 1) / kRefPieces);
+  P.dense = (uint32_t)std::max(2L * P.per, G.ntiles >= 64 ? 2 * np / G.ntiles : 0L);
+  P.max = (uint32_t)((halo ? 8 : 1) * np / P.per);  // no more: a piece beyond a tile's first holds >= per entries
+  if (halo) {
+    P.parts = std::min(P.max, (uint32_t)(2 * kRefPieces));
+    P.cells = (uint32_t)(G.tx * G.ty * G.tz);
+  }
+  return P;
+}
+
+// blocks that take the listed pieces: two per CU at most
+static unsigned piece_blocks(const RefPieces& P) { return std::min(P.max, 512u); }
+
 hipError_t ref_density_tiles(const float* pos, long np, int n, double mass, float* rho, const TileGeom& G,
-                             const Bins& B, hipStream_t st) {
-  if (hipError_t e = ref_bin(pos, np, n, true, G, B, st)) return e;
+                             const Bins& B, const RefPieces& P, hipStream_t st) {
+  if (hipError_t e = ref_bin(pos, np, n, true, G, B, P, st)) return e;
   Lattice L{};
   L.n = n;
   L.np = np;
-#define PM_L(X, Y, Z) \
-  k_ref_deposit<X, Y, Z><<<G.ntiles, kT, 0, st>>>(pos, rho, mass, L, G, B.offsets, B.entries, B.capacity)
+  const unsigned extra = piece_blocks(P);
+#define PM_L(X, Y, Z)                                                                                               \
+  k_ref_deposit<X, Y, Z><<<G.ntiles + extra, kT, 0, st>>>(pos, rho, mass, L, G, B.offsets, B.entries, B.capacity, \
+                                                          B.counts, P, extra)
   PM_REF_TILE_DISPATCH(G, PM_L);
 #undef PM_L
   return hipGetLastError();
 }
 
 hipError_t ref_integrate_tiles(float* pos, float* vel, long np, int n, double a, double fa1, double da,
-                               const float* phi, const TileGeom& G, const Bins& B, hipStream_t st) {
-  if (hipError_t e = ref_bin(pos, np, n, false, G, B, st)) return e;
-#define PM_L(X, Y, Z)                                                                                     \
-  k_ref_push<X, Y, Z><<<G.ntiles, kT, 0, st>>>(pos, vel, np, n, a, fa1, da, phi, G, B.offsets, B.entries, \
-                                               B.capacity)
+                               const float* phi, const TileGeom& G, const Bins& B, const RefPieces& P,
+                               hipStream_t st) {
+  if (hipError_t e = ref_bin(pos, np, n, false, G, B, P, st)) return e;
+  const unsigned extra = piece_blocks(P);
+#define PM_L(X, Y, Z)                                                                                            \
+  k_ref_push<X, Y, Z><<<G.ntiles + extra, kT, 0, st>>>(pos, vel, np, n, a, fa1, da, phi, G, B.offsets, B.entries, \
+                                                       B.capacity, B.counts, P, extra)
   PM_REF_TILE_DISPATCH(G, PM_L);
 #undef PM_L
   return hipGetLastError();
