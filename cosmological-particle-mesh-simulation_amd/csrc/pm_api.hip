@@ -205,6 +205,14 @@ class RefCall {
 //              2.1 M: 295 / 308 and 102 / 132
 constexpr int64_t kRefDepositMin = 1 << 16;
 constexpr int64_t kRefPushMin = 1 << 19;
+// The push without bins reads the potential out of order and the particles in order, with bins the other
+// way round, so the line is where the potential leaves the nearer caches.  In lattice order (N_p a cube)
+// that pays from 96^3 on (531 k, without / with: 80^3 60 / 80, 96^3 74 / 68, 128^3 88 / 59), in no order
+// from 144^3 on (2.1 M: 96^3 304 / 459, 128^3 480 / 504, 144^3 603 / 518, 256^3 935 / 632).
+constexpr int kRefPushLattice = 96, kRefPushAny = 144;
+bool push_bins_pay(int64_t n_p, int n) {
+  return n_p >= kRefPushMin && n >= (cube_side(n_p) ? kRefPushLattice : kRefPushAny);
+}
 // ... and above this many cells per particle (a 16^3 tile then holds fewer than 16 particles, and the
 // tile deposit's pass over the empty cells costs more than the atomics).
 constexpr int64_t kRefTileCells = 256;
@@ -214,8 +222,11 @@ constexpr int64_t kRefTileCells = 256;
 // particles, or no memory for the entries).
 bool ref_bins(RefCall& call, int64_t n_p, int n, bool halo, TileGeom& G, Bins& B, RefPieces& P) {
   if (n % 8 || kRefTileCells * n_p < (int64_t)n * n * n) return false;
-  if (n_p < (halo ? kRefDepositMin : kRefPushMin)) return false;
-  const int t = n % 16 ? 8 : 16;
+  if (halo ? n_p < kRefDepositMin : !push_bins_pay(n_p, n)) return false;
+  // 16^3 tiles, on small grids 8^3: a few tiles of 16^3 leave most of the chip idle (density of 190 k / 2.1 M
+  // random particles, us: 32^3 99 -> 77 / 372 -> 454, 48^3 88 -> 62 / 429 -> 272, 64^3 73 -> 62 / 416 -> 284,
+  // 80^3 62 -> 67; without bins 92 / 815, 93 / 848, 91 / 821, 92)
+  const int t = n % 16 || (n > 16 && n < 80) ? 8 : 16;
   G = make_tiles(n, 4, t, t, t);
   if (!ref_tiles_ok(n_p, G)) return false;
   P = ref_pieces(n_p, G, halo);
