@@ -220,6 +220,10 @@ constexpr int64_t kRefTileCells = 256;
 // The bins for a call with n_p particles on an n^3 grid, in its scratch buffer, with halo keys (the
 // deposit) or without; false: the call runs without (a grid that no tile divides, too few or too many
 // particles, or no memory for the entries).
+// The bins stay within what is kept between calls: a buffer that is allocated and freed by every call waits
+// for the driver, which clears freed memory at about 35 GB/s (134 M particles on 1024^3, 4.3 GB: 121 ms
+// a call, kernels 19).  A deposit of more than 33 M particles gets the rest of that for its entries,
+// 1.2 a particle as a rule, and runs without bins if its binning counts more.
 bool ref_bins(RefCall& call, int64_t n_p, int n, bool halo, TileGeom& G, Bins& B, RefPieces& P) {
   if (n % 8 || kRefTileCells * n_p < (int64_t)n * n * n) return false;
   if (halo ? n_p < kRefDepositMin : !push_bins_pay(n_p, n)) return false;
@@ -232,10 +236,12 @@ bool ref_bins(RefCall& call, int64_t n_p, int n, bool halo, TileGeom& G, Bins& B
   P = ref_pieces(n_p, G, halo);
   const size_t m = 2 * (size_t)G.ntiles, nb = (size_t)scan_blocks(G);
   B = Bins{};
-  B.capacity = (uint32_t)((halo ? 8 : 1) * (size_t)n_p);
   // counters, counts and ticket (cleared together), offsets, cursors, sums, entries; 8-byte values; tickets
-  const size_t head = kRefCounters + m + 1 + (m + 1) + m + nb + B.capacity, pad = head & 1;
   const size_t list = 2 * (size_t)P.max, part = 2 * (size_t)P.parts * P.cells;
+  const size_t fixed = kRefCounters + m + 1 + (m + 1) + m + nb, rest = fixed + 1 + list + part + P.parts;
+  if (rest + n_p > kScratchBytes / 4) return false;
+  B.capacity = (uint32_t)std::min((halo ? 8 : 1) * (size_t)n_p, kScratchBytes / 4 - rest);
+  const size_t head = fixed + B.capacity, pad = head & 1;
   uint32_t* w = (uint32_t*)call.scratch(4 * (head + pad + list + part + P.parts));
   if (!w) return false;
   P.n = w;
@@ -256,11 +262,9 @@ int density_into(RefCall& call, const float* pos, int64_t n_p, int n, double mas
   TileGeom G;
   Bins B;
   RefPieces P;
-  if (!ref_bins(call, n_p, n, true, G, B, P)) {
-    PM_HIP(ref_density(pos, n_p, n, mass, rho, st));
-    return PM_OK;
-  }
-  PM_HIP(ref_density_tiles(pos, n_p, n, mass, rho, G, B, P, st));
+  bool done = false;
+  if (ref_bins(call, n_p, n, true, G, B, P)) PM_HIP(ref_density_tiles(pos, n_p, n, mass, rho, G, B, P, st, done));
+  if (!done) PM_HIP(ref_density(pos, n_p, n, mass, rho, st));
   return PM_OK;
 }
 

@@ -249,11 +249,12 @@ RefPieces ref_pieces(long np, const TileGeom& G, bool halo);  // sizes; the call
 
 // The same through tile bins (own + halo entries of the tiles G, at most 8 N_p): the sums of a cell
 // meet in FP64 in LDS.  B: entries of 8 N_p words; the pieces' counters right before the 2*ntiles counts,
-// the scan's ticket right after.  ref_tiles_ok tells whether G and N_p allow it.
+// the scan's ticket right after.  Where B has fewer the deposit waits for the count of its entries and, if they do
+// not fit, does nothing (done = false).  ref_tiles_ok tells whether G and N_p allow it.
 bool ref_tiles_ok(long np, const TileGeom& G);
 int cube_side(long np);  // s where np = s^3, otherwise 0
 hipError_t ref_density_tiles(const float* pos, long np, int n, double mass, float* rho, const TileGeom& G,
-                             const Bins& B, const RefPieces& P, hipStream_t st);
+                             const Bins& B, const RefPieces& P, hipStream_t st, bool& done);
 hipError_t ref_integrate_tiles(float* pos, float* vel, long np, int n, double a, double fa1, double da,
                                const float* phi, const TileGeom& G, const Bins& B, const RefPieces& P,
                                hipStream_t st);

@@ -2141,7 +2141,7 @@ bool ref_tiles_ok(long np, const TileGeom& G) { return G.ntiles > 0 && 8 * (uint
 
 // bins the particles of one call (own entries, and the halo ones the deposit needs)
 static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const TileGeom& G, const Bins& B,
-                          const RefPieces& P, hipStream_t st) {
+                          const RefPieces& P, hipStream_t st, bool& fits) {
   const int side = cube_side(np);
   const long nb = ref_blocks(np, side);
   const long nbl = (nb + kRefP - 1) / kRefP;
@@ -2181,6 +2181,14 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
     k_scan_reduce_spine<<<nbs, kT, 0, st>>>(B.counts, m, B.block_sums, nbs, B.done, nullptr);
     k_scan_apply<true><<<nbs, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, nullptr, nullptr, P);
   }
+  fits = true;
+  if (B.capacity < (halo ? 8 : 1) * (uint64_t)np) {
+    uint32_t total = 0;
+    if (hipError_t e = hipMemcpyAsync(&total, B.offsets + m, sizeof total, hipMemcpyDeviceToHost, st)) return e;
+    if (hipError_t e = hipStreamSynchronize(st)) return e;
+    fits = total <= B.capacity;
+    if (!fits) return hipSuccess;
+  }
 #define PM_L(X, Y, Z)                                        \
   do {                                                       \
     if (halo) PM_ONE(X, Y, Z, true, true, B.cursors);        \
@@ -2208,8 +2216,9 @@ RefPieces ref_pieces(long np, const TileGeom& G, bool halo) {
 static unsigned piece_blocks(const RefPieces& P) { return std::min(P.max, 512u); }
 
 hipError_t ref_density_tiles(const float* pos, long np, int n, double mass, float* rho, const TileGeom& G,
-                             const Bins& B, const RefPieces& P, hipStream_t st) {
-  if (hipError_t e = ref_bin(pos, np, n, true, G, B, P, st)) return e;
+                             const Bins& B, const RefPieces& P, hipStream_t st, bool& done) {
+  if (hipError_t e = ref_bin(pos, np, n, true, G, B, P, st, done)) return e;
+  if (!done) return hipSuccess;
   Lattice L{};
   L.n = n;
   L.np = np;
@@ -2225,7 +2234,8 @@ hipError_t ref_density_tiles(const float* pos, long np, int n, double mass, floa
 hipError_t ref_integrate_tiles(float* pos, float* vel, long np, int n, double a, double fa1, double da,
                                const float* phi, const TileGeom& G, const Bins& B, const RefPieces& P,
                                hipStream_t st) {
-  if (hipError_t e = ref_bin(pos, np, n, false, G, B, P, st)) return e;
+  bool fits;  // (own entries: always)
+  if (hipError_t e = ref_bin(pos, np, n, false, G, B, P, st, fits)) return e;
   const unsigned extra = piece_blocks(P);
 #define PM_L(X, Y, Z)                                                                                            \
   k_ref_push<X, Y, Z><<<G.ntiles + extra, kT, 0, st>>>(pos, vel, np, n, a, fa1, da, phi, G, B.offsets, B.entries, \
