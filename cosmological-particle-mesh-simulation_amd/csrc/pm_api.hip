@@ -1108,9 +1108,9 @@ PM_API int pm_sim_set_tiles(pm_sim* s, int tx, int ty, int tz) {
   if (!s) return fail(PM_E_INVALID, "null sim");
   if ((tx || ty || tz) && !tile_shape_supported(tx, ty, tz))
     return fail(PM_E_UNSUPPORTED, "tile shape %dx%dx%d is not instantiated", tx, ty, tz);
-  if (s->ens) {  // 16^3 and the default both leave a member in its ensemble's shape
-    if (!(tx == 16 && ty == 16 && tz == 16) && (tx || ty || tz))
-      return fail(PM_E_STATE, "ensemble members keep the ensemble's tile shape");
+  if (s->ens) {  // a member keeps its ensemble's shape: that one, the default and 16^3 leave it there
+    const bool own = tx == s->G.tx && ty == s->G.ty && tz == s->G.tz, cube = tx == 16 && ty == 16 && tz == 16;
+    if (!own && !cube && (tx || ty || tz)) return fail(PM_E_STATE, "ensemble members keep the ensemble's tile shape");
     return PM_OK;
   }
   return sim_use_tiles(s, make_tiles(s->L.n, s->prec, tx, ty, tz));
