@@ -2139,6 +2139,17 @@ int cube_side(long np) {
 
 bool ref_tiles_ok(long np, const TileGeom& G) { return G.ntiles > 0 && 8 * (uint64_t)np < (uint64_t)UINT32_MAX; }
 
+// blocks above 64 KiB of LDS have to be allowed; without, the form without a table takes over
+template <int X, int Y, int Z, bool HALO, bool SCATTER> static bool wide_allowed() {
+  static const bool ok = [] {
+    const hipError_t e = hipFuncSetAttribute((const void*)k_ref_bin_wide<X, Y, Z, HALO, SCATTER>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kRefWideKeys * sizeof(uint32_t));
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  }();
+  return ok;
+}
+
 // bins the particles of one call (own entries, and the halo ones the deposit needs)
 static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const TileGeom& G, const Bins& B,
                           const RefPieces& P, hipStream_t st, bool& fits) {
@@ -2156,15 +2167,10 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
     if (lds)                                                                                                         \
       k_ref_bin_lds<X, Y, Z, HALO, SCATTER>                                                                          \
           <<<nbl, kT, keys * sizeof(uint32_t), st>>>(pos, np, side, n, G, CTR, B.offsets, B.entries, B.capacity);    \
-    else if (wide) {                                                                                                 \
-      /* (blocks above 64 KiB of LDS have to be allowed) */                                                          \
-      static const hipError_t allowed =                                                                              \
-          hipFuncSetAttribute((const void*)k_ref_bin_wide<X, Y, Z, HALO, SCATTER>,                                   \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, kRefWideKeys * sizeof(uint32_t));          \
-      if (allowed != hipSuccess) return allowed;                                                                     \
+    else if (wide && wide_allowed<X, Y, Z, HALO, SCATTER>())                                                         \
       k_ref_bin_wide<X, Y, Z, HALO, SCATTER><<<nbw, kRefWideT, keys * sizeof(uint32_t), st>>>(                       \
           pos, np, n, G, CTR, B.offsets, B.entries, B.capacity);                                                     \
-    } else                                                                                                           \
+    else                                                                                                             \
       k_ref_bin<X, Y, Z, HALO, SCATTER><<<nb, kT, 0, st>>>(pos, np, side, n, G, CTR, B.offsets, B.entries, B.capacity); \
   } while (0)
 #define PM_L(X, Y, Z)                                        \
