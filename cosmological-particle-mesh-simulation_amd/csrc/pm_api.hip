@@ -1113,7 +1113,7 @@ PM_API int pm_sim_set_tiles(pm_sim* s, int tx, int ty, int tz) {
     if (!own && !cube && (tx || ty || tz)) return fail(PM_E_STATE, "ensemble members keep the ensemble's tile shape");
     return PM_OK;
   }
-  return sim_use_tiles(s, make_tiles(s->L.n, s->prec, tx, ty, tz));
+  return sim_use_tiles(s, make_tiles(s->L.n, s->prec, tx, ty, tz, s->L.np));
 }
 
 PM_API int pm_sim_set_pencils(pm_sim* s, int y_fwd, int z, int y_inv) {
@@ -1210,7 +1210,7 @@ PM_API int pm_sim_create(int n_cells, int n_parts_side, int precision, unsigned 
       dev_malloc(&s->grid[1], nn * nn * nn * pr) != hipSuccess || dev_malloc(&s->Q, nn * nn * 2 * pr) != hipSuccess ||
       (has_edge(n_cells, s->prec) && dev_malloc(&s->edge, edge_bytes(n_cells)) != hipSuccess))
     return cleanup(fail(PM_E_NOMEM, "device allocation of %zu bytes failed", sim_bytes(n_cells, n_parts_side, s->prec)));
-  s->G = make_tiles(n_cells, s->prec);
+  s->G = make_tiles(n_cells, s->prec, 0, 0, 0, s->L.np);
   const TileGeom gmax = max_tiles(n_cells, s->prec);
   const size_t m = 2 * (size_t)gmax.ntiles;
   if (8 * (size_t)s->L.np >= (size_t)UINT32_MAX) return cleanup(fail(PM_E_INVALID, "too many particles (N_PARTS > 812)"));

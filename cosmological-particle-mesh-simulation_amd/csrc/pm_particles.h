@@ -152,8 +152,9 @@ struct Bins {
 // among those that divide the grid.
 #define PM_TILE_SHAPES(X) X(16, 16, 16) X(32, 16, 8) X(32, 8, 8) X(16, 16, 8) X(64, 8, 8) X(8, 8, 8)
 bool tile_shape_supported(int tx, int ty, int tz);
-// tiles of shape (tx, ty, tz) on an n^3 grid (all 0: the default for n); ntiles = 0 if unusable
-TileGeom make_tiles(int n, int prec_bytes, int tx = 0, int ty = 0, int tz = 0);
+// tiles of shape (tx, ty, tz) on an n^3 grid (all 0: the default for n and np particles, np = 0: the
+// usual number); ntiles = 0 if unusable
+TileGeom make_tiles(int n, int prec_bytes, int tx = 0, int ty = 0, int tz = 0, long np = 0);
 std::vector<TileGeom> tile_candidates(int n, int prec_bytes);
 int scan_blocks(const TileGeom& g);
 // tiles of at least this many cells, 4 or more per axis, take the tile scatter after a gather

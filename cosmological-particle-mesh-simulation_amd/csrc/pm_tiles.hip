@@ -1994,9 +1994,8 @@ bool tile_shape_supported(int tx, int ty, int tz) {
   return false;
 }
 
-TileGeom make_tiles(int n, int prec_bytes, int tx, int ty, int tz) {
+TileGeom make_tiles(int n, int prec_bytes, int tx, int ty, int tz, long np) {
   TileGeom g{};
-  (void)prec_bytes;  // the same line in both precisions
   if (tx == 0 && ty == 0 && tz == 0) {
     // Default shape by grid size: small grids need many tiles to occupy the chip, large ones tiles
     // whose potential box and accumulator leave the most blocks per CU and whose rows are whole cache
@@ -2016,6 +2015,15 @@ TileGeom make_tiles(int n, int prec_bytes, int tx, int ty, int tz) {
     tx = wide ? 32 : flat ? 16 : 8;
     ty = !wide && flat ? 16 : 8;
     tz = 8;
+    // Few particles (more than 16 cells each, twice the usual 8) leave the time to the tiles themselves, so
+    // fewer of them, 16^3, on the smallest grids and the largest FP32 ones: steps in the shape above and in
+    // 16^3, us, with n/8, n/4 and n/3 particles a side:
+    //    64^3  54 / 32   36 / 32   38 / 33
+    //   768^3  5921 / 5817   6013 / 5954   6259 / 6188;  1024^3  13.05 / 12.66 ms   13.29 / 13.06   13.78 / 13.50
+    // but 128^3  57.4 / 59.0   57.5 / 60.1   58.6 / 61.0;  512^3  1432 / 1410   1474 / 1480   1512 / 1533;
+    // FP64 512^3  2889 / 2946   2961 / 3024   3042 / 3076.
+    const bool few = np > 0 && 16 * np < (long)n * n * n && n % 16 == 0;
+    if (few && (n < 96 || (prec_bytes == 4 && n > 512))) tx = ty = tz = 16;
   }
   if (!tile_shape_supported(tx, ty, tz) || n % tx || n % ty || n % tz) return g;  // not usable
   g.tx = tx;

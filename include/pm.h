@@ -159,7 +159,7 @@ PM_API int pm_sim_sync(pm_sim* sim);
 /* bytes of device memory held by the sim                                                     */
 PM_API int pm_sim_footprint(int n_cells, int n_parts_side, int precision, size_t* bytes);
 /* Eulerian tile shape of the deposit / gather kernels (cells per tile along x, y, z; all 0 =
- * the default for the grid size).  Instantiated shapes: 16x16x16, 32x16x8, 32x8x8, 16x16x8, 64x8x8, 8x8x8;
+ * the default for the grid size and particle count).  Instantiated shapes: 16x16x16, 32x16x8, 32x8x8, 16x16x8, 64x8x8, 8x8x8;
  * each must divide N_CELLS.  A member of an ensemble keeps the ensemble's shape (32x8x8 from N_CELLS =
  * 128 on, 16x16x8 below): asked for that shape, the default or 16x16x16 it stays there (PM_OK), any
  * other is refused (PM_E_STATE).  No reference counterpart (the reference scatters per particle,
