@@ -1641,6 +1641,7 @@ struct pm_ensemble {
   long fft_base[2][BS_COUNT] = {}, fft_count[2][BS_COUNT] = {};
   int fft_lds[2][BS_COUNT] = {};
   long total[BS_COUNT] = {};
+  long ts_particles = 0;  // of the members with the tile scatter
   bool timing = false;
   std::vector<PendingEvent> pending;
   double stage_ms[ST_COUNT] = {};
@@ -1675,6 +1676,7 @@ void ens_describe(pm_ensemble* e) {
   D.table = e->d_table;
   D.step = e->d_step;
   for (int st = 0; st < BS_COUNT; ++st) D.off[st][0] = 0;
+  e->ts_particles = 0;
   for (int c = 0; c < 2; ++c)
     for (int st = 0; st < BS_COUNT; ++st) {
       e->fft_base[c][st] = -1;
@@ -1731,6 +1733,7 @@ void ens_describe(pm_ensemble* e) {
     blocks[BS_SCAN] = m.scan_nb;
     blocks[BS_SCATTER] = m.tile_scatter ? 0 : batch_scatter_blocks(s->L.np);
     blocks[BS_TILE_SCATTER] = m.tile_scatter ? s->G.ntiles : 0;
+    if (m.tile_scatter) e->ts_particles += s->L.np;
     const int c = batch_class(n);
     for (int st = 0; st < BS_COUNT; ++st) {
       D.off[st][i + 1] = D.off[st][i] + blocks[st];
@@ -1789,7 +1792,7 @@ int ens_step(pm_ensemble* e) {
   {
     EnsTimer t(e, ST_BIN);
     PM_HIP(batch_scan(d, e->total[BS_SCAN], (int)e->members.size(), st));
-    PM_HIP(batch_scatter(d, e->total[BS_SCATTER], e->total[BS_TILE_SCATTER], st));
+    PM_HIP(batch_scatter(d, e->total[BS_SCATTER], e->total[BS_TILE_SCATTER], e->ts_particles, st));
   }
   {
     EnsTimer t(e, ST_DEPOSIT);

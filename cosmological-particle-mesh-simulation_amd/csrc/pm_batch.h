@@ -110,7 +110,8 @@ hipError_t batch_gkd(const BatchDesc* d, long total, long total_ts, hipStream_t 
 hipError_t batch_scan(const BatchDesc* d, long total, int n_members, hipStream_t st);
 // total: blocks of the particle-parallel scatter (BS_SCATTER), total_tiles: wavefronts of the
 // tile scatter (BS_TILE_SCATTER)
-hipError_t batch_scatter(const BatchDesc* d, long total, long total_tiles, hipStream_t st);
+// tile_particles: particles of the members with the tile scatter
+hipError_t batch_scatter(const BatchDesc* d, long total, long total_tiles, long tile_particles, hipStream_t st);
 hipError_t batch_deposit(const BatchDesc* d, long total, hipStream_t st);
 long batch_scatter_blocks(long np);
 
