@@ -609,13 +609,12 @@ __device__ __forceinline__ void scan_chunk(uint32_t* __restrict__ counts, long m
   }
 }
 
-template <bool PIECES = false>
 __device__ __forceinline__ void scan_apply_body(uint32_t* __restrict__ counts, long m,
                                                 const uint32_t* __restrict__ bsum, uint32_t* __restrict__ offsets,
                                                 uint32_t* __restrict__ cursors, long blk, uint32_t* sh,
                                                 uint32_t* __restrict__ far = nullptr,
-                                                uint32_t* __restrict__ old = nullptr, const RefPieces* P = nullptr) {
-  scan_chunk<kScanPer, kT, PIECES>(counts, m, blk * (long)kScanChunk, bsum[blk], offsets, cursors, sh, far, old, P);
+                                                uint32_t* __restrict__ old = nullptr) {
+  scan_chunk<kScanPer, kT>(counts, m, blk * (long)kScanChunk, bsum[blk], offsets, cursors, sh, far, old);
 }
 
 // The whole scan in one block, for up to 2 counts per thread: one launch instead of two on small grids
@@ -623,22 +622,39 @@ __device__ __forceinline__ void scan_apply_body(uint32_t* __restrict__ counts, l
 // With 8 per thread (192^3, 6912 counts) one CU's scattered accesses take 22 us against 4.8 + 4.7.
 constexpr int kScanSmallT = 1024;
 constexpr long kScanSmall = 2 * kScanSmallT;
-template <int PER, bool PIECES>
+template <int PER>
 __global__ __launch_bounds__(kScanSmallT) void k_scan_small(uint32_t* __restrict__ counts, long m,
                                                             uint32_t* __restrict__ offsets,
                                                             uint32_t* __restrict__ cursors, uint32_t* __restrict__ far,
-                                                            uint32_t* __restrict__ old, RefPieces P) {
+                                                            uint32_t* __restrict__ old) {
   __shared__ uint32_t sh[kScanSmallT / 64];
-  scan_chunk<PER, kScanSmallT, PIECES>(counts, m, 0, 0u, offsets, cursors, sh, far, old, &P);
+  scan_chunk<PER, kScanSmallT>(counts, m, 0, 0u, offsets, cursors, sh, far, old);
 }
 
-template <bool PIECES>
 __global__ __launch_bounds__(kT) void k_scan_apply(uint32_t* __restrict__ counts, long m,
                                                    const uint32_t* __restrict__ bsum, uint32_t* __restrict__ offsets,
                                                    uint32_t* __restrict__ cursors, uint32_t* __restrict__ far,
-                                                   uint32_t* __restrict__ old, RefPieces P) {
+                                                   uint32_t* __restrict__ old) {
   __shared__ uint32_t sh[kT];
-  scan_apply_body<PIECES>(counts, m, bsum, offsets, cursors, blockIdx.x, sh, far, old, &P);
+  scan_apply_body(counts, m, bsum, offsets, cursors, blockIdx.x, sh, far, old);
+}
+
+// the same for a reference-layout call, which lists the pieces of its dense keys
+template <int PER>
+__global__ __launch_bounds__(kScanSmallT) void k_ref_scan_small(uint32_t* __restrict__ counts, long m,
+                                                                uint32_t* __restrict__ offsets,
+                                                                uint32_t* __restrict__ cursors, RefPieces P) {
+  __shared__ uint32_t sh[kScanSmallT / 64];
+  scan_chunk<PER, kScanSmallT, true>(counts, m, 0, 0u, offsets, cursors, sh, nullptr, nullptr, &P);
+}
+
+__global__ __launch_bounds__(kT) void k_ref_scan_apply(uint32_t* __restrict__ counts, long m,
+                                                       const uint32_t* __restrict__ bsum,
+                                                       uint32_t* __restrict__ offsets,
+                                                       uint32_t* __restrict__ cursors, RefPieces P) {
+  __shared__ uint32_t sh[kT];
+  scan_chunk<kScanPer, kT, true>(counts, m, blockIdx.x * (long)kScanChunk, bsum[blockIdx.x], offsets, cursors, sh,
+                                 nullptr, nullptr, &P);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -660,13 +676,13 @@ template <int TX, int TY, int TZ> constexpr int deposit_lds_cells() { return (TX
 template <typename R, int TX, int TY, int TZ, bool DET = false, bool ABS = false>
 __device__ __forceinline__ void deposit_sums(const R* __restrict__ s, const uint32_t* __restrict__ id, double mass,
                                              const Lattice& L, const TileGeom& G,
-                                             const uint32_t* __restrict__ entries, int tile, uint32_t ob,
+                                             const uint32_t* __restrict__ entries, const int (&tc)[3], uint32_t ob,
                                              uint32_t n_own, uint32_t hb, uint32_t total, double* acc,
                                              uint32_t* __restrict__ health, double fix = 0.0) {
   unsigned long long* iacc = reinterpret_cast<unsigned long long*>(acc);
   constexpr int E = 4;
   constexpr int PX = TX + 3, PLANE = PX * TY, PADDED = deposit_lds_cells<TX, TY, TZ>();
-  const int tix = tile % G.ntx, tiy = (tile / G.ntx) % G.nty, tiz = tile / (G.ntx * G.nty);
+  const int tix = tc[0], tiy = tc[1], tiz = tc[2];
   const int o0[3] = {tix * TX, tiy * TY, tiz * TZ};
   const int T[3] = {TX, TY, TZ};
   const int n = L.n;
@@ -758,16 +774,15 @@ __device__ __forceinline__ void deposit_sums(const R* __restrict__ s, const uint
 
 // f(i, index in the grid, index in the accumulator) for every cell i of the tile, U per thread unrolled
 template <int TX, int TY, int TZ, int U = TX * TY * TZ / kT, class F>
-__device__ __forceinline__ void each_tile_cell(int n, const TileGeom& G, int tile, F&& f) {
+__device__ __forceinline__ void each_tile_cell(int n, const int (&tc)[3], F&& f) {
   constexpr int CELLS = TX * TY * TZ, PX = TX + 3, PLANE = PX * TY;
   static_assert(CELLS % kT == 0, "tile must hold a multiple of the block size");
-  const int tix = tile % G.ntx, tiy = (tile / G.ntx) % G.nty, tiz = tile / (G.ntx * G.nty);
   const size_t nn = (size_t)n;
 #pragma unroll U
   for (int i0 = 0; i0 < CELLS / kT; ++i0) {
     const int i = i0 * kT + threadIdx.x;
     const int rx = i % TX, ry = (i / TX) % TY, rz = i / (TX * TY);
-    f(i, ((size_t)(tiz * TZ + rz) * nn + (tiy * TY + ry)) * nn + (tix * TX + rx), rz * PLANE + ry * PX + rx);
+    f(i, ((size_t)(tc[2] * TZ + rz) * nn + (tc[1] * TY + ry)) * nn + (tc[0] * TX + rx), rz * PLANE + ry * PX + rx);
   }
 }
 
@@ -784,12 +799,13 @@ __device__ __forceinline__ void deposit_body(const R* __restrict__ s, const uint
                                              const uint32_t* __restrict__ offsets,
                                              const uint32_t* __restrict__ entries, uint32_t capacity, int tile,
                                              double* acc, uint32_t* __restrict__ health, double fix = 0.0) {
+  const int tc[3] = {tile % G.ntx, (tile / G.ntx) % G.nty, tile / (G.ntx * G.nty)};
   uint32_t ob, oe, hb, he;
   tile_entries(offsets, capacity, (uint32_t)G.ntiles, tile, ob, oe, hb, he);
-  deposit_sums<R, TX, TY, TZ, DET>(s, id, mass, L, G, entries, tile, ob, oe - ob, hb, oe - ob + (he - hb), acc, health,
+  deposit_sums<R, TX, TY, TZ, DET>(s, id, mass, L, G, entries, tc, ob, oe - ob, hb, oe - ob + (he - hb), acc, health,
                                    fix);
   const unsigned long long* iacc = reinterpret_cast<const unsigned long long*>(acc);
-  each_tile_cell<TX, TY, TZ>(L.n, G, tile, [&](int, size_t at, int li) {
+  each_tile_cell<TX, TY, TZ>(L.n, tc, [&](int, size_t at, int li) {
     rho[at] = DET ? R((double)iacc[li] / fix) : R(acc[li]);
   });
 }
@@ -1794,6 +1810,7 @@ __global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ po
       tile = (int)(halo ? e.x - nt : e.x);
       i = e.y;
     }
+    const int tc[3] = {tile % G.ntx, (tile / G.ntx) % G.nty, tile / (G.ntx * G.nty)};
     uint32_t ob, oe, hb, he;
     tile_entries(offsets, capacity, nt, tile, ob, oe, hb, he);
     const uint32_t d_own = dense[tile], d_halo = dense[nt + tile];
@@ -1804,10 +1821,10 @@ __global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ po
       if (halo) oe = ob;
       else he = hb;
     }
-    deposit_sums<float, TX, TY, TZ, false, true>(pos, nullptr, mass, L, G, entries, tile, ob, oe - ob, hb,
+    deposit_sums<float, TX, TY, TZ, false, true>(pos, nullptr, mass, L, G, entries, tc, ob, oe - ob, hb,
                                                  oe - ob + (he - hb), acc, nullptr);
     if (!(d_own | d_halo)) {
-      each_tile_cell<TX, TY, TZ>(L.n, G, tile, [&](int, size_t at, int li) { rho[at] = float(acc[li]); });
+      each_tile_cell<TX, TY, TZ>(L.n, tc, [&](int, size_t at, int li) { rho[at] = float(acc[li]); });
       break;
     }
     // each block of the tile leaves its sums; the one that leaves them last adds them all up in FP64 and
@@ -1815,7 +1832,7 @@ __global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ po
     const uint32_t s_own = d_own - 1, s_halo = d_halo - 1;
     const uint32_t place = halo ? s_halo + i : (d_own ? s_own : s_halo) + i;
     double* mine = P.part + (size_t)place * CELLS;
-    each_tile_cell<TX, TY, TZ, 4>(L.n, G, tile, [&](int c, size_t, int li) { mine[c] = acc[li]; });
+    each_tile_cell<TX, TY, TZ, 4>(L.n, tc, [&](int c, size_t, int li) { mine[c] = acc[li]; });
     __threadfence();
     __syncthreads();
     if (threadIdx.x == 0)
@@ -1842,7 +1859,7 @@ __global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ po
       };
       if (d_own) add(s_own, 1 + p_own);
       if (d_halo) add(d_own ? s_halo + 1 : s_halo, d_own ? p_halo : 1 + p_halo);
-      each_tile_cell<TX, TY, TZ, 4>(L.n, G, tile, [&](int, size_t at, int li) { rho[at] = float(acc[li]); });
+      each_tile_cell<TX, TY, TZ, 4>(L.n, tc, [&](int, size_t at, int li) { rho[at] = float(acc[li]); });
     }
     __syncthreads();  // (the accumulator and `last` are used again)
     x += extra;
@@ -2096,16 +2113,6 @@ hipError_t bins_count(const PState<R>& p, const Lattice& L, const TileGeom& G, c
   return hipGetLastError();
 }
 
-template <bool PIECES>
-static hipError_t launch_scan_small(long m, const Bins& B, uint32_t* far, uint32_t* old, const RefPieces& P,
-                                    hipStream_t st) {
-  if (m <= kScanSmallT)
-    k_scan_small<1, PIECES><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old, P);
-  else
-    k_scan_small<2, PIECES><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old, P);
-  return hipGetLastError();
-}
-
 hipError_t bins_scan(const TileGeom& G, const Bins& B, hipStream_t st, bool after_gather) {
   const long m = 2L * G.ntiles;
   const int nb = scan_blocks(G);
@@ -2113,10 +2120,12 @@ hipError_t bins_scan(const TileGeom& G, const Bins& B, hipStream_t st, bool afte
   uint32_t* far = ts ? B.counts + ts_far_at(G.ntiles) : nullptr;
   uint32_t* old = ts ? B.counts + ts_old_at(G.ntiles) : nullptr;
   if (m <= kScanSmall) {
-    return launch_scan_small<false>(m, B, far, old, RefPieces{}, st);
+    if (m <= kScanSmallT) k_scan_small<1><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old);
+    else k_scan_small<2><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, far, old);
+    return hipGetLastError();
   }
   k_scan_reduce_spine<<<nb, kT, 0, st>>>(B.counts, m, B.block_sums, nb, B.done, far);
-  k_scan_apply<false><<<nb, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, far, old, RefPieces{});
+  k_scan_apply<<<nb, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, far, old);
   return hipGetLastError();
 }
 
@@ -2195,12 +2204,14 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
   } while (0)
   PM_REF_TILE_DISPATCH(G, PM_L);
 #undef PM_L
-  if (m <= kScanSmall) {
-    if (hipError_t e = launch_scan_small<true>(m, B, nullptr, nullptr, P, st)) return e;
+  if (m <= kScanSmallT) {
+    k_ref_scan_small<1><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, P);
+  } else if (m <= kScanSmall) {
+    k_ref_scan_small<2><<<1, kScanSmallT, 0, st>>>(B.counts, m, B.offsets, B.cursors, P);
   } else {
     const int nbs = scan_blocks(G);
     k_scan_reduce_spine<<<nbs, kT, 0, st>>>(B.counts, m, B.block_sums, nbs, B.done, nullptr);
-    k_scan_apply<true><<<nbs, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, nullptr, nullptr, P);
+    k_ref_scan_apply<<<nbs, kT, 0, st>>>(B.counts, m, B.block_sums, B.offsets, B.cursors, P);
   }
   fits = true;
   if (B.capacity < (halo ? 8 : 1) * (uint64_t)np) {
