@@ -119,7 +119,7 @@ def stage_timing(pos, vel, w, steps, tiles=(0, 0, 0)):
 
 def plain_fp64_bench(pos, vel, w, steps):
     """The reference's algorithm as plain GPU code: the reference-layout entry points
-    (density(): global float atomics into a new grid; advance_time(): complex128 FFT Poisson
+    (density(): tile bins and FP64 sums in LDS, rounded to float32; advance_time(): complex128 FFT Poisson
     solve, float32 potential, reference integrate with pre-step cells for all axes), absolute
     float32 positions, called once per step like pmesh.py:60-61."""
     from pmgpu import ops
@@ -143,7 +143,7 @@ def plain_fp64_bench(pos, vel, w, steps):
     dt = time.perf_counter() - t0
     return {"value": npart ** 3 * steps / dt, "ms_per_step": dt / steps * 1e3, "steps": steps,
             "path": "reference-layout entry points pm_density + pm_advance_time (float32 "
-                    "storage, complex128 FFT, global atomics, one call per reference function)"}
+                    "storage, complex128 FFT, tile bins made by every call, one call per reference function)"}
 
 
 # Batched ensemble workload: 48 realisations, seeds 100-147, N_grid uniform over 128/192/256

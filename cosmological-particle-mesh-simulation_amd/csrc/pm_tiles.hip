@@ -18,9 +18,9 @@
 // The gather reads the own entries with the tile's potential (plus a -1/+2 stencil margin)
 // staged in LDS, and counts the new positions through an LDS histogram of each tile's 4^3 tile
 // neighbourhood (binning from positions alone counts with a wave-aggregated atomic per distinct
-// key).  A two-kernel exclusive scan turns the counts into offsets; after a gather the tile
-// scatter writes the entries through LDS cursors from ranges the gather reserved, otherwise the
-// particle-parallel scatter through device cursors.
+// key).  An exclusive scan (one block up to 2048 counts, else two kernels) turns the counts into
+// offsets; after a gather the tile scatter writes the entries through LDS cursors from ranges the
+// gather reserved, otherwise the particle-parallel scatter through device cursors.
 #include <algorithm>
 #include <cmath>
 #include <vector>

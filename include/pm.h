@@ -152,7 +152,9 @@ PM_API int pm_sim_step(pm_sim* sim, double a, double da);
 PM_API int pm_sim_run(pm_sim* sim, double a, double da, int n_steps, double* a_out);
 /* per-stage timing with HIP events on the sim's stream (0 off, 1 on); stage order:
  * deposit, r2c_x, c2c_y_fwd, z_green, c2c_y_inv, c2r_x, gather_kick_drift, bin, deposit_r2c
- * (the fused deposit + R2C x pass, which replaces the first two where it runs)               */
+ * (the fused deposit + R2C x pass, which replaces the first two where it runs).  On grids whose
+ * z planes fit in LDS (FP32 to N_CELLS = 192, FP64 to 128) the x stages hold the y passes too and
+ * the y stages stay 0, unless pm_sim_set_pencils chose a y shape.                             */
 PM_API int pm_sim_set_timing(pm_sim* sim, int enable);
 PM_API int pm_sim_get_timing(pm_sim* sim, double* stage_ms, int64_t* stage_calls, int n_stages);
 PM_API int pm_sim_sync(pm_sim* sim);

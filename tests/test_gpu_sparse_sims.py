@@ -38,18 +38,19 @@ def test_shape_and_bits(n, side, prec, tiles):
     assert all(np.array_equal(a, b) for a, b in zip(*out))
 
 
-def test_sparse_members_keep_the_bits():
+@pytest.mark.parametrize("grids", [((192, 48), (128, 32), (64, 16)), ((256, 128), (96, 48), (192, 96), (48, 24))])
+def test_members_keep_the_bits_of_lone_runs_in_their_tiles(grids):
     from pmgpu.ensemble import PMEnsemble
     from pmgpu.sim import PMSim
     sims, lone = [], []
-    for n, side in ((192, 48), (128, 32), (64, 16)):
+    for n, side in grids:
         x, v = _state(n, side)
         for group in (sims, lone):
             s = PMSim(n, side, 32, deterministic=True, **KW)
             s.set_state(x, v)
             group.append(s)
     ens = PMEnsemble(sims)
-    ens.run([0.5] * 3, [0.01] * 3, 9)
+    ens.run([0.5] * len(sims), [0.01] * len(sims), 9)
     for a, b in zip(sims, lone):
         b.set_tiles(*a.tiles())
         b.run(0.5, 0.01, 9)
