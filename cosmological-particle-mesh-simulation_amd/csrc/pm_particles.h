@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "pm_common.h"
+#include "pm_pieces.h"
 #include "pm_fft.h"
 
 namespace pm {
@@ -224,27 +225,14 @@ hipError_t gkd_tiles(const PState<R>& in, const PState<R>& out, const R* phi, do
 
 // ---- reference-layout kernels (absolute float32 positions, reference order) ------------------
 hipError_t ref_density(const float* pos, long np, int n, double mass, float* rho, hipStream_t st);
-// Dense tiles of a reference-layout call.  A key (own or halo segment of a tile) of at least `dense`
-// entries is cut into pieces of `per` (64 longer ones at most): the tile's block takes the first,
-// the others are listed by the scan and shared out to further blocks.  The deposit's blocks of one tile
-// leave FP64 partial sums; the last to do so (ticket) adds them up, about 1 us each, and rounds.
-// per is 4096 entries, four batches of a deposit block (about 15 us, what the meeting of a tile's blocks
-// costs), or N_p / 512: at most 256 tiles have own pieces, and a block's share of a call stays small.
-// dense is 2 per, and on 64 tiles or more twice their mean: evenly filled, they keep the chip busy by
-// themselves (density of 2.1 M random particles on 96^3, whole / in pieces of 4096: 248 / 336 us; on
-// 48^3, 27 tiles, 650 / 429).  Keys beyond the room for partial sums run whole.
-struct RefPieces {
-  uint32_t per = 0, dense = 0;
-  uint32_t max = 0;             // capacity of the list: all keys' count / per
-  uint32_t parts = 0;           // partial sums (deposit; the push needs none)
-  uint32_t cells = 0;           // values of each
+// Crowded tiles of a reference-layout call (pm_pieces.h): the sizes and where the lists are kept
+struct RefPieces : PieceSizes {
+  uint32_t cells = 0;           // values of a partial sum
   uint32_t* n = nullptr;        // kRefCounters: pieces listed, partial sums taken
   uint2* list = nullptr;        // {key, piece}
   double* part = nullptr;
   uint32_t* tickets = nullptr;  // one per partial sum (a tile uses that of its first)
 };
-constexpr long kRefPiece = 4096, kRefPieces = 512;
-constexpr int kRefTilePieces = 64;  // of one key
 constexpr int kRefCounters = 32;  // (two are used: the counts that follow start a cache line)
 RefPieces ref_pieces(long np, const TileGeom& G, bool halo);  // sizes; the caller sets the pointers
 

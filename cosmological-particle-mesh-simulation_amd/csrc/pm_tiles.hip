@@ -546,24 +546,12 @@ __global__ __launch_bounds__(kT) void k_scan_reduce_spine(const uint32_t* __rest
   scan_reduce_spine_body(counts, m, bsum, nb, done, blockIdx.x, sh, &last, far);
 }
 
-// pieces of a key beyond its first
-__device__ __forceinline__ uint32_t pieces_of(const RefPieces& P, bool dense, uint32_t count) {
-  return dense ? min(count / P.per, (uint32_t)kRefTilePieces) - 1 : 0u;
-}
-// entries of piece i of the key with entries [beg, end); i = 0: what the tile's own block takes
-__device__ __forceinline__ void piece_range(const RefPieces& P, bool dense, uint32_t i, uint32_t& beg, uint32_t& end) {
-  if (!dense) return;
-  const uint32_t last = pieces_of(P, true, end - beg), len = (end - beg) / (last + 1);
-  beg += i * len;
-  if (i < last) end = beg + len;
-}
-
-// Lists the pieces of a dense key of a reference-layout call (see RefPieces) and returns what the scan
+// Lists the pieces of a dense key of a reference-layout call (see pm_pieces.h) and returns what the scan
 // leaves in its count: 1 + the first of its partial sums (1 where pieces need none), 0 for a key that one
 // block takes whole.
 __device__ __forceinline__ uint32_t list_pieces(const RefPieces& P, uint32_t key, uint32_t count) {
   if (count < P.dense) return 0u;
-  const uint32_t extra = pieces_of(P, true, count);
+  const uint32_t extra = pieces_beyond(P.per, count);
   uint32_t slot = 0u;
   if (P.part) {
     slot = atomicAdd(&P.n[1], extra + 1);
@@ -1814,9 +1802,10 @@ __global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ po
     uint32_t ob, oe, hb, he;
     tile_entries(offsets, capacity, nt, tile, ob, oe, hb, he);
     const uint32_t d_own = dense[tile], d_halo = dense[nt + tile];
-    const uint32_t p_own = pieces_of(P, d_own, oe - ob), p_halo = pieces_of(P, d_halo, he - hb);
-    piece_range(P, d_own, halo ? 0 : i, ob, oe);
-    piece_range(P, d_halo, halo ? i : 0, hb, he);
+    const uint32_t p_own = d_own ? pieces_beyond(P.per, oe - ob) : 0u;
+    const uint32_t p_halo = d_halo ? pieces_beyond(P.per, he - hb) : 0u;
+    if (d_own) piece_range(P.per, halo ? 0 : i, ob, oe);
+    if (d_halo) piece_range(P.per, halo ? i : 0, hb, he);
     if (piece) {
       if (halo) oe = ob;
       else he = hb;
@@ -1999,7 +1988,7 @@ __global__ __launch_bounds__(kT) void k_ref_push(float* __restrict__ pos, float*
     }
     uint32_t beg, end;
     tile_range(offsets, capacity, tile, beg, end);
-    piece_range(P, dense[tile], i, beg, end);
+    if (dense[tile]) piece_range(P.per, i, beg, end);
     if (beg == end) return;
     push_entries<TX, TY, TZ>(pos, vel, np, n, a, fa1, da, phi, G, entries, tile, beg, end, box);
     __syncthreads();  // (the box is used again)
@@ -2234,13 +2223,8 @@ static hipError_t ref_bin(const float* pos, long np, int n, bool halo, const Til
 
 RefPieces ref_pieces(long np, const TileGeom& G, bool halo) {
   RefPieces P;
-  P.per = (uint32_t)std::max(kRefPiece, (np + kRefPieces - 1) / kRefPieces);
-  P.dense = (uint32_t)std::max(2L * P.per, G.ntiles >= 64 ? 2 * np / G.ntiles : 0L);
-  P.max = (uint32_t)((halo ? 8 : 1) * np / P.per);  // no more: a piece beyond a tile's first holds >= per entries
-  if (halo) {
-    P.parts = std::min(P.max, (uint32_t)(2 * kRefPieces));
-    P.cells = (uint32_t)(G.tx * G.ty * G.tz);
-  }
+  static_cast<PieceSizes&>(P) = piece_sizes(np, G.ntiles, halo);
+  if (halo) P.cells = (uint32_t)(G.tx * G.ty * G.tz);
   return P;
 }
 
