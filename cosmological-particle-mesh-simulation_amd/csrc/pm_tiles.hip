@@ -678,6 +678,29 @@ __device__ __forceinline__ void deposit_sums(const R* __restrict__ s, const uint
   uint32_t sl[E], pid[E];
   R sv[E][3];
   auto load = [&](uint32_t base) {
+    if constexpr (ABS) {
+      // lanes past the end repeat the last entry: without branches the loads of the E entries, then of
+      // their positions, are in flight together
+      if (total == 0u) {
+#pragma unroll
+        for (int u = 0; u < E; ++u) sl[u] = kNone;
+        return;
+      }
+      uint32_t at[E];
+#pragma unroll
+      for (int u = 0; u < E; ++u) {
+        const uint32_t i = min(base + u * kT + threadIdx.x, total - 1u);
+        at[u] = entries[i < n_own ? ob + i : hb + (i - n_own)];
+      }
+#pragma unroll
+      for (int u = 0; u < E; ++u) {
+        const uint32_t p = min(at[u], (uint32_t)(np - 1));
+        sl[u] = base + u * kT + threadIdx.x < total ? p : kNone;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) sv[u][a] = s[a * np + p];
+      }
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < E; ++u) {
       const uint32_t i = base + u * kT + threadIdx.x;
@@ -1794,9 +1817,10 @@ __global__ __launch_bounds__(kT) void k_ref_deposit(const float* __restrict__ po
     uint32_t i = 0u;
     if (piece) {
       const uint2 e = P.list[x];
-      halo = e.x >= nt;
-      tile = (int)(halo ? e.x - nt : e.x);
-      i = e.y;
+      const uint32_t key = __builtin_amdgcn_readfirstlane(e.x);  // (block-uniform, for scalar loads below)
+      halo = key >= nt;
+      tile = (int)(halo ? key - nt : key);
+      i = __builtin_amdgcn_readfirstlane(e.y);
     }
     const int tc[3] = {tile % G.ntx, (tile / G.ntx) % G.nty, tile / (G.ntx * G.nty)};
     uint32_t ob, oe, hb, he;
@@ -1983,8 +2007,8 @@ __global__ __launch_bounds__(kT) void k_ref_push(float* __restrict__ pos, float*
     uint32_t i = 0u;
     if (piece) {
       const uint2 e = P.list[x];
-      tile = (int)e.x;  // (own keys only)
-      i = e.y;
+      tile = (int)__builtin_amdgcn_readfirstlane(e.x);  // (own keys only; block-uniform, for scalar loads below)
+      i = __builtin_amdgcn_readfirstlane(e.y);
     }
     uint32_t beg, end;
     tile_range(offsets, capacity, tile, beg, end);
